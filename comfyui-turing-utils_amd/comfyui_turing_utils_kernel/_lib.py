@@ -91,6 +91,14 @@ SIGNATURES: dict[str, tuple[object, list[object]]] = {
          _f32, _i32, _c_void_p, _i64, _c_void_p],
     ),
     "tu_sage_attn_kv_splits": (_i32, [_i64, _i64, _i64, _i64, _i32, _i32]),
+    "tu_sage_attn_workspace": (_i64, [_i64, _i64, _i64, _i64, _i64, _i32, _i32]),
+    "tu_sage_attn_fwd_auto": (
+        _i32,
+        [_c_void_p, _c_void_p, _i64, _c_void_p, _c_void_p, _i64, _c_void_p, _i64, _c_void_p,
+         _i64, _i64, _i64, _i64, _i64, _i64,
+         _i64, _i64, _i64, _i64, _i64, _i64, _i64, _i64, _i64,
+         _f32, _i32, _i32, _c_void_p, _i64, _c_void_p],
+    ),
     "tu_qk_rms_rope_int8": (
         _i32,
         [_c_void_p, _c_void_p, _i32, _i64, _i64, _i64, _i64, _i64, _i64,
@@ -139,7 +147,7 @@ SIGNATURES: dict[str, tuple[object, list[object]]] = {
     ),
 }
 
-ABI_VERSION = 13
+ABI_VERSION = 14
 
 _lock = threading.Lock()
 _lib: ctypes.CDLL | None = None

@@ -207,15 +207,18 @@ def attention_from_vt(
     """Attention kernel only: quantized Q/K and V^T from ``value_transpose``.
 
     ``kv_splits`` (this package only): key ranges computed by separate
-    workgroups and merged, for grids that fill the GPU badly; None lets
-    ``tu_sage_attn_kv_splits`` choose from the device's compute units, 1
-    never splits.  Non-causal only.  A split call needs an fp32 workspace of
-    ``split_workspace_bytes(...)`` bytes (ranges x B x H x Lq x (D + 2) x 4:
-    about 100 MB at B1 H12 L8190 D128 with two ranges); it comes from
-    ``workspace`` (a contiguous float32 tensor on the Q/K device, at least
-    that large, reusable across calls on one stream) or else from torch's
-    caching allocator.  How many ranges None picks depends on the device's
-    compute-unit count, so results are bit-identical across devices only
+    workgroups and merged.  None chooses for itself (``tu_sage_attn_fwd_auto``):
+    the query blocks that would leave compute units idle at the end of the
+    grid are split, and long causal rows where the grid is small.  A number
+    splits every block into that many ranges (non-causal only), 1 none.  A
+    split call needs an fp32 workspace, at most ``split_workspace_bytes(...)``
+    bytes for its count of ranges (ranges x B x H x Lq x (D + 2) x 4); it
+    comes from ``workspace`` (a contiguous float32 tensor on the Q/K device, at
+    least as large as ``tu_sage_attn_kv_splits``' count or ``kv_splits`` needs,
+    reusable across calls on one stream) or else from torch's caching
+    allocator.  What None picks depends on the device's compute-unit count
+    (and on the size of ``workspace``), so results are bit-identical across
+    devices only
     with an explicit ``kv_splits``."""
     batch, hq, hkv, lq, lk = _check_qk(q_int8, q_scale, k_int8, k_scale, tensor_layout, blkq, blkk)
     width = q_int8.size(-1)
@@ -235,40 +238,45 @@ def attention_from_vt(
     _, _, osb, osh, osl = _layout_dims(output, tensor_layout)
     q_scale = q_scale.contiguous()
     k_scale = k_scale.contiguous()
-    if kv_splits is None:
-        splits = int(_lib.load().tu_sage_attn_kv_splits(batch, hq, lq, lk, int(bool(is_causal)),
-                                                        _compute_units(q_int8.device)))
-    else:
-        splits = int(kv_splits)
+    device = q_int8.device
+    usable = (workspace is not None and workspace.dtype == torch.float32 and workspace.device == device
+              and workspace.is_contiguous())
+    splits = int(kv_splits) if kv_splits is not None else 1
+    if kv_splits is not None:
         if splits < 1 or (is_causal and splits > 1):
             raise ValueError("kv_splits must be >= 1, and 1 for causal attention")
-    if splits > 1:
-        # key ranges merged by a second kernel: fp32 partial O plus
-        # (exponent base, row sum) per row and range
-        need = split_workspace_bytes(batch, hq, lq, lk, width, splits) // 4
-        if workspace is not None and (workspace.dtype != torch.float32 or workspace.device != q_int8.device
-                                      or not workspace.is_contiguous() or workspace.numel() < need):
+        required = splits
+    else:
+        # a caller's workspace has to hold what tu_sage_attn_kv_splits' count
+        # needs; the automatic plan then uses what fits into it
+        lib, cus = _lib.load(), _compute_units(device)
+        required = 1 if workspace is None else int(lib.tu_sage_attn_kv_splits(batch, hq, lq, lk, int(bool(is_causal)),
+                                                                              cus))
+    if required > 1 and workspace is not None:
+        need = split_workspace_bytes(batch, hq, lq, lk, width, required) // 4
+        if not usable or workspace.numel() < need:
             raise ValueError(f"Sage split workspace must be a contiguous float32 tensor on the Q/K device "
                              f"with at least {need} elements")
-    with torch.cuda.device(q_int8.device):
+    shape = (q_int8.data_ptr(), q_scale.data_ptr(), blkq, k_int8.data_ptr(), k_scale.data_ptr(), blkk,
+             value_t.data_ptr(), lpad, output.data_ptr(), batch, hq, hkv, lq, lk, width,
+             qsb, qsh, qsl, ksb, ksh, ksl, osb, osh, osl, scale)
+    with torch.cuda.device(device):
+        # key ranges merged by a second kernel: fp32 partial O plus
+        # (exponent base, row sum) per row and range
         if splits > 1:
-            partial = workspace if workspace is not None else torch.empty(need, dtype=torch.float32,
-                                                                          device=q_int8.device)
-            _lib.call(
-                "tu_sage_attn_fwd_split",
-                q_int8.data_ptr(), q_scale.data_ptr(), blkq, k_int8.data_ptr(), k_scale.data_ptr(), blkk,
-                value_t.data_ptr(), lpad, output.data_ptr(), batch, hq, hkv, lq, lk, width,
-                qsb, qsh, qsl, ksb, ksh, ksl, osb, osh, osl,
-                scale, splits, partial.data_ptr(), partial.numel() * 4, _lib.stream_of(q_int8.device),
-            )
+            partial = workspace if workspace is not None else torch.empty(
+                split_workspace_bytes(batch, hq, lq, lk, width, splits) // 4, dtype=torch.float32, device=device)
+            _lib.call("tu_sage_attn_fwd_split", *shape, splits, partial.data_ptr(), partial.numel() * 4,
+                      _lib.stream_of(device))
+        elif kv_splits is not None:
+            _lib.call("tu_sage_attn_fwd", *shape, int(bool(is_causal)), _lib.stream_of(device))
         else:
-            _lib.call(
-                "tu_sage_attn_fwd",
-                q_int8.data_ptr(), q_scale.data_ptr(), blkq, k_int8.data_ptr(), k_scale.data_ptr(), blkk,
-                value_t.data_ptr(), lpad, output.data_ptr(), batch, hq, hkv, lq, lk, width,
-                qsb, qsh, qsl, ksb, ksh, ksl, osb, osh, osl,
-                scale, int(bool(is_causal)), _lib.stream_of(q_int8.device),
-            )
+            partial = workspace if usable and workspace.data_ptr() % 16 == 0 else None
+            if partial is None:
+                nbytes = int(lib.tu_sage_attn_workspace(batch, hq, lq, lk, width, int(bool(is_causal)), cus))
+                partial = torch.empty(nbytes // 4, dtype=torch.float32, device=device) if nbytes else None
+            _lib.call("tu_sage_attn_fwd_auto", *shape, int(bool(is_causal)), cus, _lib.ptr(partial),
+                      partial.numel() * 4 if partial is not None else 0, _lib.stream_of(device))
     return output
 
 

@@ -37,6 +37,7 @@
 //     (p <= 2^8), which after the first tiles is rare.
 //   * LDS rows are 128 B with 16-byte chunks XOR-swizzled by row bits 1..3,
 //     conflict-free for the 16 lanes that read one chunk column.
+#include <algorithm>
 #include <type_traits>
 
 #include "attn_common.h"
@@ -403,17 +404,43 @@ __device__ __forceinline__ void mfma_cluster(const int8_t *kst, const int8_t *vs
 constexpr int kStages = 4;
 constexpr int kAhead = kStages - 1;
 
-// kSplit: the workgroup covers key tiles [blockIdx.z * split_tiles, + split_tiles)
-// of a non-causal attention and writes its unnormalized O with the row's
-// exponent base and row sum to `part` for sage_combine_kernel.
+// Work plan of a launch.  Query blocks are numbered head-major (block =
+// (batch * hq + head) * nqb + query block).  Non-causal: blocks below
+// split_from run whole, one workgroup each; every later block runs as
+// `parts` workgroups of seg_tiles key tiles (the last range may be shorter),
+// all blocks' first ranges before any second range.  Causal: every block
+// runs as ceil(its key tiles / seg_tiles) workgroups; workgroups are numbered
+// by query block from the last, longest one to the first (heads fastest,
+// then ranges), so the long ones start first and the short ones fill the
+// end: at B2 H16 L4001 D128 that took the kernel from 177 to 115 us.
+struct AttnPlan {
+    uint32_t nqb;         // query blocks of a head
+    uint32_t bh;          // batch * hq
+    uint32_t split_from;  // first split block (non-causal)
+    uint32_t parts;       // key ranges of a split block (causal: of the last query block)
+    int seg_tiles;        // key tiles of a range
+    int64_t part_row0;    // query row (batch * hq * lq numbering) of the first split block
+    int64_t part_rows;    // query rows of the split blocks
+};
+
+// Workgroup i of n (XCD i mod 8) -> its place in the plan: XCD x owns the
+// contiguous x-th eighth of the n, so the query blocks of a head run on one
+// XCD and its L2 reads that head's K and V^T once for all of them.
+__device__ __forceinline__ uint32_t xcd_chunk(uint32_t i, uint32_t n) {
+    const uint32_t x = i & 7, q = n >> 3, r = n & 7;
+    return x * q + min(x, r) + (i >> 3);
+}
+
+// kSplit: workgroups that cover only a range of their block's key tiles write
+// the unnormalized O with each row's exponent base and row sum to `part` for
+// sage_combine_kernel.
 template <int D, bool kCausal, bool kSplit = false>
 __global__ __launch_bounds__(kThreads, 1) void sage_attn_kernel(
-    const int8_t *__restrict__ q8, const float *__restrict__ q_scale, int blkq, const int8_t *__restrict__ k8,
-    const float *__restrict__ k_scale, int kscale_shift, const uint16_t *__restrict__ vt, uint16_t *__restrict__ o,
-    int hq, int groups, int64_t lq, int64_t lk, int64_t lpad, int64_t q_sb, int64_t q_sh, int64_t q_sl,
-    int64_t k_sb, int64_t k_sh, int64_t k_sl, int64_t o_sb, int64_t o_sh, int64_t o_sl, float sm_log2,
-    int split_tiles, float *__restrict__ part) {
-    static_assert(!(kSplit && kCausal), "key splits are for non-causal attention");
+    const int8_t *__restrict__ q8, const float *__restrict__ q_scale, uint32_t blkq, uint32_t nbq,
+    const int8_t *__restrict__ k8, const float *__restrict__ k_scale, int kscale_shift, uint32_t nbk,
+    const uint16_t *__restrict__ vt, uint16_t *__restrict__ o, uint32_t hq, uint32_t groups, int64_t lq, int64_t lk,
+    int64_t lpad, int64_t q_sb, int64_t q_sh, int64_t q_sl, int64_t k_sb, int64_t k_sh, int64_t k_sl, int64_t o_sb,
+    int64_t o_sh, int64_t o_sl, float sm_log2, AttnPlan plan, float *__restrict__ part) {
     constexpr int kSl = Geo<D>::kKSlices;
     constexpr int kLoadsPerTile = Geo<D>::kLoadsPerTile;
     __shared__ __align__(1024) int8_t lds[kStages][Geo<D>::kStageBytes];
@@ -426,33 +453,69 @@ __global__ __launch_bounds__(kThreads, 1) void sage_attn_kernel(
     const int g = lane >> 4;
     const int lc = lane & 15;
 
-    const int64_t bh = blockIdx.y;
-    const int64_t b = bh / hq, h = bh % hq, hk = h / groups;
-    const int64_t hkv = hq / groups;
-    const int64_t qblock0 = static_cast<int64_t>(blockIdx.x) * kBQ;
+    // (batch * head, query block, key range) of this workgroup, in 32-bit
+    // arithmetic: 64-bit divisions are long instruction sequences, and a
+    // short key sequence pays for them in every workgroup
+    uint32_t bh, qb, z = 0;
+    bool whole = true;
+    if constexpr (kCausal) {
+        uint32_t id = blockIdx.x;
+        bh = id % plan.bh;
+        id /= plan.bh;
+        if constexpr (kSplit) {
+            z = id % plan.parts;
+            id /= plan.parts;
+        }
+        qb = plan.nqb - 1 - id;
+    } else {
+        const uint32_t blocks = plan.nqb * plan.bh;
+        uint32_t blk = blockIdx.x;
+        if (kSplit && blk >= plan.split_from) {
+            const uint32_t n = blocks - plan.split_from;
+            const uint32_t i = xcd_chunk(blk - plan.split_from, n * plan.parts);
+            z = i / n;
+            blk = plan.split_from + i - z * n;
+            whole = false;
+        } else {
+            blk = xcd_chunk(blk, kSplit ? plan.split_from : blocks);
+        }
+        bh = blk / plan.nqb;
+        qb = blk % plan.nqb;
+    }
+    const uint32_t b = bh / hq, h = bh % hq, hk = h / groups;
+    const uint32_t hkv = hq / groups;
+    const int64_t qblock0 = static_cast<int64_t>(qb) * kBQ;
     const int64_t q0 = qblock0 + grp * (kBQ / 2) + w4 * kWaveQ;
 
     const int8_t *qp = q8 + b * q_sb + h * q_sh;
     const int8_t *kp = k8 + b * k_sb + hk * k_sh;
-    const uint16_t *vtp = vt + (b * hkv + hk) * D * lpad;
-    const int64_t nbq = (lq + blkq - 1) / blkq;
-    const int64_t nbk = ((lk + kBKey - 1) / kBKey + (1 << kscale_shift) - 1) >> kscale_shift;
-    const float *ks_row = k_scale + (b * hkv + hk) * nbk;
+    const uint16_t *vtp = vt + static_cast<int64_t>(b * hkv + hk) * D * lpad;
+    const float *ks_row = k_scale + static_cast<int64_t>(b * hkv + hk) * nbk;
 
     int64_t key_end = lk;
     if constexpr (kCausal) key_end = min(lk, qblock0 + kBQ);
-    // first key tile of this workgroup's key range (0 unless split)
-    const int tile_base = kSplit ? static_cast<int>(blockIdx.z) * split_tiles : 0;
     int tiles = static_cast<int>((key_end + kBKey - 1) / kBKey);
-    if constexpr (kSplit) tiles = min(split_tiles, tiles - tile_base);
+    // first key tile of this workgroup's key range (0 unless split)
+    int tile_base = 0;
+    if constexpr (kSplit) {
+        tile_base = static_cast<int>(z) * plan.seg_tiles;
+        if constexpr (kCausal) {
+            whole = tiles <= plan.seg_tiles;
+            if (tile_base >= tiles) return;  // the whole workgroup: a short block has fewer ranges
+        }
+        if (!whole) tiles = min(plan.seg_tiles, tiles - tile_base);
+    }
     // Tiles this wave computes: all of them, or up to its last query's
-    // diagonal when causal.  Later tiles only keep the barrier count.
+    // diagonal when causal.  Later tiles only keep the barrier count.  (A
+    // causal range starts at a multiple of 4 tiles, at or before its block's
+    // first diagonal tile, so every row sees its first key.)
     int my_tiles = tiles;
     if constexpr (kCausal)
-        my_tiles = static_cast<int>(min<int64_t>(tiles, max<int64_t>(1, (min(q0 + kWaveQ, lq) + kBKey - 1) / kBKey)));
+        my_tiles = static_cast<int>(
+            min<int64_t>(tiles, max<int64_t>(1, (min(q0 + kWaveQ, lq) + kBKey - 1) / kBKey - tile_base)));
     // Tiles at or past this one need the Lk-tail or causal mask.
     int64_t mask_from = lk / kBKey - tile_base;
-    if constexpr (kCausal) mask_from = min(mask_from, q0 / kBKey);
+    if constexpr (kCausal) mask_from = min(mask_from, q0 / kBKey - tile_base);
     const int first_masked = static_cast<int>(min<int64_t>(tiles, mask_from));
 
     const LaneGeom<D> gm = lane_geom<D>(w4, lane, k_sl, lpad);
@@ -469,7 +532,7 @@ __global__ __launch_bounds__(kThreads, 1) void sage_attn_kernel(
 #pragma unroll
         for (int ds = 0; ds < kSl; ++ds)
             qf[qt][ds] = *reinterpret_cast<const i32x4 *>(qp + qi * q_sl + 64 * ds + 16 * g);
-        qsc[qt] = q_scale[(b * hq + h) * nbq + qi / blkq] * sm_log2;
+        qsc[qt] = q_scale[static_cast<int64_t>(bh) * nbq + static_cast<uint32_t>(qi) / blkq] * sm_log2;
     }
     if (grp == 0) {
 #pragma unroll
@@ -559,13 +622,12 @@ __global__ __launch_bounds__(kThreads, 1) void sage_attn_kernel(
     __builtin_amdgcn_s_waitcnt(0);
 
     // acc_o[ds][qt][r] = O[q0 + 16 qt + lc][16 ds + 4 g + r]; acc_l[qt][*] = l.
-    if constexpr (kSplit) {
+    if (kSplit && !whole) {
         // unnormalized O of this key range, then (m_used, l) per row:
-        // part = [splits][B * H][lq][D] fp32, followed by [splits][B * H][lq][2]
-        const int64_t rows = static_cast<int64_t>(gridDim.y) * lq;
-        const int64_t row0 = (static_cast<int64_t>(blockIdx.z) * gridDim.y + bh) * lq;
+        // part = [parts][part_rows][D] fp32, followed by [parts][part_rows][2]
+        const int64_t row0 = z * plan.part_rows + bh * lq - plan.part_row0;
         float *po = part + row0 * D;
-        float *pml = part + static_cast<int64_t>(gridDim.z) * rows * D + row0 * 2;
+        float *pml = part + plan.parts * plan.part_rows * D + row0 * 2;
 #pragma unroll
         for (int qt = 0; qt < kQT; ++qt) {
             const int64_t qi = q0 + 16 * qt + lc;
@@ -578,17 +640,35 @@ __global__ __launch_bounds__(kThreads, 1) void sage_attn_kernel(
         return;
     }
     uint16_t *op = o + b * o_sb + h * o_sh;
+    // rows that start on 8-byte but not 16-byte boundaries take two stores
+    const bool wide = ((reinterpret_cast<uintptr_t>(o) >> 1 | o_sb | o_sh | o_sl) & 7) == 0;
 #pragma unroll
     for (int qt = 0; qt < kQT; ++qt) {
         const int64_t qi = q0 + 16 * qt + lc;
         const float inv = 1.0f / st.acc_l[qt][0];
-        if (qi >= lq) continue;
+        // Two 16-channel blocks at a time: exchanging odd lane groups of the
+        // first with even ones of the second leaves each lane 8 contiguous
+        // channels of one block, one 16-byte store (64 bytes of a row per
+        // instruction instead of 32).
 #pragma unroll
-        for (int ds = 0; ds < Geo<D>::kDS; ++ds) {
-            u32x2 packed;
-            packed.x = pack_bf16x2(st.acc_o[ds][qt][0] * inv, st.acc_o[ds][qt][1] * inv);
-            packed.y = pack_bf16x2(st.acc_o[ds][qt][2] * inv, st.acc_o[ds][qt][3] * inv);
-            *reinterpret_cast<u32x2 *>(op + qi * o_sl + 16 * ds + 4 * g) = packed;
+        for (int ds = 0; ds < Geo<D>::kDS; ds += 2) {
+            uint32_t w[2][2];
+#pragma unroll
+            for (int i = 0; i < 2; ++i) {
+                const f32x4 a = st.acc_o[ds + i][qt];
+                w[i][0] = hw_bf16x2_bits(a[0] * inv, a[1] * inv);
+                w[i][1] = hw_bf16x2_bits(a[2] * inv, a[3] * inv);
+            }
+            auto lo = __builtin_amdgcn_permlane16_swap(w[0][0], w[1][0], false, false);
+            auto hi = __builtin_amdgcn_permlane16_swap(w[0][1], w[1][1], false, false);
+            if (qi >= lq) continue;
+            uint16_t *dst = op + qi * o_sl + 16 * (ds + (g & 1)) + 8 * (g >> 1);
+            if (wide) {
+                *reinterpret_cast<u32x4 *>(dst) = u32x4{lo[0], hi[0], lo[1], hi[1]};
+            } else {
+                reinterpret_cast<u32x2 *>(dst)[0] = u32x2{lo[0], hi[0]};
+                reinterpret_cast<u32x2 *>(dst)[1] = u32x2{lo[1], hi[1]};
+            }
         }
     }
 }
@@ -633,19 +713,29 @@ __global__ __launch_bounds__(256) void v_prep_kernel(const uint16_t *__restrict_
     }
 }
 
-// Merges the key-range partials of sage_attn_kernel<D, false, true>: per
+// Merges the key-range partials of sage_attn_kernel<D, ., true>: per
 // row, M = max_s m_s, w_s = 2^(m_s - M), out = sum_s w_s O_s / sum_s w_s l_s
-// rounded to bf16.  D / 8 threads per row, 8 channels each.
-template <int D>
-__global__ __launch_bounds__(256) void sage_combine_kernel(const float *__restrict__ part, int splits, int hq,
-                                                           int64_t bh_rows, int64_t lq, uint16_t *__restrict__ o,
+// rounded to bf16.  D / 8 threads per row, 8 channels each.  Causal rows have
+// as many ranges as their block's key tiles fill; rows with one range were
+// written by the attention kernel.
+template <int D, bool kCausal>
+__global__ __launch_bounds__(256) void sage_combine_kernel(const float *__restrict__ part, AttnPlan plan, uint32_t hq,
+                                                           int64_t lq, int64_t lk, uint16_t *__restrict__ o,
                                                            int64_t o_sb, int64_t o_sh, int64_t o_sl) {
     constexpr int kTpr = D / 8;  // threads per row
     const int64_t row = static_cast<int64_t>(blockIdx.x) * (256 / kTpr) + threadIdx.x / kTpr;
     const int d0 = (threadIdx.x % kTpr) * 8;
-    const int64_t rows = bh_rows * lq;
+    const int64_t rows = plan.part_rows;
     if (row >= rows) return;
-    const float *ml = part + static_cast<int64_t>(splits) * rows * D;
+    const int64_t bh = (plan.part_row0 + row) / lq, q = plan.part_row0 + row - bh * lq;
+    int splits = static_cast<int>(plan.parts);
+    if constexpr (kCausal) {
+        const int64_t key_end = min(lk, (q / kBQ + 1) * kBQ);
+        const int tiles = static_cast<int>((key_end + kBKey - 1) / kBKey);
+        splits = (tiles + plan.seg_tiles - 1) / plan.seg_tiles;
+        if (splits == 1) return;
+    }
+    const float *ml = part + plan.parts * rows * D;
     float m = -INFINITY;
     for (int sp = 0; sp < splits; ++sp) m = fmaxf(m, ml[(sp * rows + row) * 2]);
     float l = 0.0f, acc[8] = {0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f};
@@ -662,7 +752,6 @@ __global__ __launch_bounds__(256) void sage_combine_kernel(const float *__restri
         }
     }
     const float inv = 1.0f / l;
-    const int64_t bh = row / lq, q = row - bh * lq;
     uint16_t *dst = o + (bh / hq) * o_sb + (bh % hq) * o_sh + q * o_sl + d0;
     u32x2 lo, hi;
     lo.x = pack_bf16x2(acc[0] * inv, acc[1] * inv);
@@ -730,6 +819,154 @@ int32_t check_attn_args(const int8_t *q8, const float *q_scale, int64_t blkq, co
 }  // namespace
 }  // namespace tu
 
+namespace tu {
+namespace {
+
+// Launches the attention (and, when some block is split, the merge) by a plan.
+template <int D, bool kCausal>
+int32_t launch_planned(const AttnPlan &plan, const int8_t *q8, const float *q_scale, int64_t blkq, const int8_t *k8,
+                       const float *k_scale, int64_t blkk, const void *vt, int64_t lpad, void *out, int64_t hq,
+                       int64_t hkv, int64_t lq, int64_t lk, int64_t q_sb, int64_t q_sh, int64_t q_sl, int64_t k_sb,
+                       int64_t k_sh, int64_t k_sl, int64_t o_sb, int64_t o_sh, int64_t o_sl, float sm_scale,
+                       float *part, hipStream_t s) {
+    int kscale_shift = 0;
+    while ((kBKey << kscale_shift) < blkk) ++kscale_shift;
+    const uint32_t nbq = static_cast<uint32_t>((lq + blkq - 1) / blkq);
+    const uint32_t nbk = static_cast<uint32_t>((lk + blkk - 1) / blkk);
+    const int64_t blocks = static_cast<int64_t>(plan.nqb) * plan.bh;
+    const bool split = plan.parts > 1;
+    const int64_t grid = !split    ? blocks
+                         : kCausal ? blocks * plan.parts
+                                   : plan.split_from + (blocks - plan.split_from) * plan.parts;
+    TU_REQUIRE(grid <= 0x7fffffff, "Sage attention grid too large");
+#define TU_ATTN_ARGS                                                                                             \
+    q8, q_scale, static_cast<uint32_t>(blkq), nbq, k8, k_scale, kscale_shift, nbk,                                \
+        static_cast<const uint16_t *>(vt), static_cast<uint16_t *>(out), static_cast<uint32_t>(hq),               \
+        static_cast<uint32_t>(hq / hkv), lq, lk, lpad, q_sb, q_sh, q_sl, k_sb, k_sh, k_sl, o_sb, o_sh, o_sl,      \
+        sm_scale * kLog2e, plan, part
+    if (!split) {
+        sage_attn_kernel<D, kCausal, false><<<dim3(static_cast<unsigned>(grid)), kThreads, 0, s>>>(TU_ATTN_ARGS);
+    } else {
+        sage_attn_kernel<D, kCausal, true><<<dim3(static_cast<unsigned>(grid)), kThreads, 0, s>>>(TU_ATTN_ARGS);
+        constexpr int kRowsPerWg = 256 / (D / 8);
+        sage_combine_kernel<D, kCausal>
+            <<<dim3(static_cast<unsigned>((plan.part_rows + kRowsPerWg - 1) / kRowsPerWg)), 256, 0, s>>>(
+                part, plan, static_cast<uint32_t>(hq), lq, lk, static_cast<uint16_t *>(out), o_sb, o_sh, o_sl);
+    }
+#undef TU_ATTN_ARGS
+    return check_launch("tu_sage_attn_fwd");
+}
+
+// The plan that splits nothing.
+AttnPlan whole_plan(int64_t batch, int64_t hq, int64_t lq) {
+    AttnPlan p{};
+    p.nqb = static_cast<uint32_t>((lq + kBQ - 1) / kBQ);
+    p.bh = static_cast<uint32_t>(batch * hq);
+    p.split_from = 0xffffffffu;
+    p.parts = 1;
+    return p;
+}
+
+// Sets the split blocks of a plan: all blocks from `split_from` on, in ranges
+// of seg_tiles of the `tiles` key tiles of the longest block.
+void split_blocks(AttnPlan &p, int64_t split_from, int64_t seg_tiles, int64_t tiles, int64_t lq) {
+    p.split_from = static_cast<uint32_t>(split_from);
+    p.seg_tiles = static_cast<int>(seg_tiles);
+    p.parts = static_cast<uint32_t>((tiles + seg_tiles - 1) / seg_tiles);
+    p.part_row0 = split_from / p.nqb * lq + split_from % p.nqb * kBQ;
+    p.part_rows = static_cast<int64_t>(p.bh) * lq - p.part_row0;
+}
+
+int64_t plan_workspace(const AttnPlan &p, int64_t dim) {
+    return p.parts > 1 ? p.parts * p.part_rows * (dim + 2) * static_cast<int64_t>(sizeof(float)) : 0;
+}
+
+// Cost model of the automatic plan, in key tiles of one workgroup (1.26 us at
+// head_dim 128, fitted on 256 blocks over 1 .. 512 tiles).  A
+// workgroup's fixed part, its Q rows, first tile and output rows, is 7 us
+// (5 tiles); a range also writes fp32 partials (2 tiles); the merge is a
+// launch (4 tiles) and 130 KB in and out for each range.  Measured at B1 H12
+// L8190 D128 (384 blocks): 306 us and a merge of 20 us as two even ranges of
+// every block, 294 and 8 us with only the 128 blocks of the second round
+// split.
+constexpr double kFixedTiles = 5.0;
+constexpr double kSplitTiles = 2.0;
+constexpr double kMergeTiles = 4.0;
+constexpr double kMergePerPart = 0.03;
+constexpr int64_t kMinSegTiles = 8;
+
+// The cheapest plan whose workspace is at most max_bytes.
+AttnPlan auto_plan(int64_t batch, int64_t hq, int64_t lq, int64_t lk, int64_t dim, bool causal, int64_t cus,
+                   int64_t max_bytes) {
+    AttnPlan p = whole_plan(batch, hq, lq);
+    const int64_t blocks = static_cast<int64_t>(p.nqb) * p.bh;
+    const int64_t tiles = (lk + kBKey - 1) / kBKey;
+    if (blocks >= 64 * cus || p.nqb > 65536) return p;  // many rounds: nothing to even out
+    if (!causal) {
+        const int64_t full = blocks / cus * cus, rem = blocks - full;
+        double best = static_cast<double>((blocks + cus - 1) / cus) * (tiles + kFixedTiles);
+        const double base = static_cast<double>(full / cus) * (tiles + kFixedTiles);
+        AttnPlan chosen = p;
+        for (int64_t sp = 2; sp <= 16 && rem > 0; ++sp) {
+            const int64_t per = (tiles + sp - 1) / sp;
+            if (per < kMinSegTiles) break;
+            if ((tiles + per - 1) / per != sp) continue;
+            AttnPlan c = p;
+            split_blocks(c, full, per, tiles, lq);
+            if (plan_workspace(c, dim) > max_bytes) break;
+            const double cost = base + static_cast<double>((rem * sp + cus - 1) / cus) * (per + kFixedTiles + kSplitTiles) +
+                                kMergeTiles + kMergePerPart * static_cast<double>(rem * sp);
+            if (cost < best) {
+                best = cost;
+                chosen = c;
+            }
+        }
+        return chosen;
+    }
+    // Causal: the longest workgroup against the even share of all of them
+    int64_t work = 0, longest = 0;
+    for (uint32_t qb = 0; qb < p.nqb; ++qb) {
+        const int64_t t = (std::min<int64_t>(lk, (qb + int64_t{1}) * kBQ) + kBKey - 1) / kBKey;
+        work += t;
+        longest = std::max(longest, t);
+    }
+    const double even = static_cast<double>(work) * p.bh / cus;
+    double best = std::max(longest + kFixedTiles, even + kFixedTiles * blocks / cus);
+    AttnPlan chosen = p;
+    for (int64_t sp = 2; sp <= 16; ++sp) {
+        const int64_t x = (longest + 4 * sp - 1) / (4 * sp) * 4;  // multiples of 4 tiles, one query block's keys
+        if (x < kMinSegTiles) break;
+        AttnPlan c = p;
+        split_blocks(c, 0, x, longest, lq);
+        if (plan_workspace(c, dim) > max_bytes) break;
+        int64_t parts = 0, merged = 0;
+        for (uint32_t qb = 0; qb < p.nqb; ++qb) {
+            const int64_t t = (std::min<int64_t>(lk, (qb + int64_t{1}) * kBQ) + kBKey - 1) / kBKey;
+            const int64_t n = (t + x - 1) / x;
+            parts += n;
+            merged += n > 1 ? n : 0;
+        }
+        const double cost = std::max(x + kFixedTiles + kSplitTiles,
+                                     even + (kFixedTiles * parts + kSplitTiles * merged) * p.bh / cus) +
+                            kMergeTiles + kMergePerPart * static_cast<double>(merged * p.bh);
+        if (cost < best) {
+            best = cost;
+            chosen = c;
+        }
+    }
+    return chosen;
+}
+
+}  // namespace
+}  // namespace tu
+
+#define TU_LAUNCH_PLANNED(causal_)                                                                                    \
+    (dim == 128 ? (causal_ ? launch_planned<128, true>(TU_PLANNED_ARGS) : launch_planned<128, false>(TU_PLANNED_ARGS)) \
+                : (causal_ ? launch_planned<64, true>(TU_PLANNED_ARGS) : launch_planned<64, false>(TU_PLANNED_ARGS)))
+#define TU_PLANNED_ARGS                                                                                              \
+    plan, q8, q_scale, blkq, k8, k_scale, blkk, vt_bf16, lpad, o_bf16, hq, hkv, lq, lk, q_sb, q_sh, q_sl, k_sb, k_sh,  \
+        k_sl, o_sb, o_sh, o_sl, sm_scale, part, static_cast<hipStream_t>(stream)
+
 extern "C" int32_t tu_sage_attn_fwd(const int8_t *q8, const float *q_scale, int64_t blkq, const int8_t *k8,
                                     const float *k_scale, int64_t blkk, const void *vt_bf16, int64_t lpad,
                                     void *o_bf16, int64_t batch, int64_t hq, int64_t hkv, int64_t lq, int64_t lk,
@@ -740,25 +977,34 @@ extern "C" int32_t tu_sage_attn_fwd(const int8_t *q8, const float *q_scale, int6
     if (check_attn_args(q8, q_scale, blkq, k8, k_scale, blkk, vt_bf16, lpad, o_bf16, batch, hq, hkv, lq, lk, dim, q_sb,
                         q_sh, q_sl, k_sb, k_sh, k_sl, o_sb, o_sh, o_sl, sm_scale))
         return -1;
-    const dim3 grid(static_cast<unsigned>((lq + kBQ - 1) / kBQ), static_cast<unsigned>(batch * hq));
-    const float sm_log2 = sm_scale * kLog2e;
-    hipStream_t s = static_cast<hipStream_t>(stream);
-    const int groups = static_cast<int>(hq / hkv);
-    int kscale_shift = 0;
-    while ((kBKey << kscale_shift) < blkk) ++kscale_shift;
-#define TU_ATTN_ARGS                                                                                             \
-    q8, q_scale, static_cast<int>(blkq), k8, k_scale, kscale_shift, static_cast<const uint16_t *>(vt_bf16),      \
-        static_cast<uint16_t *>(o_bf16), static_cast<int>(hq), groups, lq, lk, lpad, q_sb, q_sh, q_sl, k_sb, k_sh,  \
-        k_sl, o_sb, o_sh, o_sl, sm_log2, 0, nullptr
-    if (dim == 128) {
-        if (causal) sage_attn_kernel<128, true><<<grid, kThreads, 0, s>>>(TU_ATTN_ARGS);
-        else sage_attn_kernel<128, false><<<grid, kThreads, 0, s>>>(TU_ATTN_ARGS);
-    } else {
-        if (causal) sage_attn_kernel<64, true><<<grid, kThreads, 0, s>>>(TU_ATTN_ARGS);
-        else sage_attn_kernel<64, false><<<grid, kThreads, 0, s>>>(TU_ATTN_ARGS);
-    }
-#undef TU_ATTN_ARGS
-    return check_launch("tu_sage_attn_fwd");
+    const AttnPlan plan = whole_plan(batch, hq, lq);
+    float *part = nullptr;
+    return TU_LAUNCH_PLANNED(causal);
+}
+
+extern "C" int64_t tu_sage_attn_workspace(int64_t batch, int64_t hq, int64_t lq, int64_t lk, int64_t dim,
+                                          int32_t causal, int32_t cus) {
+    using namespace tu;
+    if (batch <= 0 || hq <= 0 || lq <= 0 || lk <= 0 || dim <= 0 || cus <= 0 || batch * hq > 65535) return 0;
+    return plan_workspace(auto_plan(batch, hq, lq, lk, dim, causal != 0, cus, INT64_MAX), dim);
+}
+
+extern "C" int32_t tu_sage_attn_fwd_auto(const int8_t *q8, const float *q_scale, int64_t blkq, const int8_t *k8,
+                                         const float *k_scale, int64_t blkk, const void *vt_bf16, int64_t lpad,
+                                         void *o_bf16, int64_t batch, int64_t hq, int64_t hkv, int64_t lq, int64_t lk,
+                                         int64_t dim, int64_t q_sb, int64_t q_sh, int64_t q_sl, int64_t k_sb,
+                                         int64_t k_sh, int64_t k_sl, int64_t o_sb, int64_t o_sh, int64_t o_sl,
+                                         float sm_scale, int32_t causal, int32_t cus, void *workspace,
+                                         int64_t workspace_bytes, void *stream) {
+    using namespace tu;
+    TU_REQUIRE(cus > 0, "Sage attention: compute units must be positive, got %d", cus);
+    TU_REQUIRE((reinterpret_cast<uintptr_t>(workspace) & 15) == 0, "Sage attention workspace must be 16-byte aligned");
+    if (check_attn_args(q8, q_scale, blkq, k8, k_scale, blkk, vt_bf16, lpad, o_bf16, batch, hq, hkv, lq, lk, dim, q_sb,
+                        q_sh, q_sl, k_sb, k_sh, k_sl, o_sb, o_sh, o_sl, sm_scale))
+        return -1;
+    const AttnPlan plan = auto_plan(batch, hq, lq, lk, dim, causal != 0, cus, workspace ? workspace_bytes : 0);
+    float *part = static_cast<float *>(workspace);
+    return TU_LAUNCH_PLANNED(causal);
 }
 
 // Key splits for a grid that fills the GPU badly: a workgroup's time is about
@@ -810,28 +1056,8 @@ extern "C" int32_t tu_sage_attn_fwd_split(const int8_t *q8, const float *q_scale
     if (check_attn_args(q8, q_scale, blkq, k8, k_scale, blkk, vt_bf16, lpad, o_bf16, batch, hq, hkv, lq, lk, dim, q_sb,
                         q_sh, q_sl, k_sb, k_sh, k_sl, o_sb, o_sh, o_sl, sm_scale))
         return -1;
-    const dim3 grid(static_cast<unsigned>((lq + kBQ - 1) / kBQ), static_cast<unsigned>(batch * hq),
-                    static_cast<unsigned>(splits));
-    hipStream_t s = static_cast<hipStream_t>(stream);
-    int kscale_shift = 0;
-    while ((kBKey << kscale_shift) < blkk) ++kscale_shift;
+    AttnPlan plan = whole_plan(batch, hq, lq);
+    split_blocks(plan, 0, split_tiles, tiles, lq);
     float *part = static_cast<float *>(partial);
-#define TU_SPLIT_ARGS                                                                                            \
-    q8, q_scale, static_cast<int>(blkq), k8, k_scale, kscale_shift, static_cast<const uint16_t *>(vt_bf16),      \
-        static_cast<uint16_t *>(o_bf16), static_cast<int>(hq), static_cast<int>(hq / hkv), lq, lk, lpad, q_sb,    \
-        q_sh, q_sl, k_sb, k_sh, k_sl, o_sb, o_sh, o_sl, sm_scale * kLog2e, static_cast<int>(split_tiles), part
-    const int64_t rows = batch * hq * lq;
-    if (dim == 128) {
-        sage_attn_kernel<128, false, true><<<grid, kThreads, 0, s>>>(TU_SPLIT_ARGS);
-        sage_combine_kernel<128><<<static_cast<unsigned>((rows + 15) / 16), 256, 0, s>>>(
-            part, static_cast<int>(splits), static_cast<int>(hq), batch * hq, lq, static_cast<uint16_t *>(o_bf16),
-            o_sb, o_sh, o_sl);
-    } else {
-        sage_attn_kernel<64, false, true><<<grid, kThreads, 0, s>>>(TU_SPLIT_ARGS);
-        sage_combine_kernel<64><<<static_cast<unsigned>((rows + 31) / 32), 256, 0, s>>>(
-            part, static_cast<int>(splits), static_cast<int>(hq), batch * hq, lq, static_cast<uint16_t *>(o_bf16),
-            o_sb, o_sh, o_sl);
-    }
-#undef TU_SPLIT_ARGS
-    return check_launch("tu_sage_attn_fwd_split");
+    return TU_LAUNCH_PLANNED(false);
 }

@@ -268,6 +268,26 @@ int32_t tu_sage_attn_fwd_split(const int8_t *q8, const float *q_scale, int64_t b
  * call; no counterpart in the reference. */
 int32_t tu_sage_attn_kv_splits(int64_t batch, int64_t hq, int64_t lq, int64_t lk, int32_t causal, int32_t cus);
 
+/* The same attention, causal or not, on a work plan chosen for a GPU with
+ * `cus` compute units: non-causal, the 256-row query blocks past the last
+ * full round of `cus` run as several key ranges each (the others whole);
+ * causal, long rows run as several key ranges where whole ones would leave
+ * compute units idle.  Ranges are merged as in tu_sage_attn_fwd_split.
+ * workspace: fp32, 16-byte aligned, workspace_bytes long; the cheapest plan
+ * that fits is taken, and with none (NULL, 0) nothing is split.
+ * tu_sage_attn_workspace returns the bytes that the unrestricted plan needs
+ * (0: it splits nothing); host-only arithmetic.  No counterpart in the
+ * reference. */
+int64_t tu_sage_attn_workspace(int64_t batch, int64_t hq, int64_t lq, int64_t lk, int64_t dim, int32_t causal,
+                               int32_t cus);
+int32_t tu_sage_attn_fwd_auto(const int8_t *q8, const float *q_scale, int64_t blkq, const int8_t *k8,
+                              const float *k_scale, int64_t blkk, const void *vt_bf16, int64_t lpad,
+                              void *o_bf16, int64_t batch, int64_t hq, int64_t hkv, int64_t lq, int64_t lk,
+                              int64_t dim, int64_t q_sb, int64_t q_sh, int64_t q_sl, int64_t k_sb,
+                              int64_t k_sh, int64_t k_sl, int64_t o_sb, int64_t o_sh, int64_t o_sl,
+                              float sm_scale, int32_t causal, int32_t cus, void *workspace,
+                              int64_t workspace_bytes, void *stream);
+
 /* Sage attention: fused Q/K preprocessing -------------------------------- */
 
 /* RMSNorm + RoPE + per-tile INT8 of Q and K in one pass, the producer of the
