@@ -46,7 +46,8 @@ namespace {
 
 // Workgroup tile: BM activation rows x BN weight rows (output columns).
 // 256 x 256, or for grids that those would fill in few, partly empty rounds
-// (the tile policy) 128 x 256 or 256 x 192; the wave grid stays the same.
+// 256 x 192 and smaller ones down to 64 x 64 (pick_tile); the wave grid stays
+// the same.  Tiles under 256 rows keep a ring of 3 or 4 stages.
 constexpr int kBK = 128;  // bytes of K per step (two 64-deep MFMA slices)
 // Waves per workgroup: 2 along the weight rows x kWavesM along the activation
 // rows; each wave owns a 128 x (256 / kWavesM) output tile.
@@ -64,7 +65,7 @@ constexpr int kGroupM = 4;
 // Geometry of a workgroup tile with BM activation rows and BN weight rows.
 template <int BM, int BN>
 struct Tile {
-    static_assert((BM == 256 && (BN == 256 || BN == 192)) || (BM == 128 && BN == 256), "tile of 256 x 256, 128 x 256 or 256 x 192");
+    static_assert(BM % 64 == 0 && BN % 64 == 0 && BM <= 256 && BN <= 256, "tile sides of 64, 128, 192 or 256");
     static constexpr int kFragsM = BM / kWavesM / 16;  // 16-row activation fragments per wave
     static constexpr int kFragsN = BN / 2 / 16;        // 16-row weight fragments per wave (its half of the tile)
     static constexpr int kMma = kFragsN * kFragsM;     // MFMAs per 64-deep slice and wave
@@ -80,9 +81,11 @@ struct Tile {
     static constexpr int kChunksW = BN * 8 / kThreads;
     static constexpr int kChunks = kChunksA > kChunksW ? kChunksA : kChunksW;
     static constexpr int kRows = 16 * kFragsM;                  // activation rows per wave
-    // LDS: the K-step ring, and after the main loop each wave's 16-bit output
-    // tile (kRows rows of 256 bytes) staged for row-wide stores
-    static constexpr int kLdsBytes = 2 * kStageBytes > kWaves * kRows * 256 ? 2 * kStageBytes : kWaves * kRows * 256;
+    // LDS: the K-step ring of `stages`, and after the main loop each wave's
+    // 16-bit output tile (kRows rows of 256 bytes) staged for row-wide stores
+    static constexpr int lds_bytes(int stages) {
+        return stages * kStageBytes > kWaves * kRows * 256 ? stages * kStageBytes : kWaves * kRows * 256;
+    }
 };
 
 // LDS panel layout: 128-byte rows, the 16-byte chunk index XOR-swizzled with
@@ -153,7 +156,6 @@ __device__ __forceinline__ void tile_coords(int bid, int tiles_m, int tiles_n, i
     tile_of(t, tiles_m, tiles_n, tm, tn);
 }
 
-constexpr int kStages = 2;
 typedef __attribute__((address_space(3))) void lds_void;
 
 // Per-lane source offsets of the direct-to-LDS loads.  Wave w fills the 1 KiB
@@ -212,19 +214,31 @@ __device__ __forceinline__ const int8_t *uniform_ptr(const int8_t *p) {
                 wrs, (lds_void *)(stage + BM * kBK + (Tile<BM, BN>::kWBlocks * wave + i) * 1024), 16, gm.w_off[i], \
                 k0, 0, 0);                                                                                      \
     }
-__device__ __forceinline__ void issue_step(int8_t *stage, __amdgpu_buffer_rsrc_t ars, __amdgpu_buffer_rsrc_t wrs,
-                                           const LoadGeom<256, 256> &gm, uint32_t k0, int wave) {
-    TU_ISSUE_STEP_BODY(256, 256)
-}
-__device__ __forceinline__ void issue_step(int8_t *stage, __amdgpu_buffer_rsrc_t ars, __amdgpu_buffer_rsrc_t wrs,
-                                           const LoadGeom<128, 256> &gm, uint32_t k0, int wave) {
-    TU_ISSUE_STEP_BODY(128, 256)
-}
-__device__ __forceinline__ void issue_step(int8_t *stage, __amdgpu_buffer_rsrc_t ars, __amdgpu_buffer_rsrc_t wrs,
-                                           const LoadGeom<256, 192> &gm, uint32_t k0, int wave) {
-    TU_ISSUE_STEP_BODY(256, 192)
-}
+#define TU_ISSUE_STEP(BM, BN)                                                                                    \
+    __device__ __forceinline__ void issue_step(int8_t *stage, __amdgpu_buffer_rsrc_t ars,                         \
+                                               __amdgpu_buffer_rsrc_t wrs, const LoadGeom<BM, BN> &gm,            \
+                                               uint32_t k0, int wave) {                                           \
+        TU_ISSUE_STEP_BODY(BM, BN)                                                                              \
+    }
+TU_ISSUE_STEP(256, 256)
+TU_ISSUE_STEP(128, 256)
+TU_ISSUE_STEP(256, 192)
+TU_ISSUE_STEP(128, 192)
+TU_ISSUE_STEP(128, 128)
+TU_ISSUE_STEP(128, 64)
+TU_ISSUE_STEP(64, 64)
+#undef TU_ISSUE_STEP
 #undef TU_ISSUE_STEP_BODY
+
+// Workgroup barrier that waits for no memory and that nothing is scheduled
+// across: the ring's loads stay in flight over it.
+__device__ __forceinline__ void ring_barrier() {
+    __builtin_amdgcn_sched_barrier(0);
+    asm volatile("" ::: "memory");
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+    __builtin_amdgcn_sched_barrier(0);
+}
 
 template <int BM, int BN>
 struct Frags {
@@ -241,14 +255,24 @@ constexpr int kOutF16 = 1;   // fp16_rn of the same value (LDS-staged row stores
 constexpr int kOutF32 = 2;   // the fp32 value itself (direct 16-byte stores)
 constexpr int kOutI32 = 3;   // the int32 accumulator (direct 16-byte stores)
 
+// Two bf16 outputs of the residual epilogue: bf16_rn(fma(y, gate, residual)).
+__device__ __forceinline__ uint32_t residual_pair(uint32_t y, uint32_t r, uint32_t g) {
+    const float lo = __builtin_fmaf(__uint_as_float(y << 16), __uint_as_float(g << 16), __uint_as_float(r << 16));
+    const float hi = __builtin_fmaf(__uint_as_float(y & 0xffff0000u), __uint_as_float(g & 0xffff0000u),
+                                    __uint_as_float(r & 0xffff0000u));
+    return pack_bf16x2(lo, hi);
+}
+
 // kResidual: out = bf16_rn(fma(y, gate[row / gate_rows][col], residual[row][col]))
 // with y the bf16 epilogue value (gate 1 when absent).  residual may be out
 // (in place), so neither carries __restrict__: each output chunk is read as
 // residual and then written by the same lane, and no lane stores a chunk
 // that another lane reads (clamped reads past the last row feed only rows
 // that are never stored).
-template <int BM, int BN, int kOut, bool kResidual>
-__global__ __launch_bounds__(kThreads, kWaves / 4) void int8_gemm_kernel(
+// NST: stages of the LDS ring.  WPE: waves per SIMD, 2 (one workgroup on a
+// CU) or 4 (two).
+template <int BM, int BN, int NST, int WPE, int kOut, bool kResidual>
+__global__ __launch_bounds__(kThreads, WPE) void int8_gemm_kernel(
     const int8_t *__restrict__ a, const int8_t *__restrict__ w, const float *__restrict__ as,
     const float *__restrict__ ws, const float *__restrict__ bias, void *out,
     int64_t m, int64_t n, int64_t k, int tiles_m, int tiles_n, const uint16_t *residual, const uint16_t *gate,
@@ -257,7 +281,7 @@ __global__ __launch_bounds__(kThreads, kWaves / 4) void int8_gemm_kernel(
     constexpr int kFragsM = Tile<BM, BN>::kFragsM;
     constexpr int kFragsN = Tile<BM, BN>::kFragsN;
     constexpr int kStageBytes = Tile<BM, BN>::kStageBytes;
-    __shared__ __align__(1024) int8_t lds_mem[Tile<BM, BN>::kLdsBytes];
+    __shared__ __align__(1024) int8_t lds_mem[Tile<BM, BN>::lds_bytes(NST)];
     auto lds = [&](int st) { return lds_mem + st * kStageBytes; };
 
     const int tid = threadIdx.x;
@@ -329,45 +353,68 @@ __global__ __launch_bounds__(kThreads, kWaves / 4) void int8_gemm_kernel(
 
     const int full = static_cast<int>(k / kBK);
     if (full > 0) {
-        issue_step(lds(0), ars, wrs, gm, 0, wave);
-        if (full > 1) issue_step(lds(1), ars, wrs, gm, kBK, wave);
-        if (full > 1) __builtin_amdgcn_s_waitcnt(vmcnt_imm(Tile<BM, BN>::kLoads));
-        else __builtin_amdgcn_s_waitcnt(vmcnt_imm(0));
-        __syncthreads();
+        if constexpr (NST == 2) {
+            issue_step(lds(0), ars, wrs, gm, 0, wave);
+            if (full > 1) issue_step(lds(1), ars, wrs, gm, kBK, wave);
+            if (full > 1) __builtin_amdgcn_s_waitcnt(vmcnt_imm(Tile<BM, BN>::kLoads));
+            else __builtin_amdgcn_s_waitcnt(vmcnt_imm(0));
+            __syncthreads();
+        } else {
+            // steps past the last one load it again, so the counts below hold
+#pragma unroll
+            for (int st = 0; st < NST; ++st)
+                issue_step(lds(st), ars, wrs, gm, static_cast<uint32_t>(min(st, full - 1) * kBK), wave);
+            __builtin_amdgcn_s_waitcnt(vmcnt_imm((NST - 1) * Tile<BM, BN>::kLoads));
+            ring_barrier();
+        }
         Frags<BM, BN> f0, f1;
         load_frags(f0, lds(0), 0);
         __builtin_amdgcn_s_waitcnt(lgkmcnt_imm(0));
         // One K step:
         //   slice 1 reads, with the first kPre MFMAs of slice 0 covering them
         //   barrier: step s + 1 resident, every wave done reading stage s
-        //   rest of slice 0, interleaved with the loads of step s + 2
+        //   rest of slice 0, interleaved with the loads of step s + NST
         //   slice 1, interleaved with the reads of slice 0 of step s + 1
         // so the MFMA pipe has work on both sides of the barrier.  Slice 0's
         // fragments are in registers when a step starts (their reads retire
         // at the end of the previous step), so only 12 LDS reads are ever in
         // flight and no MFMA waits on one (with more than 15 in flight the
         // compiler can only wait for all of them).  The loop body has no
-        // branches, which the register allocation needs: the last two steps
+        // branches, which the register allocation needs: the last NST steps
         // load step full - 1 again into stages nobody reads any more, and
         // those loads are retired after the loop, before the ring is reused.
+        // Two stages: a step waits for all of its loads.  More stages: only
+        // for the next step's, so loads stay in flight over the barrier
+        // (128 x 256 at 128 x 5120 x 5120: 39.3 us with two stages, 32.4
+        // with three).
         constexpr int kMma = Tile<BM, BN>::kMma, kPre = Tile<BM, BN>::kPre;
 #pragma clang loop unroll(disable)
-        for (int s = 0; s < full; ++s) {
-            const uint32_t k2 = static_cast<uint32_t>(min(s + 2, full - 1) * kBK);
-            load_frags(f1, lds(s & 1), 1);
+        for (int s = 0, cur = 0; s < full; ++s) {
+            const uint32_t k2 = static_cast<uint32_t>(min(s + NST, full - 1) * kBK);
+            const int nxt = NST == 2 ? (s + 1) & 1 : cur + 1 == NST ? 0 : cur + 1;
+            load_frags(f1, lds(cur), 1);
             mma_part(f0, 0, kPre);
             __builtin_amdgcn_sched_barrier(0);
-            __builtin_amdgcn_s_waitcnt(vmcnt_imm(0));
-            __syncthreads();
-            issue_step(lds(s & 1), ars, wrs, gm, k2, wave);
+            if constexpr (NST == 2) {
+                __builtin_amdgcn_s_waitcnt(vmcnt_imm(0));
+                __syncthreads();
+            } else {
+                // step s + 1 resident, this wave's reads of stage s retired;
+                // the loads of the steps after it stay in flight
+                __builtin_amdgcn_s_waitcnt(vmcnt_imm((NST - 2) * Tile<BM, BN>::kLoads) & lgkmcnt_imm(0));
+                ring_barrier();
+            }
+            issue_step(lds(cur), ars, wrs, gm, k2, wave);
             mma_part(f0, kPre, kMma);
+            // spread over the MFMAs: 0.5-1 % faster than one load per MFMA
+            constexpr int kPerLoad = (kMma - kPre) / Tile<BM, BN>::kLoads;
 #pragma unroll
             for (int i = 0; i < Tile<BM, BN>::kLoads; ++i) {
                 __builtin_amdgcn_sched_group_barrier(0x020, 1, 0);
-                __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+                __builtin_amdgcn_sched_group_barrier(0x008, kPerLoad > 1 ? kPerLoad : 1, 0);
             }
             __builtin_amdgcn_sched_barrier(0);
-            load_frags(f0, lds((s + 1) & 1), 0);
+            load_frags(f0, lds(nxt), 0);
             mma(f1);
 #pragma unroll
             for (int i = 0; i < kFragsN + kFragsM; ++i) {
@@ -377,6 +424,7 @@ __global__ __launch_bounds__(kThreads, kWaves / 4) void int8_gemm_kernel(
             __builtin_amdgcn_sched_barrier(0);
             __builtin_amdgcn_s_waitcnt(lgkmcnt_imm(0));
             __builtin_amdgcn_sched_barrier(0);
+            cur = nxt;
         }
         __builtin_amdgcn_s_waitcnt(vmcnt_imm(0));
     }
@@ -553,14 +601,7 @@ __global__ __launch_bounds__(kThreads, kWaves / 4) void int8_gemm_kernel(
             u32x4 val = *reinterpret_cast<const u32x4 *>(tile + lrow * 256 + ((c ^ (lrow & 15)) << 4));
             if constexpr (kResidual) {
 #pragma unroll
-                for (int e = 0; e < 4; ++e) {
-                    const uint32_t y = val[e], r = res[pass][e], gg = gv[pass][e];
-                    const float lo = __builtin_fmaf(__uint_as_float(y << 16), __uint_as_float(gg << 16),
-                                                    __uint_as_float(r << 16));
-                    const float hi = __builtin_fmaf(__uint_as_float(y & 0xffff0000u), __uint_as_float(gg & 0xffff0000u),
-                                                    __uint_as_float(r & 0xffff0000u));
-                    val[e] = pack_bf16x2(lo, hi);
-                }
+                for (int e = 0; e < 4; ++e) val[e] = residual_pair(val[e], res[pass][e], gv[pass][e]);
             }
             if (row < m && col < n && c < BN / 16)  // n % 8 == 0: a chunk is all in or all out
                 __builtin_nontemporal_store(val, reinterpret_cast<u32x4 *>(static_cast<uint16_t *>(out) + row * n + col));
@@ -622,9 +663,11 @@ constexpr double kHalfTileCost = TU_GEMM_HALF_TILE_COST;
 // K 5120 (0.75 of the MFMAs plus the fixed part).
 constexpr double kTile192Cost = 0.85;
 
-// Tile policy from the grid: one workgroup per CU, so tiles run in rounds of
-// `cus`; 128 x 256 or 256 x 192 tiles are chosen when their rounds cost less
-// than the 256 x 256 tiles' (a grid of a few, partly empty rounds).
+// The choice among the three tiles of tu_int8_gemm_ex from the grid alone: one
+// workgroup per CU, so tiles run in rounds of `cus`; 128 x 256 or 256 x 192
+// tiles are chosen when their rounds cost less than the 256 x 256 tiles' (a
+// grid of a few, partly empty rounds).  A launch that is left to choose
+// (pick_tile below) knows K and the smaller tiles too.
 int pick_tile_policy(int64_t m, int64_t n, int cus) {
     const int64_t t256 = (m + 255) / 256 * ((n + 255) / 256);
     const int64_t t128 = (m + 127) / 128 * ((n + 255) / 256);
@@ -637,6 +680,51 @@ int pick_tile_policy(int64_t m, int64_t n, int cus) {
     return TU_GEMM_TILE_256;
 }
 
+// Tiles that only the automatic choice takes (numbers of launch_gemm's own).
+constexpr int kTile128x192 = 16, kTile128x128 = 17, kTile128x64 = 18, kTile64x64 = 19;
+
+// Automatic tile: the least of first + rounds * (fixed + per_step * steps),
+// rounds = tiles / CUs rounded up and steps of 128 bytes of K, in us.  The
+// constants are fitted to times at K 1536 and 5120 with one and several
+// rounds (graph of 12 launches, bf16 out with bias, three operand sets).  A
+// step of a small grid costs the bytes that a CU pulls past its L2, about 70
+// GB/s, so its time goes with BM + BN whatever the MFMAs do; the fewer
+// columns and rows a CU has to pull while all CUs have a tile, the better,
+// and the smallest two tiles leave room for a second workgroup on the CU.
+//   M x N x K             before (128 x 256 x 2 stages)   now
+//   1 x 9216 x 1536       14.3 us                          6.8 us (64 x 64)
+//   128 x 5120 x 5120     39.3                             12.6 (64 x 64)
+//   1024 x 1536 x 1536    16.2                             8.5 (128 x 64)
+//   512 x 5120 x 5120     38.8                             22.5 (128 x 128)
+//   512 x 10240 x 5120    39.4                             30.0 (128 x 192)
+// 256 x 192 stays best from 1024 x 8960 x 1536 (20.2 us against 25.5 with
+// 128 x 192) and 256 x 256 from about ten rounds on.
+struct TileCost {
+    int policy, bm, bn;
+    double first, fixed, per_step;
+};
+constexpr TileCost kTileCosts[] = {
+    {TU_GEMM_TILE_256, 256, 256, 1.5, 10.0, 1.125}, {TU_GEMM_TILE_192, 256, 192, 1.5, 8.7, 0.957},
+    {TU_GEMM_TILE_128, 128, 256, 1.5, 5.3, 0.668},  {kTile128x192, 128, 192, 1.5, 3.9, 0.56},
+    {kTile128x128, 128, 128, 1.5, 3.2, 0.44},       {kTile128x64, 128, 64, 3.0, 1.6, 0.27},
+    {kTile64x64, 64, 64, 2.3, 1.65, 0.178},
+};
+
+int pick_tile(int64_t m, int64_t n, int64_t k, int cus) {
+    const double steps = static_cast<double>((k + kBK - 1) / kBK);
+    int best = TU_GEMM_TILE_256;
+    double best_cost = 0.0;
+    for (const TileCost &t : kTileCosts) {
+        const int64_t tiles = (m + t.bm - 1) / t.bm * ((n + t.bn - 1) / t.bn);
+        const double cost = t.first + static_cast<double>((tiles + cus - 1) / cus) * (t.fixed + t.per_step * steps);
+        if (&t == kTileCosts || cost < best_cost) {
+            best = t.policy;
+            best_cost = cost;
+        }
+    }
+    return best;
+}
+
 template <int kOut, bool kResidual = false>
 int32_t launch_gemm(const int8_t *a, const int8_t *w, const float *as, const float *ws, const float *bias,
                     void *out, int64_t m, int64_t n, int64_t k, void *stream, const uint16_t *residual = nullptr,
@@ -645,22 +733,25 @@ int32_t launch_gemm(const int8_t *a, const int8_t *w, const float *as, const flo
     if (policy == TU_GEMM_TILE_AUTO) {
         int cus = 0;
         if (device_cus(cus)) return -1;
-        policy = pick_tile_policy(m, n, cus);
+        policy = pick_tile(m, n, k, cus);
     }
     hipStream_t st = static_cast<hipStream_t>(stream);
-    if (policy == TU_GEMM_TILE_128) {
-        const int tiles_m = static_cast<int>((m + 127) / 128), tiles_n = static_cast<int>((n + 255) / 256);
-        int8_gemm_kernel<128, 256, kOut, kResidual><<<dim3(tiles_m * tiles_n), kThreads, 0, st>>>(
-            a, w, as, ws, bias, out, m, n, k, tiles_m, tiles_n, residual, gate, gate_rows);
-    } else if (policy == TU_GEMM_TILE_192) {
-        const int tiles_m = static_cast<int>((m + 255) / 256), tiles_n = static_cast<int>((n + 191) / 192);
-        int8_gemm_kernel<256, 192, kOut, kResidual><<<dim3(tiles_m * tiles_n), kThreads, 0, st>>>(
-            a, w, as, ws, bias, out, m, n, k, tiles_m, tiles_n, residual, gate, gate_rows);
-    } else {
-        const int tiles_m = static_cast<int>((m + 255) / 256), tiles_n = static_cast<int>((n + 255) / 256);
-        int8_gemm_kernel<256, 256, kOut, kResidual><<<dim3(tiles_m * tiles_n), kThreads, 0, st>>>(
-            a, w, as, ws, bias, out, m, n, k, tiles_m, tiles_n, residual, gate, gate_rows);
+#define TU_TILE(BM, BN, NST, WPE)                                                                                 \
+    do {                                                                                                        \
+        const int tiles_m = static_cast<int>((m + BM - 1) / BM), tiles_n = static_cast<int>((n + BN - 1) / BN);     \
+        int8_gemm_kernel<BM, BN, NST, WPE, kOut, kResidual><<<dim3(tiles_m * tiles_n), kThreads, 0, st>>>(           \
+            a, w, as, ws, bias, out, m, n, k, tiles_m, tiles_n, residual, gate, gate_rows);                      \
+    } while (0)
+    switch (policy) {
+    case TU_GEMM_TILE_128: TU_TILE(128, 256, 3, 2); break;
+    case TU_GEMM_TILE_192: TU_TILE(256, 192, 2, 2); break;
+    case kTile128x192: TU_TILE(128, 192, 3, 2); break;
+    case kTile128x128: TU_TILE(128, 128, 4, 2); break;
+    case kTile128x64: TU_TILE(128, 64, 3, 4); break;
+    case kTile64x64: TU_TILE(64, 64, 4, 4); break;
+    default: TU_TILE(256, 256, 2, 2); break;
     }
+#undef TU_TILE
     return check_launch(kOut == kOutI32   ? "tu_int8_gemm_i32"
                         : kResidual       ? "tu_int8_gemm_bf16_residual"
                         : kOut == kOutF16 ? "tu_int8_gemm_f16"

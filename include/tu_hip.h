@@ -115,7 +115,7 @@ int32_t tu_int8_gemm_f32(const int8_t *a, const int8_t *w, const float *a_scale,
 #define TU_OUT_F16 1
 #define TU_OUT_F32 2
 #define TU_OUT_I32 3
-#define TU_GEMM_TILE_AUTO 0 /* chosen from the grid: tu_int8_gemm_tile_policy */
+#define TU_GEMM_TILE_AUTO 0 /* chosen by m, n, k and the compute units, smaller tiles included */
 #define TU_GEMM_TILE_256 1  /* 256 x 256 output tiles */
 #define TU_GEMM_TILE_128 2  /* 128 (rows of a) x 256 output tiles */
 #define TU_GEMM_TILE_192 3  /* 256 (rows of a) x 192 output tiles */
@@ -130,9 +130,11 @@ int32_t tu_int8_gemm_ex(const int8_t *a, const int8_t *w, const float *a_scale, 
                         const float *bias, void *out, int32_t out_type, int64_t m, int64_t n, int64_t k,
                         int32_t tile_policy, void *stream);
 
-/* The tile policy TU_GEMM_TILE_AUTO picks for an m x n output on a device
+/* The choice among the three tile policies for an m x n output on a device
  * with `cus` compute units: TU_GEMM_TILE_128 or TU_GEMM_TILE_192 when that
- * tile's rounds of `cus` workgroups cost less than the 256 x 256 tiles'
+ * tile's rounds of `cus` workgroups cost less than the 256 x 256 tiles'.
+ * TU_GEMM_TILE_AUTO also weighs k and tiles down to 64 x 64, which have no
+ * policy number: every tile gives the same bits
  * (host only, no HIP call).  Counterpart of the heuristic of
  * w4a8.cu:837-851. */
 int32_t tu_int8_gemm_tile_policy(int64_t m, int64_t n, int32_t cus);
