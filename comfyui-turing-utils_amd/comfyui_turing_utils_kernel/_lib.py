@@ -76,6 +76,14 @@ SIGNATURES: dict[str, tuple[object, list[object]]] = {
         _i32,
         [_c_void_p, _i64, _i64, _i64, _i64, _i64, _i64, _i64, _c_void_p, _i64, _c_void_p],
     ),
+    "tu_sage_prep_workspace": (_i64, [_i64, _i64, _i64, _i64, _i32]),
+    "tu_sage_prep": (
+        _i32,
+        [_c_void_p, _c_void_p, _c_void_p, _i64, _i64, _i64, _i64, _i64, _i64,
+         _i64, _i64, _i64, _i64, _i64, _i64, _i64, _i64, _i64, _i32, _i64, _i64,
+         _c_void_p, _i64, _i64, _i64, _c_void_p, _i64, _i64, _i64, _c_void_p, _c_void_p, _c_void_p, _i64,
+         _c_void_p, _i64, _c_void_p],
+    ),
     "tu_sage_attn_fwd": (
         _i32,
         [_c_void_p, _c_void_p, _i64, _c_void_p, _c_void_p, _i64, _c_void_p, _i64, _c_void_p,
@@ -147,7 +155,7 @@ SIGNATURES: dict[str, tuple[object, list[object]]] = {
     ),
 }
 
-ABI_VERSION = 14
+ABI_VERSION = 15
 
 _lock = threading.Lock()
 _lib: ctypes.CDLL | None = None

@@ -30,10 +30,9 @@ from .. import _lib
 from .quant import (
     SUPPORTED_BLOCKS,
     _layout_dims,
-    per_block_int8,
     per_warp_int8_hadamard,
     quantize_v_int8,
-    rms_rope_per_warp_int8,
+    sage_prologue,
     value_transpose,
 )
 
@@ -145,11 +144,8 @@ def prequantize_sageattn(
     output_dtype = q.dtype
     width = _sage_head_dim(head_dim)
     qp, kp, vp = _prepare(q, width), _prepare(k, width), _prepare(v, width)
-    with torch.cuda.device(q.device):
-        q_int8, q_scale, k_int8, k_scale, _ = per_block_int8(
-            qp, kp, BLKQ=BLKQ, BLKK=BLKK, tensor_layout=tensor_layout, smooth_k=smooth_k
-        )
-        value_t, _ = value_transpose(vp, tensor_layout)
+    q_int8, q_scale, k_int8, k_scale, value_t = sage_prologue(
+        qp, kp, vp, BLKQ=BLKQ, BLKK=BLKK, tensor_layout=tensor_layout, smooth_k=smooth_k)
     return PrequantizedSageAttention(
         query_int8=q_int8, query_scale=q_scale, key_int8=k_int8, key_scale=k_scale, value_t=value_t,
         tensor_layout=tensor_layout, original_head_dim=head_dim, is_causal=bool(is_causal),

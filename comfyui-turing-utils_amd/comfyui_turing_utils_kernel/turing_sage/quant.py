@@ -90,6 +90,42 @@ def value_transpose(v: torch.Tensor, tensor_layout: str = "HND") -> tuple[torch.
     return vt, lpad
 
 
+def sage_prologue(
+    q: torch.Tensor,
+    k: torch.Tensor,
+    v: torch.Tensor,
+    BLKQ: int = 128,
+    BLKK: int = 128,
+    tensor_layout: str = "HND",
+    smooth_k: bool = True,
+) -> tuple[torch.Tensor, torch.Tensor, torch.Tensor, torch.Tensor, torch.Tensor]:
+    """``per_block_int8`` of Q and K and ``value_transpose`` of V in one call
+    (two or three launches): (q_int8, q_scale, k_int8, k_scale, value_t)."""
+    hq, lq, *q_strides = _layout_dims(q, tensor_layout)
+    hkv, lk, *k_strides = _layout_dims(k, tensor_layout)
+    _, _, *v_strides = _layout_dims(v, tensor_layout)
+    batch, dim, device = q.size(0), q.size(-1), q.device
+    lpad = (lk + 63) // 64 * 64
+    if batch * (hkv * (lpad // 32) + hq * ((lq + BLKQ - 1) // BLKQ)) > 1 << 23:
+        # past the one grid of the shared launch: every part by itself
+        q_int8, q_scale, k_int8, k_scale, _ = per_block_int8(q, k, BLKQ, BLKK, tensor_layout, smooth_k)
+        return q_int8, q_scale, k_int8, k_scale, value_transpose(v, tensor_layout)[0]
+    q_int8 = torch.empty(q.shape, dtype=torch.int8, device=device)
+    k_int8 = torch.empty(k.shape, dtype=torch.int8, device=device)
+    q_scale = torch.empty((batch, hq, (lq + BLKQ - 1) // BLKQ), dtype=torch.float32, device=device)
+    k_scale = torch.empty((batch, hkv, (lk + BLKK - 1) // BLKK), dtype=torch.float32, device=device)
+    value_t = torch.empty((batch, hkv, dim, lpad), dtype=torch.bfloat16, device=device)
+    nbytes = int(_lib.load().tu_sage_prep_workspace(batch, hkv, lk, dim, int(smooth_k)))
+    workspace = torch.empty(nbytes, dtype=torch.uint8, device=device) if nbytes else None
+    with torch.cuda.device(device):
+        _lib.call("tu_sage_prep", q.data_ptr(), k.data_ptr(), v.data_ptr(), batch, hq, hkv, lq, lk, dim, *q_strides,
+                  *k_strides, *v_strides, int(smooth_k), BLKQ, BLKK, q_int8.data_ptr(),
+                  *_layout_dims(q_int8, tensor_layout)[2:], k_int8.data_ptr(), *_layout_dims(k_int8, tensor_layout)[2:],
+                  q_scale.data_ptr(), k_scale.data_ptr(), value_t.data_ptr(), lpad, _lib.ptr(workspace), nbytes,
+                  _lib.stream_of(device))
+    return q_int8, q_scale, k_int8, k_scale, value_t
+
+
 def rms_rope_per_warp_int8(
     q: torch.Tensor,
     k: torch.Tensor,

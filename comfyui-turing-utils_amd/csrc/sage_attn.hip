@@ -41,6 +41,7 @@
 #include <type_traits>
 
 #include "attn_common.h"
+#include "sage_prep.h"
 
 namespace tu {
 namespace {
@@ -673,44 +674,12 @@ __global__ __launch_bounds__(kThreads, 1) void sage_attn_kernel(
     }
 }
 
-// V [key][d] (bf16, strides) -> V^T [b][h][d][lpad] with zero keys in [lk, lpad).
-// One workgroup per 64-key tile: 64 x 128 staged through LDS (rows padded to
-// 132 elements so the column reads are bank-conflict free).
 template <int D>
-__global__ __launch_bounds__(256) void v_prep_kernel(const uint16_t *__restrict__ v, int64_t lk, int64_t lpad,
-                                                     int64_t v_sb, int64_t v_sh, int64_t v_sl,
-                                                     uint16_t *__restrict__ vt) {
-    constexpr int kChunks = D / 8;             // 16-byte chunks of a key row
-    constexpr int kRowsPerPass = 256 / kChunks;
-    __shared__ uint16_t tile[kBKey][D + 4];
-    const int tid = threadIdx.x;
-    const int64_t key0 = static_cast<int64_t>(blockIdx.x) * kBKey;
-    const int64_t h = blockIdx.y, b = blockIdx.z, heads = gridDim.y;
-    const uint16_t *vp = v + b * v_sb + h * v_sh;
-#pragma unroll
-    for (int i = 0; i < kBKey / kRowsPerPass; ++i) {
-        const int row = i * kRowsPerPass + tid / kChunks;
-        const int c = tid % kChunks;
-        u32x4 val = u32x4{0u, 0u, 0u, 0u};
-        if (key0 + row < lk) val = *reinterpret_cast<const u32x4 *>(vp + (key0 + row) * v_sl + c * 8);
-#pragma unroll
-        for (int e = 0; e < 4; ++e) {
-            tile[row][c * 8 + 2 * e] = static_cast<uint16_t>(val[e] & 0xffffu);
-            tile[row][c * 8 + 2 * e + 1] = static_cast<uint16_t>(val[e] >> 16);
-        }
-    }
-    __syncthreads();
-    uint16_t *dst = vt + (b * heads + h) * D * lpad + key0;
-#pragma unroll
-    for (int i = 0; i < D * 8 / 256; ++i) {
-        const int item = tid + 256 * i;  // (d, 8-key chunk)
-        const int d = item >> 3, c = item & 7;
-        u32x4 out;
-#pragma unroll
-        for (int e = 0; e < 4; ++e)
-            out[e] = static_cast<uint32_t>(tile[c * 8 + 2 * e][d]) | (static_cast<uint32_t>(tile[c * 8 + 2 * e + 1][d]) << 16);
-        *reinterpret_cast<u32x4 *>(dst + d * lpad + c * 8) = out;
-    }
+__global__ __launch_bounds__(kPrepThreads) void v_prep_kernel(const uint16_t *__restrict__ v, int64_t lk, int64_t lpad,
+                                                              int64_t v_sb, int64_t v_sh, int64_t v_sl,
+                                                              uint16_t *__restrict__ vt) {
+    __shared__ uint16_t tile[kPrepKeys][D + 4];
+    v_prep_tile<D>(v, lk, lpad, v_sb, v_sh, v_sl, vt, blockIdx.x, blockIdx.y, blockIdx.z, gridDim.y, tile);
 }
 
 // Merges the key-range partials of sage_attn_kernel<D, ., true>: per

@@ -221,6 +221,22 @@ int32_t tu_sage_quant(const void *x_bf16, const void *mean_bf16, int64_t batch, 
 int32_t tu_sage_v_prep(const void *v_bf16, int64_t batch, int64_t heads, int64_t len, int64_t dim,
                        int64_t s_b, int64_t s_h, int64_t s_l, void *vt_bf16, int64_t lpad, void *stream);
 
+/* The whole prologue of one attention call: tu_sage_quant of Q (no mean),
+ * with smooth_k tu_sage_kmean of K, tu_sage_quant of K (with that mean) and
+ * tu_sage_v_prep of V, the same bits in two launches (three past 8192 keys).
+ * Strides, shapes and alignments as in those; blkq 16, 32, 64 or 128, blkk 64
+ * or 128.  workspace: 16-byte aligned, at least
+ * tu_sage_prep_workspace(batch, hkv, lk, dim, smooth_k) bytes (0 without
+ * smoothing).  No counterpart in the reference. */
+int64_t tu_sage_prep_workspace(int64_t batch, int64_t hkv, int64_t lk, int64_t dim, int32_t smooth_k);
+int32_t tu_sage_prep(const void *q_bf16, const void *k_bf16, const void *v_bf16, int64_t batch, int64_t hq,
+                     int64_t hkv, int64_t lq, int64_t lk, int64_t dim, int64_t q_sb, int64_t q_sh, int64_t q_sl,
+                     int64_t k_sb, int64_t k_sh, int64_t k_sl, int64_t v_sb, int64_t v_sh, int64_t v_sl,
+                     int32_t smooth_k, int64_t blkq, int64_t blkk, int8_t *q8, int64_t q8_sb, int64_t q8_sh,
+                     int64_t q8_sl, int8_t *k8, int64_t k8_sb, int64_t k8_sh, int64_t k8_sl, float *q_scale,
+                     float *k_scale, void *vt_bf16, int64_t lpad, void *workspace, int64_t workspace_bytes,
+                     void *stream);
+
 /* Sage attention: forward --------------------------------------------------- */
 
 /* O = softmax(Q K^T * sm_scale) V on INT8 Q/K and bf16 V:
