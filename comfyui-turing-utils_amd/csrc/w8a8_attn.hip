@@ -14,8 +14,8 @@
 // The masked score is the reference's finite -5e6 in the raw score domain.
 //
 // MI355X mapping (shared with the Sage kernel: 8 wave64, two groups of 4
-// whose MFMA and softmax clusters interleave, 32 query rows a wave, a
-// 4-stage LDS ring filled by buffer_load ... lds from group 0):
+// whose MFMA and softmax clusters interleave, 32 query rows a wave (16 where
+// the grid would leave compute units idle), a 4-stage LDS ring filled by buffer_load ... lds from group 0):
 //   * S^T = K Q^T on v_mfma_i32_16x16x64_i8 as in the Sage kernel, with the
 //     K rows permuted so that lane group g holds the 16 consecutive keys
 //     16 g .. 16 g + 15 of each query: exactly one 16-byte B operand of the
@@ -36,6 +36,7 @@
 //   * V^T arrives channel-major as INT8 codes [d][key] (keys padded to a
 //     multiple of 64 with zeros) from tu_w8a8_quant_v: the V^T stage is
 //     8 KiB, half of the Sage kernel's bf16 stage.
+#include <algorithm>
 #include <type_traits>
 
 #include "attn_common.h"
@@ -45,9 +46,7 @@ namespace {
 
 constexpr int kThreads = 512;
 constexpr int kD = 128;
-constexpr int kQT = 2;
-constexpr int kWaveQ = 16 * kQT;
-constexpr int kBQ = 8 * kWaveQ;
+constexpr int kBQ = 256;                   // query rows of a whole block: 8 waves of QT = 2 16-row fragments
 constexpr int kBKey = 64;
 constexpr int kKTileBytes = kBKey * kD;   // int8 K tile, 8 KiB
 constexpr int kVTileBytes = kD * kBKey;   // int8 V^T tile, 8 KiB
@@ -112,14 +111,15 @@ __device__ __forceinline__ void issue_tile8(int8_t *stage, __amdgpu_buffer_rsrc_
                                                  gm.v_src[i], key0, 0, 0);
 }
 
-__device__ __forceinline__ void qk_tile8(const int8_t *stage, const LaneGeom8 &gm, const i32x4 (&qf)[kQT][2],
-                                         i32x4 (&s)[4][kQT]) {
+template <int QT>
+__device__ __forceinline__ void qk_tile8(const int8_t *stage, const LaneGeom8 &gm, const i32x4 (&qf)[QT][2],
+                                         i32x4 (&s)[4][QT]) {
 #pragma unroll
     for (int kt = 0; kt < 4; ++kt) {
         const i32x4 kf0 = *reinterpret_cast<const i32x4 *>(stage + gm.k_rd[0] + kt * 16 * 128);
         const i32x4 kf1 = *reinterpret_cast<const i32x4 *>(stage + gm.k_rd[1] + kt * 16 * 128);
 #pragma unroll
-        for (int qt = 0; qt < kQT; ++qt) {
+        for (int qt = 0; qt < QT; ++qt) {
             const i32x4 z = __builtin_amdgcn_mfma_i32_16x16x64_i8(kf0, qf[qt][0], i32x4{kBias, kBias, kBias, kBias},
                                                                   0, 0, 0);
             s[kt][qt] = __builtin_amdgcn_mfma_i32_16x16x64_i8(kf1, qf[qt][1], z, 0, 0, 0);
@@ -134,21 +134,22 @@ __device__ __forceinline__ void qk_tile8(const int8_t *stage, const LaneGeom8 &g
 // running maximum rescales nothing (O / l does not depend on the base).  The
 // fixed base moves up to m_used, with acc_o and l rescaled, only when beta
 // passes kRebase.
+template <int QT>
 struct W8State {
-    float m_used[kQT];
-    float beta[kQT];
-    float l[kQT];
-    f32x4 acc_o[8][kQT];
-    i32x4 acc_i[8][kQT];
-    int seg[kQT];
+    float m_used[QT];
+    float beta[QT];
+    float l[QT];
+    f32x4 acc_o[8][QT];
+    i32x4 acc_i[8][QT];
+    int seg[QT];
 };
 constexpr float kRebase = 0x1p64f;
 
-template <bool kCausal>
-__device__ __forceinline__ void mask_tile8(i32x4 (&s)[4][kQT], int key_lim, int q_rel, int g, int lc) {
+template <bool kCausal, int QT>
+__device__ __forceinline__ void mask_tile8(i32x4 (&s)[4][QT], int key_lim, int q_rel, int g, int lc) {
     const int masked = __float_as_int(kMaskedF);
 #pragma unroll
-    for (int qt = 0; qt < kQT; ++qt) {
+    for (int qt = 0; qt < QT; ++qt) {
         // key = 16 g + c with c = 4 kt + r; masked iff c > t
         int t = key_lim - 1 - 16 * g;
         if constexpr (kCausal) t = min(t, q_rel + 16 * qt + lc - 16 * g);
@@ -165,8 +166,8 @@ __device__ __forceinline__ void mask_tile8(i32x4 (&s)[4][kQT], int key_lim, int 
 
 // Adds fragment qt's int32 segment [st.seg[qt], tile) to acc_o: acc_i holds
 // -(P . v8) exactly, so acc_o += float(acc_i) * -beta; then clears acc_i.
-template <int qt>
-__device__ __forceinline__ void flush_fragment(W8State &st, int tile) {
+template <int qt, int QT>
+__device__ __forceinline__ void flush_fragment(W8State<QT> &st, int tile) {
     if (tile > st.seg[qt]) {
 #pragma unroll
         for (int ds = 0; ds < 8; ++ds) {
@@ -180,17 +181,18 @@ __device__ __forceinline__ void flush_fragment(W8State &st, int tile) {
     st.seg[qt] = tile;
 }
 
-// Flushes both fragments (at the end of the key range).
-__device__ __forceinline__ void flush_segment(W8State &st, int tile) {
+// Flushes every fragment (at the end of the key range).
+template <int QT>
+__device__ __forceinline__ void flush_segment(W8State<QT> &st, int tile) {
     flush_fragment<0>(st, tile);
-    flush_fragment<1>(st, tile);
+    if constexpr (QT > 1) flush_fragment<1>(st, tile);
 }
 
 // The reference's exact running maximum of fragment qt: when some row's
 // maximum moves (or the int32 headroom runs out), only this fragment's
 // segment is flushed.
-template <int qt>
-__device__ __forceinline__ void move_max(W8State &st, const float (&mlane)[kQT], int tile) {
+template <int qt, int QT>
+__device__ __forceinline__ void move_max(W8State<QT> &st, const float (&mlane)[QT], int tile) {
     if (__any(mlane[qt] > st.m_used[qt]) || tile - st.seg[qt] >= kFlushTiles) {
         flush_fragment<qt>(st, tile);
         const float mx = xmax_f32(mlane[qt]);
@@ -218,11 +220,12 @@ __device__ __forceinline__ i32x4 neg127_operand() {
 // Softmax of tile `tile`: new row maxima (with the u8 offset), flush and
 // rescale when one moved, then 127 - P packed as the PV B operands p8[qt]
 // (dword kt = keys 16 g + 4 kt .. + 3 of query 16 qt + lc) and l += p.
-__device__ __forceinline__ void softmax_tile8(const i32x4 (&s)[4][kQT], const float (&f)[kQT], W8State &st,
-                                              i32x4 (&p8)[kQT], int tile) {
-    float mlane[kQT];
+template <int QT>
+__device__ __forceinline__ void softmax_tile8(const i32x4 (&s)[4][QT], const float (&f)[QT], W8State<QT> &st,
+                                              i32x4 (&p8)[QT], int tile) {
+    float mlane[QT];
 #pragma unroll
-    for (int qt = 0; qt < kQT; ++qt) {
+    for (int qt = 0; qt < QT; ++qt) {
         int mi = imax3(s[0][qt][0], s[0][qt][1], s[0][qt][2]);
         mi = imax3(mi, s[0][qt][3], s[1][qt][0]);
         mi = imax3(mi, s[1][qt][1], s[1][qt][2]);
@@ -234,17 +237,17 @@ __device__ __forceinline__ void softmax_tile8(const i32x4 (&s)[4][kQT], const fl
         mlane[qt] = __builtin_fmaf(__int_as_float(mi) - kBiasF, f[qt], -kU8Offset);
     }
     move_max<0>(st, mlane, tile);
-    move_max<1>(st, mlane, tile);
-    float c[kQT];
+    if constexpr (QT > 1) move_max<1>(st, mlane, tile);
+    float c[QT];
     bool exact = false;
 #pragma unroll
-    for (int qt = 0; qt < kQT; ++qt) {
+    for (int qt = 0; qt < QT; ++qt) {
         c[qt] = -__builtin_fmaf(kBiasF, f[qt], st.m_used[qt]);
         exact = exact || !(fabsf(c[qt]) < 4096.0f);
     }
     auto make_p = [&](auto exact_tag) {
 #pragma unroll
-        for (int qt = 0; qt < kQT; ++qt) {
+        for (int qt = 0; qt < QT; ++qt) {
             const float nm = -st.m_used[qt];
             float lsum = 0.0f;
 #pragma unroll
@@ -272,13 +275,14 @@ __device__ __forceinline__ void softmax_tile8(const i32x4 (&s)[4][kQT], const fl
     else make_p(std::false_type{});
 }
 
-__device__ __forceinline__ void pv_tile8(const int8_t *stage, const LaneGeom8 &gm, const i32x4 (&p8)[kQT],
-                                         W8State &st) {
+template <int QT>
+__device__ __forceinline__ void pv_tile8(const int8_t *stage, const LaneGeom8 &gm, const i32x4 (&p8)[QT],
+                                         W8State<QT> &st) {
 #pragma unroll
     for (int ds = 0; ds < 8; ++ds) {
         const i32x4 vf = *reinterpret_cast<const i32x4 *>(stage + gm.v_rd + ds * 16 * 64);
 #pragma unroll
-        for (int qt = 0; qt < kQT; ++qt) {
+        for (int qt = 0; qt < QT; ++qt) {
             st.acc_i[ds][qt] = __builtin_amdgcn_mfma_i32_16x16x64_i8(vf, p8[qt], st.acc_i[ds][qt], 0, 0, 0);
             st.acc_i[ds][qt] = __builtin_amdgcn_mfma_i32_16x16x64_i8(vf, neg127_operand(), st.acc_i[ds][qt], 0, 0, 0);
         }
@@ -286,9 +290,10 @@ __device__ __forceinline__ void pv_tile8(const int8_t *stage, const LaneGeom8 &g
 }
 
 // Steady-state MFMA cluster: QK^T of the tile in kst, PV of the tile in vst.
+template <int QT>
 __device__ __forceinline__ void mfma_cluster8(const int8_t *kst, const int8_t *vst, const LaneGeom8 &gm,
-                                              const i32x4 (&qf)[kQT][2], i32x4 (&s)[4][kQT], const i32x4 (&p8)[kQT],
-                                              W8State &st) {
+                                              const i32x4 (&qf)[QT][2], i32x4 (&s)[4][QT], const i32x4 (&p8)[QT],
+                                              W8State<QT> &st) {
     // PV first: the V^T fragments and P die before the K fragments and the
     // S accumulators come alive, which keeps the two accumulator sets (int32
     // PV, fp32 O) resident without spills.
@@ -298,7 +303,7 @@ __device__ __forceinline__ void mfma_cluster8(const int8_t *kst, const int8_t *v
 #pragma unroll
     for (int ds = 0; ds < 8; ++ds)
 #pragma unroll
-        for (int qt = 0; qt < kQT; ++qt) {
+        for (int qt = 0; qt < QT; ++qt) {
             st.acc_i[ds][qt] = __builtin_amdgcn_mfma_i32_16x16x64_i8(vf[ds], p8[qt], st.acc_i[ds][qt], 0, 0, 0);
             st.acc_i[ds][qt] =
                 __builtin_amdgcn_mfma_i32_16x16x64_i8(vf[ds], neg127_operand(), st.acc_i[ds][qt], 0, 0, 0);
@@ -308,40 +313,54 @@ __device__ __forceinline__ void mfma_cluster8(const int8_t *kst, const int8_t *v
     for (int i = 0; i < 2; ++i)
 #pragma unroll
         for (int kt = 0; kt < 4; ++kt) kf[kt][i] = *reinterpret_cast<const i32x4 *>(kst + gm.k_rd[i] + kt * 16 * 128);
-    i32x4 z[4][kQT];
+    i32x4 z[4][QT];
 #pragma unroll
     for (int kt = 0; kt < 4; ++kt)
 #pragma unroll
-        for (int qt = 0; qt < kQT; ++qt)
+        for (int qt = 0; qt < QT; ++qt)
             z[kt][qt] = __builtin_amdgcn_mfma_i32_16x16x64_i8(kf[kt][0], qf[qt][0], i32x4{kBias, kBias, kBias, kBias},
                                                               0, 0, 0);
 #pragma unroll
     for (int kt = 0; kt < 4; ++kt)
 #pragma unroll
-        for (int qt = 0; qt < kQT; ++qt)
+        for (int qt = 0; qt < QT; ++qt)
             s[kt][qt] = __builtin_amdgcn_mfma_i32_16x16x64_i8(kf[kt][1], qf[qt][1], z[kt][qt], 0, 0, 0);
     // V^T reads (first half), K reads of the first QK^T half, V^T second
     // half, PV MFMAs, K second half, QK^T MFMAs.
     __builtin_amdgcn_sched_group_barrier(0x100, 4, 0);
     __builtin_amdgcn_sched_group_barrier(0x100, 4, 0);
-    __builtin_amdgcn_sched_group_barrier(0x008, 8, 0);
+    __builtin_amdgcn_sched_group_barrier(0x008, 4 * QT, 0);
     __builtin_amdgcn_sched_group_barrier(0x100, 4, 0);
-    __builtin_amdgcn_sched_group_barrier(0x008, 8, 0);
+    __builtin_amdgcn_sched_group_barrier(0x008, 4 * QT, 0);
     __builtin_amdgcn_sched_group_barrier(0x100, 4, 0);
-    __builtin_amdgcn_sched_group_barrier(0x008, 16, 0);
+    __builtin_amdgcn_sched_group_barrier(0x008, 8 * QT, 0);
 }
 
 // Schedule of the Sage kernel (see sage_attn.hip): per key tile t an MFMA
 // cluster {QK(t+1), PV(t)} and a VALU cluster {softmax(t+1)}, one barrier
 // per tile, the two groups' barriers on either side of the softmax.
-template <bool kCausal, bool kFp16Out>
-__global__ __launch_bounds__(kThreads, 1) void w8a8_attn_kernel(
-    const int8_t *__restrict__ q8, const float *__restrict__ q_scale, const int8_t *__restrict__ k8,
-    const float *__restrict__ k_scale, const int8_t *__restrict__ vt, const float *__restrict__ v_scale,
-    uint16_t *__restrict__ o, int hq, int groups, int64_t lq, int64_t lk,
-    int64_t lpad, int64_t nqs, int64_t nks, int64_t q_sb, int64_t q_sh, int64_t q_sl, int64_t k_sb, int64_t k_sh,
-    int64_t k_sl, int64_t o_sb, int64_t o_sh, int64_t o_sl, float sm_log2) {
-    __shared__ __align__(1024) int8_t lds[kStages][kStageBytes];
+struct W8Dims {
+    uint32_t hq, groups;
+    int64_t lq, lk, lpad, nqs, nks;
+    int64_t q_sb, q_sh, q_sl, k_sb, k_sh, k_sl, o_sb, o_sh, o_sl;
+    float sm_log2;
+};
+
+// The tensors, as kernel parameters: __restrict__ there is what makes the key
+// scales' loads scalar (as members of a struct they became vector loads, 3 %
+// of the kernel's time).
+#define TU_W8_TENSORS                                                                                           \
+    const int8_t *__restrict__ q8, const float *__restrict__ q_scale, const int8_t *__restrict__ k8,              \
+        const float *__restrict__ k_scale, const int8_t *__restrict__ vt, const float *__restrict__ v_scale,      \
+        uint16_t *__restrict__ o
+
+// One workgroup: 128 QT query rows from qblock0 on of (batch, head) bh.
+template <bool kCausal, bool kFp16Out, int QT>
+__device__ __forceinline__ void w8a8_block(TU_W8_TENSORS, const W8Dims &a, int8_t (*lds)[kStageBytes], uint32_t bh,
+                                           int64_t qblock0) {
+    constexpr int kRows = 128 * QT;  // query rows of the workgroup
+    constexpr int kWaveQ = 16 * QT;
+    const int64_t lq = a.lq, lk = a.lk;
 
     const int tid = threadIdx.x;
     const int lane = tid & 63;
@@ -351,19 +370,17 @@ __global__ __launch_bounds__(kThreads, 1) void w8a8_attn_kernel(
     const int g = lane >> 4;
     const int lc = lane & 15;
 
-    const int64_t bh = blockIdx.y;
-    const int64_t b = bh / hq, h = bh % hq, hk = h / groups;
-    const int64_t hkv = hq / groups;
-    const int64_t qblock0 = static_cast<int64_t>(blockIdx.x) * kBQ;
-    const int64_t q0 = qblock0 + grp * (kBQ / 2) + w4 * kWaveQ;
+    const uint32_t b = bh / a.hq, h = bh % a.hq, hk = h / a.groups;
+    const int64_t bhk = b * (a.hq / a.groups) + hk;
+    const int64_t q0 = qblock0 + grp * (kRows / 2) + w4 * kWaveQ;
 
-    const int8_t *qp = q8 + b * q_sb + h * q_sh;
-    const int8_t *kp = k8 + b * k_sb + hk * k_sh;
-    const int8_t *vtp = vt + (b * hkv + hk) * kD * lpad;
-    const float *ks_row = k_scale + (b * hkv + hk) * nks;
+    const int8_t *qp = q8 + b * a.q_sb + h * a.q_sh;
+    const int8_t *kp = k8 + b * a.k_sb + hk * a.k_sh;
+    const int8_t *vtp = vt + bhk * kD * a.lpad;
+    const float *ks_row = k_scale + bhk * a.nks;
 
     int64_t key_end = lk;
-    if constexpr (kCausal) key_end = min(lk, qblock0 + kBQ);
+    if constexpr (kCausal) key_end = min(lk, qblock0 + kRows);
     const int tiles = static_cast<int>((key_end + kBKey - 1) / kBKey);
     int my_tiles = tiles;
     if constexpr (kCausal)
@@ -372,30 +389,30 @@ __global__ __launch_bounds__(kThreads, 1) void w8a8_attn_kernel(
     if constexpr (kCausal) mask_from = min(mask_from, q0 / kBKey);
     const int first_masked = static_cast<int>(min<int64_t>(tiles, mask_from));
 
-    const LaneGeom8 gm = lane_geom8(w4, lane, k_sl, lpad);
-    const __amdgpu_buffer_rsrc_t krs = make_rsrc(kp, static_cast<uint32_t>(lk * k_sl));
-    const __amdgpu_buffer_rsrc_t vrs = make_rsrc(vtp, static_cast<uint32_t>(kD * lpad));
-    const uint32_t k_sl32 = static_cast<uint32_t>(k_sl);
+    const LaneGeom8 gm = lane_geom8(w4, lane, a.k_sl, a.lpad);
+    const __amdgpu_buffer_rsrc_t krs = make_rsrc(kp, static_cast<uint32_t>(lk * a.k_sl));
+    const __amdgpu_buffer_rsrc_t vrs = make_rsrc(vtp, static_cast<uint32_t>(kD * a.lpad));
+    const uint32_t k_sl32 = static_cast<uint32_t>(a.k_sl);
     auto tile_key0 = [&](int it) { return static_cast<uint32_t>(min(it, tiles - 1) * kBKey); };
 
-    i32x4 qf[kQT][2];
-    float qsc[kQT];
+    i32x4 qf[QT][2];
+    float qsc[QT];
 #pragma unroll
-    for (int qt = 0; qt < kQT; ++qt) {
+    for (int qt = 0; qt < QT; ++qt) {
         const int64_t qi = min(q0 + 16 * qt + lc, lq - 1);
 #pragma unroll
         for (int ds = 0; ds < 2; ++ds)
-            qf[qt][ds] = *reinterpret_cast<const i32x4 *>(qp + qi * q_sl + 64 * ds + 16 * g);
-        qsc[qt] = sm_log2 * q_scale[(b * hq + h) * nqs + qi / 16];
+            qf[qt][ds] = *reinterpret_cast<const i32x4 *>(qp + qi * a.q_sl + 64 * ds + 16 * g);
+        qsc[qt] = a.sm_log2 * q_scale[bh * a.nqs + qi / 16];
     }
     if (grp == 0) {
 #pragma unroll
         for (int j = 0; j < kAhead; ++j) issue_tile8(lds[j], krs, vrs, gm, k_sl32, tile_key0(j), w4);
     }
-    W8State st;
-    st.seg[0] = st.seg[1] = 0;
+    W8State<QT> st;
 #pragma unroll
-    for (int qt = 0; qt < kQT; ++qt) {
+    for (int qt = 0; qt < QT; ++qt) {
+        st.seg[qt] = 0;
         st.m_used[qt] = -INFINITY;
         st.beta[qt] = 1.0f;
         st.l[qt] = 0.0f;
@@ -406,20 +423,20 @@ __global__ __launch_bounds__(kThreads, 1) void w8a8_attn_kernel(
         }
     }
 
-    i32x4 s[4][kQT];
-    i32x4 p8[kQT];
+    i32x4 s[4][QT];
+    i32x4 p8[QT];
 
     auto softmax = [&](int it, auto mask_tag) {
         const float kscale = ks_row[it];
-        float f[kQT];
+        float f[QT];
 #pragma unroll
-        for (int qt = 0; qt < kQT; ++qt) f[qt] = qsc[qt] * kscale;
+        for (int qt = 0; qt < QT; ++qt) f[qt] = qsc[qt] * kscale;
         if (decltype(mask_tag)::value && it >= first_masked) {
             const int64_t key0 = static_cast<int64_t>(it) * kBKey;
             const int key_lim = static_cast<int>(min(lk - key0, static_cast<int64_t>(kBKey)));
             const int q_rel =
-                static_cast<int>(max(min(q0 - key0, static_cast<int64_t>(kBKey)), static_cast<int64_t>(-kBQ)));
-            mask_tile8<kCausal>(s, key_lim, q_rel, g, lc);
+                static_cast<int>(max(min(q0 - key0, static_cast<int64_t>(kBKey)), static_cast<int64_t>(-kRows)));
+            mask_tile8<kCausal, QT>(s, key_lim, q_rel, g, lc);
         }
         softmax_tile8(s, f, st, p8, it);
     };
@@ -467,10 +484,10 @@ __global__ __launch_bounds__(kThreads, 1) void w8a8_attn_kernel(
     // Final segment, then out = O / l * v_scale.  acc_o[ds][qt][r] holds
     // O^T[16 ds + 4 g + r][q0 + 16 qt + lc].
     flush_segment(st, my_tiles);
-    const float *vs = v_scale + (b * hkv + hk) * kD + 4 * g;
-    uint16_t *op = o + b * o_sb + h * o_sh;
+    const float *vs = v_scale + bhk * kD + 4 * g;
+    uint16_t *op = o + b * a.o_sb + h * a.o_sh;
 #pragma unroll
-    for (int qt = 0; qt < kQT; ++qt) {
+    for (int qt = 0; qt < QT; ++qt) {
         const int64_t qi = q0 + 16 * qt + lc;
         const float inv = 1.0f / xsum_f32(st.l[qt]);
         if (qi >= lq) continue;
@@ -490,9 +507,111 @@ __global__ __launch_bounds__(kThreads, 1) void w8a8_attn_kernel(
                 packed.x = pack_bf16x2(y[0], y[1]);
                 packed.y = pack_bf16x2(y[2], y[3]);
             }
-            *reinterpret_cast<u32x2 *>(op + qi * o_sl + 16 * ds + 4 * g) = packed;
+            *reinterpret_cast<u32x2 *>(op + qi * a.o_sl + 16 * ds + 4 * g) = packed;
         }
     }
+}
+
+#define TU_W8_POINTERS q8, q_scale, k8, k_scale, vt, v_scale, o
+
+// Work plan of a launch.  Query blocks of 256 rows are numbered head-major.
+// Blocks below split_from run whole, one workgroup of 32 rows a wave; every
+// later one as two workgroups of 128 rows, 16 a wave (an end block of at most
+// 128 rows leaves its second one empty).  Neither changes a row's arithmetic.
+// Causal workgroups are numbered by query block from the last, longest one
+// to the first, heads fastest.
+struct W8Plan {
+    uint32_t nqb;         // query blocks of a head
+    uint32_t bh;          // batch * hq
+    uint32_t split_from;  // first block that runs as two workgroups (causal: all or none)
+};
+
+// kMode: 0 every block whole, 1 every block in two, 2 both.
+template <bool kCausal, bool kFp16Out, int kMode>
+__global__ __launch_bounds__(kThreads, 1) void w8a8_attn_kernel(TU_W8_TENSORS, W8Dims a,
+                                                                W8Plan plan) {
+    __shared__ __align__(1024) int8_t lds[kStages][kStageBytes];
+    uint32_t id = blockIdx.x, half = 0;
+    bool whole = kMode == 0;
+    uint32_t bh, qb;
+    if constexpr (kCausal) {
+        bh = id % plan.bh;
+        id /= plan.bh;
+        if constexpr (kMode == 1) {
+            half = 1 - (id & 1);  // the later rows are the longer ones
+            id >>= 1;
+        }
+        qb = plan.nqb - 1 - id;
+    } else {
+        const uint32_t blocks = plan.nqb * plan.bh;
+        if constexpr (kMode == 2) whole = id < plan.split_from;
+        if (whole) {
+            id = xcd_chunk(id, kMode == 0 ? blocks : plan.split_from);
+        } else {
+            const uint32_t from = kMode == 1 ? 0 : plan.split_from;
+            id = xcd_chunk(id - from, 2 * (blocks - from));
+            half = id & 1;
+            id = from + (id >> 1);
+        }
+        bh = id / plan.nqb;
+        qb = id % plan.nqb;
+    }
+    const int64_t q0 = static_cast<int64_t>(qb) * kBQ + 128 * half;
+    if (q0 >= a.lq) return;  // the whole workgroup
+    if constexpr (kMode == 2) {
+        if (whole) w8a8_block<kCausal, kFp16Out, 2>(TU_W8_POINTERS, a, lds, bh, q0);
+        else w8a8_block<kCausal, kFp16Out, 1>(TU_W8_POINTERS, a, lds, bh, q0);
+    } else {
+        w8a8_block<kCausal, kFp16Out, kMode == 0 ? 2 : 1>(TU_W8_POINTERS, a, lds, bh, q0);
+    }
+}
+
+// Workgroups of 128 rows read K and V^T once for half the rows: they take
+// 0.55-0.6 of a whole block's time (28.7 and 51.4 us for 8 and 25 key tiles
+// of 84 blocks against 26.1 and 61.5 for whole ones).  They pay where whole
+// blocks leave compute units idle:
+//   non-causal, the blocks past the last full round when they are at most
+//     half a round: B1 H12 L1560 (84 blocks) 61.5 -> 37 us, H56 L4096 (896)
+//     509 -> 461, B1 H12 L8190 (384) 461 -> 368; with more left over, two
+//     half rounds are slower than one whole one (H60 L4096, 192 left: 512 and
+//     531 us);
+//   causal, every block when the longest block outweighs the even share of
+//     all of them by more than the halves' extra work: H4 L4001 117 -> 72 us,
+//     H40 L1000 41 -> 26; B2 H16 L4001 stays whole (149 against 166).
+W8Plan w8_plan(int64_t batch, int64_t hq, int64_t lq, int64_t lk, bool causal, int64_t cus) {
+    W8Plan p{static_cast<uint32_t>((lq + kBQ - 1) / kBQ), static_cast<uint32_t>(batch * hq), 0xffffffffu};
+    const int64_t blocks = static_cast<int64_t>(p.nqb) * p.bh;
+    if (!causal) {
+        const int64_t full = blocks / cus * cus;
+        if (full < 0x7fffffff && 2 * (blocks - full) <= cus) p.split_from = static_cast<uint32_t>(full);
+        return p;
+    }
+    if (blocks >= 8 * cus) return p;  // an even share longer than any block
+    int64_t work = 0, longest = 0;
+    for (uint32_t qb = 0; qb < p.nqb; ++qb) {
+        const int64_t t = (std::min<int64_t>(lk, (qb + int64_t{1}) * kBQ) + kBKey - 1) / kBKey;
+        work += t;
+        longest = std::max(longest, t);
+    }
+    if (8 * work * p.bh < 7 * longest * cus) p.split_from = 0;
+    return p;
+}
+
+template <bool kCausal, bool kFp16Out>
+int32_t launch_w8(const W8Plan &plan, TU_W8_TENSORS, const W8Dims &a, hipStream_t s) {
+    const int64_t blocks = static_cast<int64_t>(plan.nqb) * plan.bh;
+    const int64_t whole = std::min<int64_t>(plan.split_from, blocks);
+    const int64_t grid = whole + 2 * (blocks - whole);
+    TU_REQUIRE(grid <= 0x7fffffff, "W8A8 attention grid too large");
+    const dim3 g(static_cast<unsigned>(grid));
+    if (whole == blocks) {
+        w8a8_attn_kernel<kCausal, kFp16Out, 0><<<g, kThreads, 0, s>>>(TU_W8_POINTERS, a, plan);
+    } else if (whole == 0) {
+        w8a8_attn_kernel<kCausal, kFp16Out, 1><<<g, kThreads, 0, s>>>(TU_W8_POINTERS, a, plan);
+    } else if constexpr (!kCausal) {
+        w8a8_attn_kernel<kCausal, kFp16Out, 2><<<g, kThreads, 0, s>>>(TU_W8_POINTERS, a, plan);
+    }
+    return check_launch("tu_w8a8_attn_fwd");
 }
 
 }  // namespace
@@ -525,20 +644,16 @@ extern "C" int32_t tu_w8a8_attn_fwd(const int8_t *q8, const float *q_scale, int6
                    o_sb % 4 == 0 && (reinterpret_cast<uintptr_t>(out) & 7) == 0,
                "W8A8 attention V^T/scales/O must be aligned");
     if (require_gfx950()) return -1;
-    const dim3 grid(static_cast<unsigned>((lq + kBQ - 1) / kBQ), static_cast<unsigned>(batch * hq));
-    const float sm_log2 = sm_scale * kLog2e;
+    int cus = 0;
+    if (device_cus(cus)) return -1;
+    const W8Plan plan = w8_plan(batch, hq, lq, lk, causal != 0, cus);
+    const W8Dims a{static_cast<uint32_t>(hq), static_cast<uint32_t>(hq / hkv), lq, lk, lpad, nqs, nks, q_sb, q_sh, q_sl,
+                   k_sb, k_sh, k_sl, o_sb, o_sh, o_sl, sm_scale * kLog2e};
+    auto *o = static_cast<uint16_t *>(out);
     hipStream_t s = static_cast<hipStream_t>(stream);
-    const int groups = static_cast<int>(hq / hkv);
-#define TU_W8_ARGS                                                                                            \
-    q8, q_scale, k8, k_scale, vt, v_scale, static_cast<uint16_t *>(out), static_cast<int>(hq), groups,           \
-        lq, lk, lpad, nqs, nks, q_sb, q_sh, q_sl, k_sb, k_sh, k_sl, o_sb, o_sh, o_sl, sm_log2
-    if (causal) {
-        if (out_fp16) w8a8_attn_kernel<true, true><<<grid, kThreads, 0, s>>>(TU_W8_ARGS);
-        else w8a8_attn_kernel<true, false><<<grid, kThreads, 0, s>>>(TU_W8_ARGS);
-    } else {
-        if (out_fp16) w8a8_attn_kernel<false, true><<<grid, kThreads, 0, s>>>(TU_W8_ARGS);
-        else w8a8_attn_kernel<false, false><<<grid, kThreads, 0, s>>>(TU_W8_ARGS);
-    }
-#undef TU_W8_ARGS
-    return check_launch("tu_w8a8_attn_fwd");
+    if (causal)
+        return out_fp16 ? launch_w8<true, true>(plan, TU_W8_POINTERS, a, s)
+                        : launch_w8<true, false>(plan, TU_W8_POINTERS, a, s);
+    return out_fp16 ? launch_w8<false, true>(plan, TU_W8_POINTERS, a, s)
+                    : launch_w8<false, false>(plan, TU_W8_POINTERS, a, s);
 }

@@ -34,10 +34,15 @@ K_AHEAD = K_STAGES - 1
 # per kernel: 1 KiB blocks a group-0 wave loads per tile (Sage head_dim 128:
 # 2 K + 4 V^T, Sage head_dim 64: 1 K + 2 V^T, W8A8 2 K + 2 V^T), and whether
 # it issues them after the softmax
-KERNELS = {"sage": (6, False), "sage64": (3, False), "w8a8": (4, False), "w8a8_after": (4, True)}
+KERNELS = {"sage": (6, False), "sage64": (3, False), "w8a8": (4, False), "w8a8_after": (4, True),
+           "w8a8_half": (4, False)}
 KBKEY = 64
 KBQ = 256
-KWAVEQ = 32
+
+
+def block_rows(kernel: str) -> int:
+    """Query rows of a workgroup: 8 waves of 32, or of 16 (the W8A8 kernel's half blocks)."""
+    return KBQ // 2 if kernel == "w8a8_half" else KBQ
 
 
 class Wave:
@@ -85,9 +90,10 @@ def kernel_program(wave: int, lq: int, lk: int, causal: bool, qblock: int, kerne
     LOADS_PER_TILE, issue_late = KERNELS[kernel]
     w = Wave(wave)
     grp, w4 = wave >> 2, wave & 3
-    qblock0 = qblock * KBQ
-    q0 = qblock0 + grp * (KBQ // 2) + w4 * KWAVEQ
-    key_end = min(lk, qblock0 + KBQ) if causal else lk
+    rows = block_rows(kernel)
+    qblock0 = qblock * rows
+    q0 = qblock0 + grp * (rows // 2) + w4 * (rows // 8)
+    key_end = min(lk, qblock0 + rows) if causal else lk
     tile_base = split_z * split_tiles if split_z is not None else 0
     tiles = (key_end + KBKEY - 1) // KBKEY
     if split_z is not None:
@@ -95,7 +101,7 @@ def kernel_program(wave: int, lq: int, lk: int, causal: bool, qblock: int, kerne
         tiles = min(split_tiles, tiles - tile_base)
     my_tiles = tiles
     if causal:
-        my_tiles = min(tiles, max(1, (min(q0 + KWAVEQ, lq) + KBKEY - 1) // KBKEY))
+        my_tiles = min(tiles, max(1, (min(q0 + rows // 8, lq) + KBKEY - 1) // KBKEY))
     mask_from = lk // KBKEY - tile_base
     if causal:
         mask_from = min(mask_from, q0 // KBKEY)
@@ -249,7 +255,7 @@ def check_schedule(lq: int, lk: int, causal: bool, qblock: int, kernel: str = "s
 @pytest.mark.parametrize("lk", [1, 2, 63, 64, 65, 127, 128, 129, 191, 256, 257, 300, 333, 511, 700, 1000, 32760])
 def test_schedule_every_block(causal, lk, kernel):
     lq = lk if causal else max(lk, 300)
-    nblk = (lq + KBQ - 1) // KBQ
+    nblk = (lq + block_rows(kernel) - 1) // block_rows(kernel)
     # non-causal: the schedule does not depend on the query block
     blocks = range(nblk) if causal else sorted({0, nblk - 1})
     for qblock in blocks:
@@ -260,7 +266,7 @@ def test_schedule_every_block(causal, lk, kernel):
 @pytest.mark.parametrize("lq,lk", list(itertools.product([1, 40, 129, 256, 257, 700], [1, 2, 64, 65, 151, 333])))
 def test_schedule_ragged_pairs(lq, lk, kernel):
     for causal in (False, True):
-        for qblock in range((lq + KBQ - 1) // KBQ):
+        for qblock in range((lq + block_rows(kernel) - 1) // block_rows(kernel)):
             check_schedule(lq, lk, causal, qblock, kernel)
 
 
