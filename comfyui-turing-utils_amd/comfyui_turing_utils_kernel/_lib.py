@@ -129,6 +129,13 @@ SIGNATURES: dict[str, tuple[object, list[object]]] = {
         [_c_void_p, _i32, _i64, _i64, _i64, _i64, _i64, _i64, _i64, _c_void_p, _i64,
          _c_void_p, _c_void_p, _i64, _c_void_p],
     ),
+    "tu_w8a8_prep": (
+        _i32,
+        [_c_void_p, _c_void_p, _c_void_p, _i32, _i64, _i64, _i64, _i64, _i64, _i64,
+         _i64, _i64, _i64, _i64, _i64, _i64, _i64, _i64, _i64,
+         _c_void_p, _i64, _i64, _i64, _c_void_p, _i64, _i64, _i64, _c_void_p, _c_void_p, _c_void_p, _i32,
+         _c_void_p, _i64, _c_void_p, _i32, _c_void_p, _i64, _c_void_p],
+    ),
     "tu_w8a8_attn_fwd": (
         _i32,
         [_c_void_p, _c_void_p, _i64, _c_void_p, _c_void_p, _i64, _c_void_p, _c_void_p,
@@ -155,7 +162,7 @@ SIGNATURES: dict[str, tuple[object, list[object]]] = {
     ),
 }
 
-ABI_VERSION = 15
+ABI_VERSION = 16
 
 _lock = threading.Lock()
 _lib: ctypes.CDLL | None = None

@@ -30,10 +30,10 @@ from .. import _lib
 from .quant import (
     SUPPORTED_BLOCKS,
     _layout_dims,
-    per_warp_int8_hadamard,
     quantize_v_int8,
     sage_prologue,
     value_transpose,
+    w8a8_prologue,
 )
 
 KERNEL_HEAD_DIM = 128  # widest head; the W8A8 kernel's only width
@@ -586,17 +586,19 @@ def prequantize_w8a8attn(
         raise ValueError("Sol sparse attention requires head_dim in [1, 128]")
     if q.stride(-1) != 1 or k.stride(-1) != 1 or v.stride(-1) != 1:
         raise ValueError("the last Q/K/V dimension must be contiguous")
+    tile = _key_tile_tokens(key_tile_tokens, k.size(2))
     kernel_head_dim = 64 if head_dim <= 64 else 128
     with torch.cuda.device(q.device):
         q, k, v = (_pad_channels(t, kernel_head_dim) for t in (q, k, v))
-        q_int8, q_scale, k_int8, k_scale = per_warp_int8_hadamard(
-            q, k, tensor_layout="HND", stabilize_k=bool(stabilize_k) and bool(rotate_qk), rotate=bool(rotate_qk))
-    qk = PrequantizedQK(
-        query_int8=q_int8, query_scale=q_scale, key_int8=k_int8, key_scale=k_scale, tensor_layout="HND",
-        input_dtype=v.dtype, original_head_dim=head_dim, route_original_basis=bool(rotate_qk),
+        q_int8, q_scale, k_int8, k_scale, value_int8, value_scale = w8a8_prologue(
+            q, k, v, stabilize_k=bool(stabilize_k) and bool(rotate_qk), rotate=bool(rotate_qk))
+    return PrequantizedW8A8Attention(
+        query_int8=q_int8, query_scale=q_scale, key_int8=k_int8, key_scale=k_scale,
+        value_int8=value_int8, value_scale=value_scale, output_dtype=v.dtype,
+        sm_scale=float(sm_scale) if sm_scale is not None else head_dim ** -0.5,
+        original_head_dim=head_dim, key_tile_tokens=tile,
+        is_causal=bool(is_causal), route_original_basis=bool(rotate_qk),
     )
-    return prequantize_w8a8attn_from_qk(qk, v, sm_scale=sm_scale, key_tile_tokens=key_tile_tokens,
-                                        is_causal=is_causal)
 
 
 def w8a8attn_from_prequantized(quantized: PrequantizedW8A8Attention) -> torch.Tensor:

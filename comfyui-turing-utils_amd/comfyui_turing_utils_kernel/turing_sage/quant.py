@@ -290,3 +290,37 @@ def quantize_v_int8(value: torch.Tensor) -> tuple[torch.Tensor, torch.Tensor]:
                   length, dim, value.stride(0), value.stride(1), value.stride(2), codes.data_ptr(), lpad,
                   scale.data_ptr(), workspace.data_ptr(), ws_bytes, _lib.stream_of(value.device))
     return codes, scale
+
+
+def w8a8_prologue(
+    q: torch.Tensor,
+    k: torch.Tensor,
+    v: torch.Tensor,
+    *,
+    stabilize_k: bool,
+    rotate: bool,
+) -> tuple[torch.Tensor, ...]:
+    """``per_warp_int8_hadamard`` of HND Q/K and ``quantize_v_int8`` of HND V in
+    two launches, for the 128 channels of the attention kernel: (q_int8,
+    q_scale, k_int8, k_scale, value_int8, value_scale), head_dim 64 padded with
+    zero codes (V scales 1e-12).  The caller has checked shapes and types."""
+    if v.data_ptr() % 16 or any(s % 8 for s in v.stride()[:-1]):
+        v = v.contiguous()
+    (batch, hq, lq, dim), (hk, lk), device = q.shape, k.shape[1:3], q.device
+    lpad = (lk + 63) // 64 * 64
+    q_int8 = torch.empty((batch, hq, lq, 128), dtype=torch.int8, device=device)
+    k_int8 = torch.empty((batch, hk, lk, 128), dtype=torch.int8, device=device)
+    v_int8 = torch.empty((batch, hk, 128, lpad), dtype=torch.int8, device=device)
+    q_scale = torch.empty((batch, hq, (lq + 63) // 64 * 4), dtype=torch.float32, device=device)
+    k_scale = torch.empty((batch, hk, (lk + 63) // 64), dtype=torch.float32, device=device)
+    v_scale = torch.empty((batch, hk, 128), dtype=torch.float32, device=device)
+    anchors = torch.empty((batch, hk), dtype=torch.int32, device=device) if stabilize_k else None
+    nbytes = max(0, int(_lib.load().tu_w8a8_quant_v_workspace(batch, hk, lk, dim)))
+    workspace = torch.empty((nbytes,), dtype=torch.uint8, device=device)
+    with torch.cuda.device(device):
+        _lib.call("tu_w8a8_prep", q.data_ptr(), k.data_ptr(), v.data_ptr(), int(q.dtype == torch.float16), batch, hq,
+                  hk, lq, lk, dim, *q.stride()[:3], *k.stride()[:3], *v.stride()[:3], q_int8.data_ptr(),
+                  *q_int8.stride()[:3], k_int8.data_ptr(), *k_int8.stride()[:3], q_scale.data_ptr(),
+                  k_scale.data_ptr(), _lib.ptr(anchors), int(rotate), v_int8.data_ptr(), lpad, v_scale.data_ptr(),
+                  int(dim == 64), workspace.data_ptr(), nbytes, _lib.stream_of(device))
+    return q_int8, q_scale, k_int8, k_scale, v_int8, v_scale

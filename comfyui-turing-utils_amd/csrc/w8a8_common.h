@@ -28,39 +28,51 @@ __device__ __forceinline__ float wave_max_nonneg(float v) {
     return __int_as_float(xmax_i32(b));
 }
 
-// v of lane i ^ kBit (kBit < 16) with no index arithmetic: DPP quad
-// permutations for 1 and 2; for 4 the mirror of each 8-lane half (lane
-// 7 - i) and then the reversal of each quad, which together give i ^ 4; for
-// 8 the rotation of each 16-lane row by 8 ((i + 8) mod 16 = i ^ 8).
-template <int kBit>
-__device__ __forceinline__ float w8a8_lane_xor(float v) {
-    int x = __float_as_int(v);
-    if constexpr (kBit == 1) {
-        x = __builtin_amdgcn_update_dpp(0, x, 0xB1, 0xf, 0xf, true);
-    } else if constexpr (kBit == 2) {
-        x = __builtin_amdgcn_update_dpp(0, x, 0x4E, 0xf, 0xf, true);
-    } else if constexpr (kBit == 4) {
-        x = __builtin_amdgcn_update_dpp(0, x, 0x141, 0xf, 0xf, true);   // row_half_mirror
-        x = __builtin_amdgcn_update_dpp(0, x, 0x1B, 0xf, 0xf, true);    // quad (3, 2, 1, 0)
-    } else {
-        static_assert(kBit == 8, "lane xor of 1, 2, 4 or 8");
-        x = __builtin_amdgcn_update_dpp(0, x, 0x128, 0xf, 0xf, true);   // row_ror:8
-    }
-    return __int_as_float(x);
-}
-
-// One cross-pack butterfly stage: v = other - v on lanes with bit `kBit` of
-// the pack index set, v + other elsewhere, as other + (+-1 * v): IEEE
-// subtraction is addition of the negation, and addition commutes, so the
-// bits are those of the two-sided form.
+// One cross-pack butterfly stage up to the sign of the lane's values: v +
+// sgn * other with other the value of lane i ^ kBit and sgn -1 on lanes with
+// bit `kBit` of the pack index set.  That is the stage's result (other - v
+// there, v + other elsewhere) times sgn; both lanes of every later stage's
+// pairs carry the signs of the earlier stages alike, so w8a8_hadamard_pack
+// applies their product once, with the normalisation.  A multiplication by
+// +-1 and a negation are exact: the magnitudes have the bits of the two-sided
+// form.
+//
+// The lane exchange is the DPP operand of v_fmac_f32, one instruction a value
+// (written out: the compiler keeps a v_mov_b32_dpp and a cleared destination
+// beside each v_fmac).  Quad permutations give i ^ 1 and i ^ 2, the rotation
+// of a 16-lane row by 8 gives i ^ 8; i ^ 4 is the mirror of each 8-lane half
+// (lane 7 - i), then the reversal of each quad.  A DPP operand has to be two
+// instructions older than its reader: the s_nop covers what was written
+// before the block, eight values in turn the rest.
+#define TU_DPP8(OP, CTRL)                                                                                     \
+    OP(0, CTRL) OP(1, CTRL) OP(2, CTRL) OP(3, CTRL) OP(4, CTRL) OP(5, CTRL) OP(6, CTRL) OP(7, CTRL)
+#define TU_FMAC_DPP(J, CTRL) "v_fmac_f32_dpp %" #J ", %" #J ", %8 " CTRL " row_mask:0xf bank_mask:0xf\n"
+#define TU_FMAC_DPP_T(J, CTRL) "v_fmac_f32_dpp %" #J ", %[t" #J "], %[s] " CTRL " row_mask:0xf bank_mask:0xf\n"
+#define TU_MOV_DPP_T(J, CTRL) "v_mov_b32_dpp %[t" #J "], %" #J " " CTRL " row_mask:0xf bank_mask:0xf\n"
+#define TU_V8 "+&v"(v[0]), "+&v"(v[1]), "+&v"(v[2]), "+&v"(v[3]), "+&v"(v[4]), "+&v"(v[5]), "+&v"(v[6]), "+&v"(v[7])
 template <int kBit>
 __device__ __forceinline__ void w8a8_cross_stage(float (&v)[8], int p) {
-    float sgn = (p & kBit) ? -1.0f : 1.0f;
-    // opaque to the compiler, which would otherwise form both sums and select
-    asm("" : "+v"(sgn));
-#pragma unroll
-    for (int j = 0; j < 8; ++j) v[j] = w8a8_lane_xor<kBit>(v[j]) + sgn * v[j];
+    const float sgn = (p & kBit) ? -1.0f : 1.0f;
+    if constexpr (kBit == 1) {
+        asm("s_nop 1\n" TU_DPP8(TU_FMAC_DPP, "quad_perm:[1,0,3,2]") : TU_V8 : "v"(sgn));
+    } else if constexpr (kBit == 2) {
+        asm("s_nop 1\n" TU_DPP8(TU_FMAC_DPP, "quad_perm:[2,3,0,1]") : TU_V8 : "v"(sgn));
+    } else if constexpr (kBit == 8) {
+        asm("s_nop 1\n" TU_DPP8(TU_FMAC_DPP, "row_ror:8") : TU_V8 : "v"(sgn));
+    } else {
+        static_assert(kBit == 4, "lane xor of 1, 2, 4 or 8");
+        float t[8];
+        asm("s_nop 1\n" TU_DPP8(TU_MOV_DPP_T, "row_half_mirror") TU_DPP8(TU_FMAC_DPP_T, "quad_perm:[3,2,1,0]")
+            : TU_V8, [t0] "=&v"(t[0]), [t1] "=&v"(t[1]), [t2] "=&v"(t[2]), [t3] "=&v"(t[3]), [t4] "=&v"(t[4]),
+              [t5] "=&v"(t[5]), [t6] "=&v"(t[6]), [t7] "=&v"(t[7])
+            : [s] "v"(sgn));
+    }
 }
+#undef TU_DPP8
+#undef TU_FMAC_DPP
+#undef TU_FMAC_DPP_T
+#undef TU_MOV_DPP_T
+#undef TU_V8
 
 // The transform of one pack (8 channels of pack index p) across the lanes of
 // a token (attention_hadamard8, fused.cu:214-260): signs, the in-pack
@@ -88,8 +100,9 @@ __device__ __forceinline__ void w8a8_hadamard_pack(float (&v)[8], int p) {
     w8a8_cross_stage<4>(v, p);
     if constexpr (D == 128) w8a8_cross_stage<8>(v, p);
     constexpr float kNorm = D == 64 ? 0.125f : 0.08838834764831845f;
+    const float norm = __builtin_popcount(p & (D / 8 - 1)) & 1 ? -kNorm : kNorm;
 #pragma unroll
-    for (int j = 0; j < 8; ++j) v[j] *= kNorm;
+    for (int j = 0; j < 8; ++j) v[j] *= norm;
 }
 
 // Lane 0 / lane 32 of a wave64 end with the sum (max) of their 32-lane half,

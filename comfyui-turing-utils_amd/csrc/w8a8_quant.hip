@@ -21,6 +21,9 @@
 // MI355X layout of V: channel-major codes [B][H][D][Lpad] with keys in
 // natural order (the INT8 PV MFMA reads 16 consecutive keys of one channel
 // per lane).
+#include <algorithm>
+#include <type_traits>
+
 #include "w8a8_common.h"
 
 namespace tu {
@@ -32,30 +35,20 @@ __device__ __forceinline__ float h_to_f32(uint32_t bits16) {
     else return __uint_as_float(bits16 << 16);
 }
 
-// cvt.rni.sat.s8.f32: round half to even, saturate to [-128, 127].
-__device__ __forceinline__ int32_t sat_rne_s8(float v) {
-    const float r = __builtin_rintf(v);
-    return static_cast<int32_t>(fminf(127.0f, fmaxf(-128.0f, r)));
-}
-
-// sat_rne_s8 of four values packed little-endian, without conversions: the
-// clamp comes first (the bounds are integers, so clamping and rounding
-// commute; NaN clamps to -128 as above), then adding 1.5 * 2^23 rounds half
-// to even to an integer whose two's complement sits in the low byte.
+// cvt.rni.sat.s8.f32 (round half to even, saturate to [-128, 127]) of four
+// values packed little-endian, without conversions: the clamp comes first
+// (the bounds are integers, so clamping and rounding commute; NaN clamps to
+// -128), then adding 1.5 * 2^23 rounds half to even to an integer whose two's
+// complement sits in the low byte.
 __device__ __forceinline__ uint32_t sat_rne_s8x4(float a, float b, float c, float d) {
     const float vs[4] = {a, b, c, d};
-    uint32_t w = 0u;
+    uint32_t w[4];
 #pragma unroll
-    for (int k = 0; k < 4; ++k) {
-        const float x = fminf(127.0f, fmaxf(-128.0f, vs[k]));
-        w |= (__float_as_uint(x + 12582912.0f) & 0xffu) << (8 * k);
-    }
-    return w;
-}
-
-__device__ __forceinline__ uint32_t pack_s8x4(int32_t a, int32_t b, int32_t c, int32_t d) {
-    return (static_cast<uint32_t>(a) & 0xffu) | ((static_cast<uint32_t>(b) & 0xffu) << 8) |
-           ((static_cast<uint32_t>(c) & 0xffu) << 16) | (static_cast<uint32_t>(d) << 24);
+    for (int k = 0; k < 4; ++k) w[k] = __float_as_uint(fminf(127.0f, fmaxf(-128.0f, vs[k])) + 12582912.0f);
+    // low bytes of two words, then of two pairs
+    const uint32_t lo = __builtin_amdgcn_perm(w[1], w[0], 0x0c0c0400u);
+    const uint32_t hi = __builtin_amdgcn_perm(w[3], w[2], 0x0c0c0400u);
+    return __builtin_amdgcn_perm(hi, lo, 0x05040100u);
 }
 
 // ---------------------------------------------------------------------------
@@ -63,12 +56,11 @@ __device__ __forceinline__ uint32_t pack_s8x4(int32_t a, int32_t b, int32_t c, i
 // per (kv head, batch).
 // ---------------------------------------------------------------------------
 template <bool kFp16>
-__global__ __launch_bounds__(kAnchorThreads) void anchor_kernel(const uint16_t *__restrict__ k, int64_t len, int dim,
-                                                                int64_t s_b, int64_t s_h, int64_t s_l,
-                                                                int32_t *__restrict__ anchors) {
+__device__ __forceinline__ void anchor_body(const uint16_t *__restrict__ k, int64_t len, int dim, int64_t s_b,
+                                            int64_t s_h, int64_t s_l, int32_t *__restrict__ anchors, int64_t h,
+                                            int64_t b, int64_t heads) {
     __shared__ float samples[kAnchorSamples][128];
     const int c = threadIdx.x;
-    const int64_t h = blockIdx.x, b = blockIdx.y, heads = gridDim.x;
     const uint16_t *kb = k + b * s_b + h * s_h;
 #pragma unroll
     for (int s = 0; s < kAnchorSamples; ++s) {
@@ -80,6 +72,13 @@ __global__ __launch_bounds__(kAnchorThreads) void anchor_kernel(const uint16_t *
     if (c == 0)
         anchors[b * heads + h] =
             sel >= 0 ? static_cast<int32_t>(static_cast<int64_t>(sel) * (len - 1) / (kAnchorSamples - 1)) : -1;
+}
+
+template <bool kFp16>
+__global__ __launch_bounds__(kAnchorThreads) void anchor_kernel(const uint16_t *__restrict__ k, int64_t len, int dim,
+                                                                int64_t s_b, int64_t s_h, int64_t s_l,
+                                                                int32_t *__restrict__ anchors) {
+    anchor_body<kFp16>(k, len, dim, s_b, s_h, s_l, anchors, blockIdx.x, blockIdx.y, gridDim.x);
 }
 
 // ---------------------------------------------------------------------------
@@ -102,10 +101,11 @@ struct RotArgs {
     int64_t x_sb[2], x_sh[2], x_sl[2];
     int64_t o_sb[2], o_sh[2], o_sl[2];
     int rotate;
+    int wide;  // head_dim 64 into 128-byte rows, channels 64 .. 127 zero
 };
 
 template <bool kFp16, int D>
-__global__ __launch_bounds__(kQkThreads) void rot_quant_kernel(RotArgs args) {
+__device__ __forceinline__ void rot_quant_body(const RotArgs &args, uint32_t task, int64_t b) {
     constexpr int kPacks = D / 8;
     constexpr int kTokPerPass = kQkThreads / kPacks;   // 16 (D 128) or 32 (D 64)
     constexpr int kIters = kChunk / kTokPerPass;        // 4 or 2
@@ -115,15 +115,14 @@ __global__ __launch_bounds__(kQkThreads) void rot_quant_kernel(RotArgs args) {
     const int tid = threadIdx.x;
     const int wave = tid >> 6;
     const int pack = tid % kPacks;
-    const int64_t b = blockIdx.y;
-    int64_t task = blockIdx.x;
-    const int64_t nch_q = (args.len[0] + kChunk - 1) / kChunk;
-    const int which = task < args.heads[0] * nch_q ? 0 : 1;
-    if (which) task -= args.heads[0] * nch_q;
+    // 32-bit block arithmetic: a 64-bit division is a long instruction sequence
+    const uint32_t nq_blocks = static_cast<uint32_t>(args.heads[0]) * static_cast<uint32_t>(args.ntiles[0] / 4);
+    const int which = task < nq_blocks ? 0 : 1;
+    if (which) task -= nq_blocks;
     const int64_t len = args.len[which];
-    const int64_t nch = (len + kChunk - 1) / kChunk;
+    const uint32_t nch = static_cast<uint32_t>((len + kChunk - 1) / kChunk);
     const int64_t head = task / nch;
-    const int64_t chunk = task - head * nch;
+    const int64_t chunk = task % nch;
     const int64_t t0 = chunk * kChunk;
     const uint16_t *xbase = args.x[which] + b * args.x_sb[which] + head * args.x_sh[which];
 
@@ -220,34 +219,63 @@ __global__ __launch_bounds__(kQkThreads) void rot_quant_kernel(RotArgs args) {
 #pragma unroll
         for (int j = 0; j < 8; ++j) y[j] = v[it][j] * mult[it];
         const u32x2 packed{sat_rne_s8x4(y[0], y[1], y[2], y[3]), sat_rne_s8x4(y[4], y[5], y[6], y[7])};
-        *reinterpret_cast<u32x2 *>(obase + t * args.o_sl[which] + pack * 8) = packed;
+        int8_t *dst = obase + t * args.o_sl[which] + pack * 8;
+        *reinterpret_cast<u32x2 *>(dst) = packed;
+        if (D == 64 && args.wide) *reinterpret_cast<u32x2 *>(dst + 64) = u32x2{0u, 0u};
     }
 }
 
+template <bool kFp16, int D>
+__global__ __launch_bounds__(kQkThreads) void rot_quant_kernel(RotArgs args) {
+    rot_quant_body<kFp16, D>(args, blockIdx.x, blockIdx.y);
+}
+
 // ---------------------------------------------------------------------------
-// V: per-channel amax over token chunks, scales, codes.
+// V: per-channel amax over token chunks, then codes.  Every code workgroup
+// reduces its head's chunk maxima itself (at most 64 rows of 512 bytes from
+// L2): a launch for the scales alone costs more than that.
 // ---------------------------------------------------------------------------
 constexpr int kVThreads = 256;
-constexpr int kVChunk = 1024;  // tokens per amax workgroup
+constexpr int kAmaxThreads = kAnchorThreads;
+constexpr int64_t kAmaxTokens = 128;  // fewest tokens of an amax chunk
+
+// Tokens of an amax chunk: 128, more where that would pass 64 chunks a head,
+// or 16 once the heads alone fill the GPU.
+int64_t v_chunk_tokens(int64_t bh, int64_t len) {
+    const int64_t most = std::max<int64_t>(16, std::min<int64_t>(64, 1024 / bh));
+    const int64_t chunks = std::min<int64_t>((len + kAmaxTokens - 1) / kAmaxTokens, most);
+    return (len + chunks - 1) / chunks;
+}
+int64_t v_chunks(int64_t bh, int64_t len) {
+    const int64_t tokens = v_chunk_tokens(bh, len);
+    return (len + tokens - 1) / tokens;
+}
+
+struct VArgs {
+    const uint16_t *v;
+    int64_t heads, len, lpad, s_b, s_h, s_l;
+    int64_t chunk_tokens, chunks;
+    float *partial;  // [B][H][chunks][D]
+    float *scale;    // [B][H][D], or [B][H][128] when wide
+    int8_t *vq;      // channel-major codes, D or (wide) 128 channels
+    int wide;
+};
 
 template <bool kFp16, int D>
-__global__ __launch_bounds__(kVThreads) void v_amax_kernel(const uint16_t *__restrict__ v, int64_t len, int64_t s_b,
-                                                          int64_t s_h, int64_t s_l, float *__restrict__ partial) {
+__device__ __forceinline__ void v_amax_body(const VArgs &a, int64_t chunk, int64_t h, int64_t b) {
     constexpr int kPacks = D / 8;
-    constexpr int kRows = kVThreads / kPacks;
-    __shared__ float wave_max[kVThreads / 64][D];
+    constexpr int kRows = kAmaxThreads / kPacks;
+    __shared__ float wave_max[kAmaxThreads / 64][D];
     const int tid = threadIdx.x;
     const int pack = tid % kPacks;
-    const int64_t chunk = blockIdx.x, h = blockIdx.y, b = blockIdx.z;
-    const int64_t chunks = gridDim.x, heads = gridDim.y;
-    const uint16_t *base = v + b * s_b + h * s_h;
+    const uint16_t *base = a.v + b * a.s_b + h * a.s_h;
     float m[8];
 #pragma unroll
     for (int j = 0; j < 8; ++j) m[j] = 0.0f;
-    const int64_t t_end = min(len, (chunk + 1) * kVChunk);
-#pragma unroll 4
-    for (int64_t t = chunk * kVChunk + tid / kPacks; t < t_end; t += kRows) {
-        const u32x4 raw = *reinterpret_cast<const u32x4 *>(base + t * s_l + pack * 8);
+    const int64_t t_end = min(a.len, (chunk + 1) * a.chunk_tokens);
+#pragma unroll 8
+    for (int64_t t = chunk * a.chunk_tokens + tid / kPacks; t < t_end; t += kRows) {
+        const u32x4 raw = *reinterpret_cast<const u32x4 *>(base + t * a.s_l + pack * 8);
 #pragma unroll
         for (int j = 0; j < 4; ++j) {
             m[2 * j] = fmaxf(m[2 * j], fabsf(h_to_f32<kFp16>(raw[j] & 0xffffu)));
@@ -265,58 +293,66 @@ __global__ __launch_bounds__(kVThreads) void v_amax_kernel(const uint16_t *__res
     }
     __syncthreads();
     if (tid < D) {
-        float a = 0.0f;
+        float x = 0.0f;
 #pragma unroll
-        for (int w = 0; w < kVThreads / 64; ++w) a = fmaxf(a, wave_max[w][tid]);
-        partial[((b * heads + h) * chunks + chunk) * D + tid] = a;
+        for (int w = 0; w < kAmaxThreads / 64; ++w) x = fmaxf(x, wave_max[w][tid]);
+        a.partial[((b * a.heads + h) * a.chunks + chunk) * D + tid] = x;
     }
-}
-
-template <int D>
-__global__ __launch_bounds__(D) void v_scale_kernel(const float *__restrict__ partial, int64_t chunks,
-                                                    float *__restrict__ scale) {
-    const int c = threadIdx.x;
-    const int64_t bh = blockIdx.x;
-    float a = 0.0f;
-    for (int64_t i = 0; i < chunks; ++i) a = fmaxf(a, partial[(bh * chunks + i) * D + c]);
-    scale[bh * D + c] = fmaxf(a / 127.0f, 1.0e-12f);
 }
 
 // One workgroup per 64-key tile: codes through an LDS byte tile (rows of D
 // + 16 bytes), written channel-major as 16-byte key runs.
 template <bool kFp16, int D>
-__global__ __launch_bounds__(kVThreads) void v_quant_kernel(const uint16_t *__restrict__ v, int64_t len, int64_t lpad,
-                                                           int64_t s_b, int64_t s_h, int64_t s_l,
-                                                           const float *__restrict__ scale, int8_t *__restrict__ vq) {
+__device__ __forceinline__ void v_quant_body(const VArgs &a, int64_t tix, int64_t h, int64_t b) {
     constexpr int kPacks = D / 8;
     constexpr int kRows = kVThreads / kPacks;
+    constexpr int kIters = 64 / kRows;
     constexpr int kRowBytes = D + 16;
+    constexpr int kParts = kVThreads / D;  // threads that share a channel's chunks
     __shared__ __align__(16) int8_t tile[64 * kRowBytes];
+    __shared__ float part_max[kParts][D];
+    __shared__ __align__(16) float inv_scale[D];
     const int tid = threadIdx.x;
     const int pack = tid % kPacks;
-    const int64_t tix = blockIdx.x, h = blockIdx.y, b = blockIdx.z;
-    const int64_t heads = gridDim.y;
-    const int64_t bh = b * heads + h;
-    const uint16_t *base = v + b * s_b + h * s_h;
+    const int64_t bh = b * a.heads + h;
+    const int64_t dout = a.wide ? 128 : D;
+    const uint16_t *base = a.v + b * a.s_b + h * a.s_h;
+    u32x4 raw[kIters];
+#pragma unroll
+    for (int it = 0; it < kIters; ++it) {
+        const int64_t t = tix * 64 + it * kRows + tid / kPacks;
+        raw[it] = u32x4{0u, 0u, 0u, 0u};
+        if (t < a.len) raw[it] = *reinterpret_cast<const u32x4 *>(base + t * a.s_l + pack * 8);
+    }
+    float m = 0.0f;
+#pragma unroll 4
+    for (int64_t i = tid / D; i < a.chunks; i += kParts) m = fmaxf(m, a.partial[(bh * a.chunks + i) * D + tid % D]);
+    part_max[tid / D][tid % D] = m;
+    __syncthreads();
+    if (tid < D) {
+#pragma unroll
+        for (int i = 0; i < kParts; ++i) m = fmaxf(m, part_max[i][tid]);
+        const float scale = fmaxf(m / 127.0f, 1.0e-12f);
+        inv_scale[tid] = 1.0f / scale;
+        if (tix == 0) {
+            a.scale[bh * dout + tid] = scale;
+            if (a.wide) a.scale[bh * dout + 64 + tid] = 1.0e-12f;  // D = 64
+        }
+    }
+    __syncthreads();
     float inv[8];
 #pragma unroll
-    for (int j = 0; j < 8; ++j) inv[j] = 1.0f / scale[bh * D + pack * 8 + j];
+    for (int j = 0; j < 8; ++j) inv[j] = inv_scale[pack * 8 + j];
 #pragma unroll
-    for (int r0 = 0; r0 < 64; r0 += kRows) {
-        const int r = r0 + tid / kPacks;
-        const int64_t t = tix * 64 + r;
-        u32x4 raw = u32x4{0u, 0u, 0u, 0u};
-        if (t < len) raw = *reinterpret_cast<const u32x4 *>(base + t * s_l + pack * 8);
-        int32_t q[8];
+    for (int it = 0; it < kIters; ++it) {
+        float y[8];
 #pragma unroll
         for (int j = 0; j < 4; ++j) {
-            q[2 * j] = sat_rne_s8(h_to_f32<kFp16>(raw[j] & 0xffffu) * inv[2 * j]);
-            q[2 * j + 1] = sat_rne_s8(h_to_f32<kFp16>(raw[j] >> 16) * inv[2 * j + 1]);
+            y[2 * j] = h_to_f32<kFp16>(raw[it][j] & 0xffffu) * inv[2 * j];
+            y[2 * j + 1] = h_to_f32<kFp16>(raw[it][j] >> 16) * inv[2 * j + 1];
         }
-        u32x2 packed;
-        packed.x = pack_s8x4(q[0], q[1], q[2], q[3]);
-        packed.y = pack_s8x4(q[4], q[5], q[6], q[7]);
-        *reinterpret_cast<u32x2 *>(tile + r * kRowBytes + pack * 8) = packed;
+        *reinterpret_cast<u32x2 *>(tile + (it * kRows + tid / kPacks) * kRowBytes + pack * 8) =
+            u32x2{sat_rne_s8x4(y[0], y[1], y[2], y[3]), sat_rne_s8x4(y[4], y[5], y[6], y[7])};
     }
     __syncthreads();
     // item = (channel, 16-key run)
@@ -334,20 +370,52 @@ __global__ __launch_bounds__(kVThreads) void v_quant_kernel(const uint16_t *__re
             }
             out[w] = word;
         }
-        *reinterpret_cast<u32x4 *>(vq + (bh * D + c) * lpad + tix * 64 + run * 16) = out;
+        int8_t *dst = a.vq + (bh * dout + c) * a.lpad + tix * 64 + run * 16;
+        *reinterpret_cast<u32x4 *>(dst) = out;
+        if (D == 64 && a.wide) *reinterpret_cast<u32x4 *>(dst + 64 * a.lpad) = u32x4{0u, 0u, 0u, 0u};
     }
 }
 
-}  // namespace
-}  // namespace tu
+template <bool kFp16, int D>
+__global__ __launch_bounds__(kAmaxThreads) void v_amax_kernel(VArgs a) {
+    v_amax_body<kFp16, D>(a, blockIdx.x, blockIdx.y, blockIdx.z);
+}
 
-extern "C" int32_t tu_w8a8_quant_qk(const void *q, const void *k, int32_t dtype, int64_t batch, int64_t hq,
-                                    int64_t hk, int64_t lq, int64_t lk, int64_t dim, int64_t q_sb, int64_t q_sh,
-                                    int64_t q_sl, int64_t k_sb, int64_t k_sh, int64_t k_sl, int8_t *q8,
-                                    int64_t q8_sb, int64_t q8_sh, int64_t q8_sl, int8_t *k8, int64_t k8_sb,
-                                    int64_t k8_sh, int64_t k8_sl, float *q_scale, float *k_scale,
-                                    int32_t *anchors, int32_t rotate, void *stream) {
-    using namespace tu;
+template <bool kFp16, int D>
+__global__ __launch_bounds__(kVThreads) void v_quant_kernel(VArgs a) {
+    v_quant_body<kFp16, D>(a, blockIdx.x, blockIdx.y, blockIdx.z);
+}
+
+// ---------------------------------------------------------------------------
+// The whole prologue in two launches (five kernels one after the other left
+// most of the GPU idle on ordinary lengths): what needs only the inputs, the
+// K anchors and the V chunk maxima, then what needs those, the Q / K and the
+// V codes.  Workgroups in that order along x, batches along y.
+// ---------------------------------------------------------------------------
+template <bool kFp16, int D>
+__global__ __launch_bounds__(kAnchorThreads) void w8a8_prep_stats_kernel(RotArgs r, VArgs a, int32_t *anchors,
+                                                                         uint32_t anchor_blocks) {
+    const uint32_t id = blockIdx.x, chunks = static_cast<uint32_t>(a.chunks);
+    const int64_t b = blockIdx.y;
+    if (id < anchor_blocks)
+        anchor_body<kFp16>(r.x[1], r.len[1], D, r.x_sb[1], r.x_sh[1], r.x_sl[1], anchors, id, b, r.heads[1]);
+    else
+        v_amax_body<kFp16, D>(a, (id - anchor_blocks) % chunks, (id - anchor_blocks) / chunks, b);
+}
+
+template <bool kFp16, int D>
+__global__ __launch_bounds__(kVThreads) void w8a8_prep_codes_kernel(RotArgs r, VArgs a, uint32_t rot_blocks) {
+    const uint32_t id = blockIdx.x, tiles = static_cast<uint32_t>(a.lpad / 64);
+    const int64_t b = blockIdx.y;
+    if (id < rot_blocks) rot_quant_body<kFp16, D>(r, id, b);
+    else v_quant_body<kFp16, D>(a, (id - rot_blocks) % tiles, (id - rot_blocks) / tiles, b);
+}
+
+// Argument checks and kernel arguments shared by the entry points (host only).
+int32_t check_qk(const void *q, const void *k, int32_t dtype, int64_t batch, int64_t hq, int64_t hk, int64_t lq,
+                 int64_t lk, int64_t dim, int64_t q_sb, int64_t q_sh, int64_t q_sl, int64_t k_sb, int64_t k_sh,
+                 int64_t k_sl, int8_t *q8, int64_t q8_sb, int64_t q8_sh, int64_t q8_sl, int8_t *k8, int64_t k8_sb,
+                 int64_t k8_sh, int64_t k8_sl, float *q_scale, float *k_scale) {
     TU_REQUIRE(dtype == 0 || dtype == 1, "W8A8 Q/K dtype must be 0 (bf16) or 1 (fp16)");
     TU_REQUIRE(dim == 64 || dim == 128, "W8A8 Q/K quantizer requires head_dim 64 or 128, got %lld",
                static_cast<long long>(dim));
@@ -363,16 +431,14 @@ extern "C" int32_t tu_w8a8_quant_qk(const void *q, const void *k, int32_t dtype,
                    k8_sl % 8 == 0 && (reinterpret_cast<uintptr_t>(q8) & 7) == 0 &&
                    (reinterpret_cast<uintptr_t>(k8) & 7) == 0,
                "W8A8 Q/K codes need 8-byte aligned rows");
-    if (require_gfx950()) return -1;
-    hipStream_t s = static_cast<hipStream_t>(stream);
-    if (anchors != nullptr) {
-        const dim3 grid(static_cast<unsigned>(hk), static_cast<unsigned>(batch));
-        if (dtype) anchor_kernel<true><<<grid, kAnchorThreads, 0, s>>>(static_cast<const uint16_t *>(k), lk,
-                                                                        static_cast<int>(dim), k_sb, k_sh, k_sl, anchors);
-        else anchor_kernel<false><<<grid, kAnchorThreads, 0, s>>>(static_cast<const uint16_t *>(k), lk,
-                                                                   static_cast<int>(dim), k_sb, k_sh, k_sl, anchors);
-        if (int32_t rc = check_launch("tu_w8a8_quant_qk (anchor)")) return rc;
-    }
+    return 0;
+}
+
+RotArgs rot_args(const void *q, const void *k, int64_t hq, int64_t hk, int64_t lq, int64_t lk, int64_t q_sb,
+                 int64_t q_sh, int64_t q_sl, int64_t k_sb, int64_t k_sh, int64_t k_sl, int8_t *q8, int64_t q8_sb,
+                 int64_t q8_sh, int64_t q8_sl, int8_t *k8, int64_t k8_sb, int64_t k8_sh, int64_t k8_sl, float *q_scale,
+                 float *k_scale, const int32_t *anchors, int32_t rotate) {
+    const int64_t nq = (lq + kChunk - 1) / kChunk, nk = (lk + kChunk - 1) / kChunk;
     RotArgs a{};
     a.x[0] = static_cast<const uint16_t *>(q);
     a.x[1] = static_cast<const uint16_t *>(k);
@@ -392,29 +458,12 @@ extern "C" int32_t tu_w8a8_quant_qk(const void *q, const void *k, int32_t dtype,
     a.o_sb[0] = q8_sb; a.o_sh[0] = q8_sh; a.o_sl[0] = q8_sl;
     a.o_sb[1] = k8_sb; a.o_sh[1] = k8_sh; a.o_sl[1] = k8_sl;
     a.rotate = rotate != 0;
-    const dim3 grid(static_cast<unsigned>(hq * nq + hk * nk), static_cast<unsigned>(batch));
-    if (dtype) {
-        if (dim == 128) rot_quant_kernel<true, 128><<<grid, kQkThreads, 0, s>>>(a);
-        else rot_quant_kernel<true, 64><<<grid, kQkThreads, 0, s>>>(a);
-    } else {
-        if (dim == 128) rot_quant_kernel<false, 128><<<grid, kQkThreads, 0, s>>>(a);
-        else rot_quant_kernel<false, 64><<<grid, kQkThreads, 0, s>>>(a);
-    }
-    return check_launch("tu_w8a8_quant_qk");
+    return a;
 }
 
-extern "C" int64_t tu_w8a8_quant_v_workspace(int64_t batch, int64_t heads, int64_t len, int64_t dim) {
-    if (batch <= 0 || heads <= 0 || len <= 0 || dim <= 0) return -1;
-    const int64_t chunks = (len + tu::kVChunk - 1) / tu::kVChunk;
-    // partial maxima (fp32)
-    return batch * heads * dim * chunks * 4;
-}
-
-extern "C" int32_t tu_w8a8_quant_v(const void *v, int32_t dtype, int64_t batch, int64_t heads, int64_t len,
-                                   int64_t dim, int64_t s_b, int64_t s_h, int64_t s_l, int8_t *vq, int64_t lpad,
-                                   float *scale, void *workspace, int64_t workspace_bytes,
-                                   void *stream) {
-    using namespace tu;
+int32_t check_v(const void *v, int32_t dtype, int64_t batch, int64_t heads, int64_t len, int64_t dim, int64_t s_b,
+                int64_t s_h, int64_t s_l, int8_t *vq, int64_t lpad, float *scale, void *workspace,
+                int64_t workspace_bytes) {
     TU_REQUIRE(dtype == 0 || dtype == 1, "W8A8 V dtype must be 0 (bf16) or 1 (fp16)");
     TU_REQUIRE(dim == 64 || dim == 128, "W8A8 V quantizer requires head_dim 64 or 128, got %lld",
                static_cast<long long>(dim));
@@ -422,33 +471,115 @@ extern "C" int32_t tu_w8a8_quant_v(const void *v, int32_t dtype, int64_t batch, 
                "W8A8 V quantizer dimensions out of range");
     TU_REQUIRE(lpad == (len + 63) / 64 * 64, "W8A8 V padded length must be ceil(len / 64) * 64");
     TU_REQUIRE(v && vq && scale && workspace, "W8A8 V quantizer pointers must be non-null");
-    TU_REQUIRE(workspace_bytes >= tu_w8a8_quant_v_workspace(batch, heads, len, dim),
+    TU_REQUIRE(workspace_bytes >= batch * heads * dim * v_chunks(batch * heads, len) * 4,
                "W8A8 V quantizer workspace too small");
     TU_REQUIRE(s_b % 8 == 0 && s_h % 8 == 0 && s_l % 8 == 0 && (reinterpret_cast<uintptr_t>(v) & 15) == 0 &&
                    (reinterpret_cast<uintptr_t>(vq) & 15) == 0 && (reinterpret_cast<uintptr_t>(workspace) & 3) == 0,
                "W8A8 V quantizer needs 16-byte aligned rows");
+    return 0;
+}
+
+VArgs v_args(const void *v, int64_t batch, int64_t heads, int64_t len, int64_t s_b, int64_t s_h, int64_t s_l,
+             int8_t *vq, int64_t lpad, float *scale, void *workspace, int wide) {
+    return VArgs{static_cast<const uint16_t *>(v), heads, len, lpad, s_b, s_h, s_l,
+                 v_chunk_tokens(batch * heads, len), v_chunks(batch * heads, len),
+                 static_cast<float *>(workspace), scale, vq, wide};
+}
+
+// f(kFp16, D) as compile-time constants.
+template <typename F>
+void with_type_and_dim(int32_t dtype, int64_t dim, F &&f) {
+    using std::bool_constant;
+    using std::integral_constant;
+    if (dtype) {
+        if (dim == 128) f(bool_constant<true>{}, integral_constant<int, 128>{});
+        else f(bool_constant<true>{}, integral_constant<int, 64>{});
+    } else {
+        if (dim == 128) f(bool_constant<false>{}, integral_constant<int, 128>{});
+        else f(bool_constant<false>{}, integral_constant<int, 64>{});
+    }
+}
+
+}  // namespace
+}  // namespace tu
+
+extern "C" int32_t tu_w8a8_quant_qk(const void *q, const void *k, int32_t dtype, int64_t batch, int64_t hq,
+                                    int64_t hk, int64_t lq, int64_t lk, int64_t dim, int64_t q_sb, int64_t q_sh,
+                                    int64_t q_sl, int64_t k_sb, int64_t k_sh, int64_t k_sl, int8_t *q8,
+                                    int64_t q8_sb, int64_t q8_sh, int64_t q8_sl, int8_t *k8, int64_t k8_sb,
+                                    int64_t k8_sh, int64_t k8_sl, float *q_scale, float *k_scale,
+                                    int32_t *anchors, int32_t rotate, void *stream) {
+    using namespace tu;
+    if (check_qk(q, k, dtype, batch, hq, hk, lq, lk, dim, q_sb, q_sh, q_sl, k_sb, k_sh, k_sl, q8, q8_sb, q8_sh, q8_sl,
+                 k8, k8_sb, k8_sh, k8_sl, q_scale, k_scale))
+        return -1;
     if (require_gfx950()) return -1;
     hipStream_t s = static_cast<hipStream_t>(stream);
-    const int64_t chunks = (len + kVChunk - 1) / kVChunk;
-    const int64_t ntiles = lpad / 64;
-    float *partial = static_cast<float *>(workspace);
-    const uint16_t *vp = static_cast<const uint16_t *>(v);
-    const dim3 g1(static_cast<unsigned>(chunks), static_cast<unsigned>(heads), static_cast<unsigned>(batch));
-    const dim3 g3(static_cast<unsigned>(ntiles), static_cast<unsigned>(heads), static_cast<unsigned>(batch));
-    const unsigned bh = static_cast<unsigned>(batch * heads);
-#define TU_V_LAUNCH(F16, DD)                                                                                  \
-    do {                                                                                                      \
-        v_amax_kernel<F16, DD><<<g1, kVThreads, 0, s>>>(vp, len, s_b, s_h, s_l, partial);                     \
-        v_scale_kernel<DD><<<bh, DD, 0, s>>>(partial, chunks, scale);                                         \
-        v_quant_kernel<F16, DD><<<g3, kVThreads, 0, s>>>(vp, len, lpad, s_b, s_h, s_l, scale, vq);            \
-    } while (0)
-    if (dtype) {
-        if (dim == 128) TU_V_LAUNCH(true, 128);
-        else TU_V_LAUNCH(true, 64);
-    } else {
-        if (dim == 128) TU_V_LAUNCH(false, 128);
-        else TU_V_LAUNCH(false, 64);
-    }
-#undef TU_V_LAUNCH
+    const RotArgs a = rot_args(q, k, hq, hk, lq, lk, q_sb, q_sh, q_sl, k_sb, k_sh, k_sl, q8, q8_sb, q8_sh, q8_sl, k8,
+                               k8_sb, k8_sh, k8_sl, q_scale, k_scale, anchors, rotate);
+    const dim3 grid(static_cast<unsigned>(hq * (a.ntiles[0] / 4) + hk * a.ntiles[1]), static_cast<unsigned>(batch));
+    const dim3 heads(static_cast<unsigned>(hk), static_cast<unsigned>(batch));
+    with_type_and_dim(dtype, dim, [&](auto f16, auto d) {
+        if (anchors != nullptr)
+            anchor_kernel<f16.value><<<heads, kAnchorThreads, 0, s>>>(a.x[1], lk, static_cast<int>(dim), k_sb, k_sh,
+                                                                      k_sl, anchors);
+        rot_quant_kernel<f16.value, d.value><<<grid, kQkThreads, 0, s>>>(a);
+    });
+    return check_launch("tu_w8a8_quant_qk");
+}
+
+extern "C" int64_t tu_w8a8_quant_v_workspace(int64_t batch, int64_t heads, int64_t len, int64_t dim) {
+    if (batch <= 0 || heads <= 0 || len <= 0 || dim <= 0) return -1;
+    // chunk maxima (fp32)
+    return batch * heads * dim * tu::v_chunks(batch * heads, len) * 4;
+}
+
+extern "C" int32_t tu_w8a8_quant_v(const void *v, int32_t dtype, int64_t batch, int64_t heads, int64_t len,
+                                   int64_t dim, int64_t s_b, int64_t s_h, int64_t s_l, int8_t *vq, int64_t lpad,
+                                   float *scale, void *workspace, int64_t workspace_bytes,
+                                   void *stream) {
+    using namespace tu;
+    if (check_v(v, dtype, batch, heads, len, dim, s_b, s_h, s_l, vq, lpad, scale, workspace, workspace_bytes)) return -1;
+    if (require_gfx950()) return -1;
+    hipStream_t s = static_cast<hipStream_t>(stream);
+    const VArgs a = v_args(v, batch, heads, len, s_b, s_h, s_l, vq, lpad, scale, workspace, 0);
+    const unsigned h = static_cast<unsigned>(heads), b = static_cast<unsigned>(batch);
+    with_type_and_dim(dtype, dim, [&](auto f16, auto d) {
+        v_amax_kernel<f16.value, d.value><<<dim3(static_cast<unsigned>(a.chunks), h, b), kAmaxThreads, 0, s>>>(a);
+        v_quant_kernel<f16.value, d.value><<<dim3(static_cast<unsigned>(lpad / 64), h, b), kVThreads, 0, s>>>(a);
+    });
     return check_launch("tu_w8a8_quant_v");
+}
+
+extern "C" int32_t tu_w8a8_prep(const void *q, const void *k, const void *v, int32_t dtype, int64_t batch, int64_t hq,
+                                int64_t hk, int64_t lq, int64_t lk, int64_t dim, int64_t q_sb, int64_t q_sh,
+                                int64_t q_sl, int64_t k_sb, int64_t k_sh, int64_t k_sl, int64_t v_sb, int64_t v_sh,
+                                int64_t v_sl, int8_t *q8, int64_t q8_sb, int64_t q8_sh, int64_t q8_sl, int8_t *k8,
+                                int64_t k8_sb, int64_t k8_sh, int64_t k8_sl, float *q_scale, float *k_scale,
+                                int32_t *anchors, int32_t rotate, int8_t *vq, int64_t lpad, float *v_scale,
+                                int32_t wide, void *workspace, int64_t workspace_bytes, void *stream) {
+    using namespace tu;
+    if (check_qk(q, k, dtype, batch, hq, hk, lq, lk, dim, q_sb, q_sh, q_sl, k_sb, k_sh, k_sl, q8, q8_sb, q8_sh, q8_sl,
+                 k8, k8_sb, k8_sh, k8_sl, q_scale, k_scale))
+        return -1;
+    if (check_v(v, dtype, batch, hk, lk, dim, v_sb, v_sh, v_sl, vq, lpad, v_scale, workspace, workspace_bytes)) return -1;
+    TU_REQUIRE(!wide || (dim == 64 && q8_sl >= 128 && k8_sl >= 128), "W8A8 wide codes are for head_dim 64 in rows of 128");
+    RotArgs r = rot_args(q, k, hq, hk, lq, lk, q_sb, q_sh, q_sl, k_sb, k_sh, k_sl, q8, q8_sb, q8_sh, q8_sl, k8, k8_sb,
+                         k8_sh, k8_sl, q_scale, k_scale, anchors, rotate);
+    r.wide = wide != 0;
+    const VArgs a = v_args(v, batch, hk, lk, v_sb, v_sh, v_sl, vq, lpad, v_scale, workspace, r.wide);
+    const int64_t anchor_blocks = anchors != nullptr ? hk : 0;
+    const int64_t rot_blocks = hq * (r.ntiles[0] / 4) + hk * r.ntiles[1];
+    const int64_t stats = anchor_blocks + hk * a.chunks, codes = rot_blocks + hk * (lpad / 64);
+    TU_REQUIRE(stats <= 0x7fffffff && codes <= 0x7fffffff, "W8A8 prologue grid too large");
+    if (require_gfx950()) return -1;
+    hipStream_t s = static_cast<hipStream_t>(stream);
+    const unsigned b = static_cast<unsigned>(batch);
+    with_type_and_dim(dtype, dim, [&](auto f16, auto d) {
+        w8a8_prep_stats_kernel<f16.value, d.value>
+            <<<dim3(static_cast<unsigned>(stats), b), kAnchorThreads, 0, s>>>(r, a, anchors, static_cast<uint32_t>(anchor_blocks));
+        w8a8_prep_codes_kernel<f16.value, d.value>
+            <<<dim3(static_cast<unsigned>(codes), b), kVThreads, 0, s>>>(r, a, static_cast<uint32_t>(rot_blocks));
+    });
+    return check_launch("tu_w8a8_prep");
 }

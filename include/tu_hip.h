@@ -387,6 +387,18 @@ int32_t tu_w8a8_quant_v(const void *v, int32_t dtype, int64_t batch, int64_t hea
                         int64_t dim, int64_t s_b, int64_t s_h, int64_t s_l, int8_t *vq, int64_t lpad,
                         float *scale, void *workspace, int64_t workspace_bytes, void *stream);
 
+/* tu_w8a8_quant_qk and tu_w8a8_quant_v in two launches: same arguments, codes,
+ * scales and anchors (rotate, anchors and the workspace as there).  wide (dim
+ * 64 only): q8 / k8 rows and vq / v_scale hold 128 channels, 64 .. 127 with
+ * zero codes and scale 1e-12, the layout tu_w8a8_attn_fwd reads. */
+int32_t tu_w8a8_prep(const void *q, const void *k, const void *v, int32_t dtype, int64_t batch, int64_t hq,
+                     int64_t hk, int64_t lq, int64_t lk, int64_t dim, int64_t q_sb, int64_t q_sh,
+                     int64_t q_sl, int64_t k_sb, int64_t k_sh, int64_t k_sl, int64_t v_sb, int64_t v_sh,
+                     int64_t v_sl, int8_t *q8, int64_t q8_sb, int64_t q8_sh, int64_t q8_sl, int8_t *k8,
+                     int64_t k8_sb, int64_t k8_sh, int64_t k8_sl, float *q_scale, float *k_scale,
+                     int32_t *anchors, int32_t rotate, int8_t *vq, int64_t lpad, float *v_scale,
+                     int32_t wide, void *workspace, int64_t workspace_bytes, void *stream);
+
 /* Dense W8A8 attention forward on INT8 Q/K/V:
  *   s = float(q8 . k8); masked keys (>= lk; causal: key > query, top-left)
  *       get the raw score -5e6
