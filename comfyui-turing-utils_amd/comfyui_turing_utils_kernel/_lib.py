@@ -193,6 +193,24 @@ def load() -> ctypes.CDLL:
         return lib
 
 
+_host = None
+
+
+def host_calls():
+    """The native host side of the hot calls (csrc/host_calls.cpp): functions
+    that serve a call in its plain form and return None for every other, which
+    then takes the general route.  Not for code that is being compiled."""
+    global _host
+    if _host is None:
+        load()
+        try:
+            from . import _host_calls
+        except ImportError as exc:
+            raise RuntimeError(f"failed to load the native host calls: {exc}; {BUILD_HINT}") from exc
+        _host = _host_calls
+    return _host
+
+
 def call(name: str, *args) -> None:
     """Calls a tu_* entry point and raises RuntimeError with tu_last_error() on failure."""
     lib = load()
@@ -216,6 +234,10 @@ def device_supported(device: torch.device) -> bool:
 
 def ptr(t: torch.Tensor | None) -> int | None:
     return None if t is None else t.data_ptr()
+
+
+# the current torch stream of a device index as a raw hipStream_t
+raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None)
 
 
 def stream_of(device: torch.device) -> int:

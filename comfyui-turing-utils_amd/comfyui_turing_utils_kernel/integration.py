@@ -27,6 +27,8 @@ import torch
 
 from . import _lib, ops  # noqa: F401  (ops registers torch.ops.turing_utils.*)
 
+_OUT_KIND = {torch.bfloat16: 0, torch.float16: 1, torch.float32: 2}
+_INPUT_ACT = {None: ops.ACT_NONE, "none": ops.ACT_NONE, "gelu_tanh": ops.ACT_GELU_TANH, "swiglu": ops.ACT_SWIGLU}
 SUPPORTED_INPUT_DTYPES = (torch.float16, torch.bfloat16, torch.float32)
 
 
@@ -65,6 +67,13 @@ def int8_linear(
     """
     if input_act not in (None, "none", "swiglu", "gelu_tanh"):
         raise ValueError(f"unsupported fused INT8 activation: {input_act!r}")
+    if type(x) is torch.Tensor and x.is_cuda and convrot and not torch.compiler.is_compiling():
+        kind = _OUT_KIND.get(out_dtype or x.dtype)
+        if kind is not None:
+            out = _lib.host_calls().int8_linear(x, weight, weight_scale, bias, kind, convrot_groupsize,
+                                                _INPUT_ACT[input_act], _lib.raw_stream(x.get_device()))
+            if out is not None:
+                return out
     if x.dtype != torch.bfloat16:
         raise NotImplementedError("gfx950 W8A8 linear takes bfloat16 activations")
     if not convrot:

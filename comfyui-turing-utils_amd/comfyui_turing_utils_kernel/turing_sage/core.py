@@ -350,6 +350,13 @@ def sageattn(
 ) -> torch.Tensor:
     """One-call Sage attention: K mean-smoothing, per-block INT8 Q/K, INT8 QK^T,
     online softmax, bf16 PV.  Output has q's shape and dtype."""
+    if type(q) is torch.Tensor and q.is_cuda and q.ndim == 4 and tensor_layout in ("HND", "NHD") \
+            and q.size(3) and not torch.compiler.is_compiling():
+        scale = float(sm_scale) if sm_scale is not None else q.size(3) ** -0.5
+        out = _lib.host_calls().sageattn(q, k, v, tensor_layout == "NHD", bool(is_causal), scale, bool(smooth_k), BLKQ,
+                                         BLKK, _compute_units(q.device), _lib.raw_stream(q.get_device()))
+        if out is not None:
+            return out
     quantized = prequantize_sageattn(
         q, k, v, tensor_layout=tensor_layout, is_causal=is_causal, sm_scale=sm_scale,
         smooth_k=smooth_k, BLKQ=BLKQ, BLKK=BLKK,
@@ -642,6 +649,13 @@ def w8a8attn(
     channel, P packed to unsigned 8 bits with the exp2 offset log2(255)."""
     if tensor_layout not in {"HND", "NHD"}:
         raise ValueError(f"Unsupported tensor_layout: {tensor_layout}")
+    if type(q) is torch.Tensor and q.is_cuda and q.ndim == 4 and tensor_layout == "HND" \
+            and key_tile_tokens in (0, 64, 128) and q.size(3) and not torch.compiler.is_compiling():
+        scale = float(sm_scale) if sm_scale is not None else q.size(3) ** -0.5
+        out = _lib.host_calls().w8a8attn(q, k, v, bool(is_causal), scale, bool(rotate_qk), bool(stabilize_k),
+                                         _lib.raw_stream(q.get_device()))
+        if out is not None:
+            return out
     if tensor_layout == "NHD":
         q_hnd, k_hnd, v_hnd = (t.transpose(1, 2).contiguous() for t in (q, k, v))
     else:
