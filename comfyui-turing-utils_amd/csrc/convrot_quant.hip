@@ -43,6 +43,7 @@
 // bits, so the quotient is never that close to a bf16 rounding midpoint, and
 // the CPU tests check, over every (value, scale) pair the quantizer can
 // produce, that the INT8 code is the IEEE division's.
+#include <algorithm>
 #include <type_traits>
 
 #include "ln_common.h"
@@ -154,7 +155,8 @@ __device__ __forceinline__ float gelu_tanh_f32(float x) {
     return (0.5f * x) * (1.0f + tanh_det<kF16>(inner));
 }
 
-__device__ __forceinline__ float swiglu(float gate, float up) { return (gate / (1.0f + exp_det(-gate))) * up; }
+__device__ __forceinline__ float silu(float gate) { return gate / (1.0f + exp_det(-gate)); }
+__device__ __forceinline__ float swiglu(float gate, float up) { return silu(gate) * up; }
 
 // Round-to-nearest-even to bf16 by the gfx950 conversion instruction
 // (v_cvt_pk_bf16_f32).  Identical to bf16_rne_bits for every non-NaN input;
@@ -246,7 +248,40 @@ __device__ __forceinline__ uint32_t gelu_lut_entry(int idx) {
     return __float_as_uint(g) >> 16;  // exact: g is a bf16 value (or the canonical NaN)
 }
 
+// SwiGLU's g / (1 + exp(-g)) by table: a function of the gate's 16 bits, as
+// fp32 values for |g| in [2^-18, 128) (25 exponents, 128 mantissas, both
+// signs, entry 2 (mag - kSiluLutLo) + sign), built in LDS by each workgroup
+// with the same operations.  A wave whose pass holds any other gate (about one
+// in 300 passes of unit-variance gates) computes all of it.  The upper end
+// covers outlier channels: with a table up to 16 and one channel in 1000 at
+// 20 times the others' scale, two passes in five were computed, and 2050 x
+// 14336 took 15 us longer than without a table.
+constexpr uint32_t kSiluLutLo = 109u << 7;  // magnitude bits of 2^-18
+constexpr int kSiluLutHalf = 25 * 128;
+constexpr int kSiluLut = 2 * kSiluLutHalf;
+constexpr int kSiluWaves = 3;  // waves per SIMD of the kernel with this table
+
+__device__ __forceinline__ float silu_lut_entry(int idx) {
+    return silu(bf16_bits_to_f32((static_cast<uint32_t>(idx & 1) << 15) | (kSiluLutLo + static_cast<uint32_t>(idx >> 1))));
+}
+
 typedef uint16_t u16x2 __attribute__((ext_vector_type(2)));
+
+// Table values of the two gates packed in w (halves outside the table read its
+// last entries) and, or-ed into `unusual`, bit 15 of each half outside it.
+__device__ __forceinline__ f32x2 silu_pair_lookup(uint32_t w, const float *lut, uint32_t &unusual) {
+    const u16x2 rel = __builtin_bit_cast(u16x2, w & 0x7fff7fffu) - static_cast<uint16_t>(kSiluLutLo);
+    // rel + (0x8000 - kSiluLutHalf), saturating: bit 15 set iff rel >= kSiluLutHalf
+    unusual |= __builtin_bit_cast(uint32_t, __builtin_elementwise_add_sat(
+                                                rel, static_cast<u16x2>(static_cast<uint16_t>(0x8000 - kSiluLutHalf))));
+    const u16x2 in = __builtin_elementwise_min(rel, static_cast<u16x2>(static_cast<uint16_t>(kSiluLutHalf - 1)));
+    const uint32_t t = __builtin_bit_cast(uint32_t, in << static_cast<uint16_t>(3));
+    const uint32_t sg = __builtin_bit_cast(uint32_t, __builtin_bit_cast(u16x2, w) >> static_cast<uint16_t>(13));
+    const uint32_t off = t | (sg & 0x00040004u);
+    const unsigned char *base = reinterpret_cast<const unsigned char *>(lut);
+    return f32x2{*reinterpret_cast<const float *>(base + (off & 0xffffu)),
+                 *reinterpret_cast<const float *>(base + (off >> 16))};
+}
 
 // 0xffff in each 16-bit half of x whose bit 15 is set, else 0 (one
 // v_pk_ashrrev_i16; written out because the compiler otherwise splits the
@@ -446,19 +481,24 @@ __device__ __forceinline__ void load_lane(LaneInput<kAct> &in, const uint16_t *x
 // element index 16 L + p with L = l % (G/16), p = d0 + 4 d1.  After the
 // transpose a lane holds, for G = 256, p = L and t = d2 + 4 d3 = 0..15; for
 // G = 128, p = 2L and 2L + 1 (z[t] and z[8 + t]) with t = d2 + 4 d3 = 0..7.
-// rows_per_block: rows per workgroup, in order (> 1 only for the bf16 GELU
-// by table, whose table build is then shared by that many rows).
-// kGeluTable: bf16 GELU by the LDS table, for rows of up to
+// rows_per_block: rows per workgroup, in order (> 1 only for activations by
+// table, whose build is then shared by that many rows).
+// kTable: the bf16 activation by its LDS table, for rows of up to
 // kTableThreads / 64 waves; its launch bound leaves the kernel twice the
 // registers (the 1024-thread bound capped it at 128 VGPRs, and it spilled).
-template <int G, int kAct, int kPasses, bool kF16, bool kGeluTable = false>
-__global__ __launch_bounds__(kGeluTable ? kTableThreads : 1024) void convrot_quant_i8_kernel(
+// SwiGLU's is held to three waves per SIMD: two, at 176 registers, took 59 us
+// for 2050 x 14336 of group 256 against 46.
+template <int G, int kAct, int kPasses, bool kF16, bool kTable = false>
+__global__ __launch_bounds__(kTable ? kTableThreads : 1024, kTable && kAct == 2 ? kSiluWaves : 1)
+void convrot_quant_i8_kernel(
     const uint16_t *__restrict__ x, int8_t *__restrict__ q, float *__restrict__ scales, int k, int staged_scale,
     int64_t rows, int rows_per_block) {
-    static_assert(!kGeluTable || (kAct == 1 && !kF16), "the GELU table is for bf16 GELU input");
+    static_assert(!kTable || (kAct != 0 && !kF16), "the tables are for bf16 activations");
+    constexpr bool kGeluTable = kTable && kAct == 1, kSiluTable = kTable && kAct == 2;
     extern __shared__ __align__(16) unsigned char smem[];
     __shared__ float wave_amax[kMaxWaves];
     __shared__ uint16_t gelu_lut[kGeluTable ? kGeluLut : 1];
+    __shared__ float silu_lut[kSiluTable ? kSiluLut : 1];
     constexpr int kLanesPerGroup = G / 16;
     // Transpose scratch: group gi starts at dword gi * kGroupDwords (padded so
     // the groups of a wave fall on different banks); element p of source lane
@@ -483,9 +523,13 @@ __global__ __launch_bounds__(kGeluTable ? kTableThreads : 1024) void convrot_qua
         for (int i = tid; i < kGeluLut; i += blockDim.x) gelu_lut[i] = static_cast<uint16_t>(gelu_lut_entry(i));
         __syncthreads();
     }
-    // one row per workgroup unless the GELU table is shared by several
-    const int64_t row0 = kGeluTable ? static_cast<int64_t>(blockIdx.x) * rows_per_block : blockIdx.x;
-    const int64_t row_end = kGeluTable ? min(rows, row0 + rows_per_block) : row0 + 1;
+    if constexpr (kSiluTable) {
+        for (int i = tid; i < kSiluLut; i += blockDim.x) silu_lut[i] = silu_lut_entry(i);
+        __syncthreads();
+    }
+    // one row per workgroup unless a table is shared by several
+    const int64_t row0 = kTable ? static_cast<int64_t>(blockIdx.x) * rows_per_block : blockIdx.x;
+    const int64_t row_end = kTable ? min(rows, row0 + rows_per_block) : row0 + 1;
     for (int64_t row = row0; row < row_end; ++row) {
         const uint16_t *xrow = x + row * in_stride;
         LaneInput<kAct> in[kPasses];
@@ -543,6 +587,23 @@ __global__ __launch_bounds__(kGeluTable ? kTableThreads : 1024) void convrot_qua
                             v[2 * j + 1] = activate<false>(__uint_as_float(w & 0xffff0000u), 0.0f,
                                                            std::integral_constant<int, 1>{});
                         }
+                    }
+                }
+            } else if constexpr (kSiluTable) {
+                uint32_t unusual = 0;
+#pragma unroll
+                for (int j = 0; j < 8; ++j) {
+                    const uint32_t u = in[pass].up[j / 4][j % 4];
+                    const f32x2 g = silu_pair_lookup(in[pass].x[j / 4][j % 4], silu_lut, unusual);
+                    v[2 * j] = g.x * __uint_as_float(u << 16);
+                    v[2 * j + 1] = g.y * __uint_as_float(u & 0xffff0000u);
+                }
+                if (__builtin_expect(__builtin_amdgcn_ballot_w64(active && (unusual & 0x80008000u) != 0) != 0, 0)) {
+#pragma unroll
+                    for (int j = 0; j < 8; ++j) {
+                        const uint32_t w = in[pass].x[j / 4][j % 4], u = in[pass].up[j / 4][j % 4];
+                        v[2 * j] = swiglu(__uint_as_float(w << 16), __uint_as_float(u << 16));
+                        v[2 * j + 1] = swiglu(__uint_as_float(w & 0xffff0000u), __uint_as_float(u & 0xffff0000u));
                     }
                 }
             } else {
@@ -830,8 +891,26 @@ extern "C" int32_t tu_convrot_quant_i8(const void *x_bf16, int8_t *q, float *sca
     const auto *xp = static_cast<const uint16_t *>(x_bf16);
     // The bf16 GELU of rows up to 8 waves builds a 7.5 KiB table per
     // workgroup, which 8 rows share; wider rows compute every GELU.
-    const bool table = act == TU_ACT_GELU_TANH && !f16 && waves * 64 <= kTableThreads;
-    const int rpb = table ? 8 : 1;
+    bool table = act == TU_ACT_GELU_TANH && !f16 && waves * 64 <= kTableThreads;
+    int rpb = table ? 8 : 1;
+    // The bf16 SwiGLU of rows of three to eight waves (of three from two rows a
+    // CU on) builds its 25 KiB table per workgroup; as many rows share it, up
+    // to 8, as leave the workgroups that fit the GPU together.  A workgroup
+    // evaluates 6400 gates for it, against 8960 in the narrowest of these rows.
+    //   2050 x 14336 (group 256)   58.8 -> 46.8 us     32760 x 13824   672 -> 532
+    //   4096 x 8960                63.3 -> 50.4        4096 x 20480    194 -> 182
+    //   1 x 14336                  14.0 -> 11.2        300 x 14336     17.1 -> 14.9
+    // Narrower rows or fewer of them are faster without: 64 x 8448 11.5 us
+    // against 12.9, 4000 x 5120 (two waves) 38.5 against 50.6.
+    if (act == TU_ACT_SWIGLU && !f16 && waves >= 3 && waves * 64 <= kTableThreads) {
+        int cus = 0;
+        if (device_cus(cus)) return -1;
+        if (waves > 3 || rows >= 2 * cus) {
+            const int64_t resident = static_cast<int64_t>(cus) * (kSiluWaves * 4 / waves);
+            table = true;
+            rpb = static_cast<int>(std::min<int64_t>(8, (rows + resident - 1) / resident));
+        }
+    }
     const dim3 grid(static_cast<unsigned>((rows + rpb - 1) / rpb));
 #define TU_CONVROT_LAUNCH_T(G, A, F, T)                                                                          \
     do {                                                                                                         \
@@ -845,7 +924,7 @@ extern "C" int32_t tu_convrot_quant_i8(const void *x_bf16, int8_t *q, float *sca
 #define TU_CONVROT_LAUNCH(G, A)                                         \
     do {                                                                \
         if (f16) TU_CONVROT_LAUNCH_T(G, A, true, false);                \
-        else if (table) TU_CONVROT_LAUNCH_T(G, A, false, (A == 1));     \
+        else if (table) TU_CONVROT_LAUNCH_T(G, A, false, (A != 0));     \
         else TU_CONVROT_LAUNCH_T(G, A, false, false);                   \
     } while (0)
     if (group == 256) {
