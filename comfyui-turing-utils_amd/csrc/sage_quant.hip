@@ -381,9 +381,10 @@ extern "C" int32_t tu_sage_prep(const void *q_bf16, const void *k_bf16, const vo
     TU_REQUIRE(need == 0 || (workspace && (reinterpret_cast<uintptr_t>(workspace) & 15) == 0 && workspace_bytes >= need),
                "Sage prologue workspace must be 16-byte aligned and hold %lld bytes", static_cast<long long>(need));
     const int64_t chunks = (lk + 127) / 128, q_blocks = (lq + blkq - 1) / blkq, k_blocks = (lk + blkk - 1) / blkk;
-    // every grid, and so every part of one, below 2^23 workgroups (2^31 threads)
+    // heads and batch as in the separate entry points; every grid, and so every
+    // part of one, below 2^23 workgroups (2^31 threads)
     constexpr int64_t kMost = int64_t{1} << 23;
-    TU_REQUIRE(batch <= kMost && hq <= kMost && hkv <= kMost && q_blocks <= kMost && lpad / kPrepKeys <= kMost &&
+    TU_REQUIRE(batch <= 65535 && hq <= 65535 && hkv <= 65535 && q_blocks <= kMost && lpad / kPrepKeys <= kMost &&
                    batch * hkv <= kMost && batch * hq <= kMost &&
                    batch * (hkv * (lpad / kPrepKeys + chunks) + hq * q_blocks) <= kMost && batch * hkv * k_blocks <= kMost,
                "Sage prologue grid too large");

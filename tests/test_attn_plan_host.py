@@ -64,3 +64,14 @@ def test_workspace_plan():
         for causal in (0, 1):
             # never more than 16 ranges of every row
             assert need(b, h, lq, lk, causal=causal) <= 16 * b * h * lq * (128 + 2) * 4
+
+
+@pytest.mark.parametrize("batch,hq,hkv", [(65536, 1, 1), (1, 65536, 1), (1, 65536, 65536)])
+def test_prologue_refuses_what_its_parts_refuse(batch, hq, hkv):
+    """tu_sage_quant and tu_sage_v_prep take at most 65535 heads and batch
+    entries; the shared prologue as well, before it looks for a device."""
+    buf = 1 << 12  # aligned, never dereferenced: the refusal comes first
+    need = _lib.load().tu_sage_prep_workspace(batch, hkv, 64, 64, 0)
+    with pytest.raises(RuntimeError, match="grid too large"):
+        _lib.call("tu_sage_prep", buf, buf, buf, batch, hq, hkv, 64, 64, 64, *(64,) * 9, 0, 128, 128, buf, 64, 64, 64,
+                  buf, 64, 64, 64, buf, buf, buf, 64, None, need, None)
