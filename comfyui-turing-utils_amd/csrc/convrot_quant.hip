@@ -240,6 +240,7 @@ constexpr int kGeluLutHalf = 15 * 128;      // exponents 2^-12 .. 2^2, 128 manti
 // Both signs, each padded to 2048 entries so that any 11-bit rel indexes
 // inside the table (the padding is never selected).
 constexpr int kGeluLut = 2 * 2048;
+constexpr int kGeluTableCost = 5000;         // building it, in lookups of row elements (fitted)
 
 __device__ __forceinline__ uint32_t gelu_lut_entry(int idx) {
     if ((idx >> 1) >= kGeluLutHalf) return 0u;  // padding
@@ -890,9 +891,34 @@ extern "C" int32_t tu_convrot_quant_i8(const void *x_bf16, int8_t *q, float *sca
     hipStream_t s = static_cast<hipStream_t>(stream);
     const auto *xp = static_cast<const uint16_t *>(x_bf16);
     // The bf16 GELU of rows up to 8 waves builds a 7.5 KiB table per
-    // workgroup, which 8 rows share; wider rows compute every GELU.
+    // workgroup, which up to 8 rows share; wider rows compute every GELU.
+    // Eight rows each on few workgroups left most compute units idle and each
+    // workgroup its rows one after another, so up to 24 rows a CU (32 for rows
+    // of one wave) the rows per workgroup minimise (the most loaded CU's waves, at least the 12 that hide
+    // its latencies) x (rows x columns + a table's cost), against the same
+    // without a table, where an element costs 1.65 of a lookup's.  Both
+    // constants fit rows 1..16000 x columns 512..26880 to 0.7 % of the best
+    // choice on average, 6.5 % at most:
+    //   16 x 512      25.9 -> 4.8 us (no table)    2050 x 13824   62.9 -> 42.1 (3 rows)
+    //   512 x 4096    59.4 -> 14.0 (no table)      4096 x 8960    66.2 -> 50.7 (4)
+    //   512 x 13824   57.8 -> 15.3 (1 row)         8190 x 3072    56.2 -> 44.4 (no table)
+    // Past that 8 rows stay: 7800 x 8960 and 13824 gain under 1 %, and 8192 x
+    // 8192 of group 256 took 97.0 us in fours against 89.9.
     bool table = act == TU_ACT_GELU_TANH && !f16 && waves * 64 <= kTableThreads;
     int rpb = table ? 8 : 1;
+    if (table) {
+        int cus = 0;
+        if (device_cus(cus)) return -1;
+        if (rows <= (waves == 1 ? 32 : 24) * static_cast<int64_t>(cus)) {
+            const auto load = [&](int64_t blocks) { return std::max<int64_t>(12, (blocks + cus - 1) / cus * waves); };
+            int64_t best = load(rows) * k * 33 / 20;
+            table = false, rpb = 1;
+            for (int r = 1; r <= 8; ++r) {
+                const int64_t cost = load((rows + r - 1) / r) * (static_cast<int64_t>(r) * k + kGeluTableCost);
+                if (cost < best) best = cost, table = true, rpb = r;
+            }
+        }
+    }
     // The bf16 SwiGLU of rows of three to eight waves (of three from two rows a
     // CU on) builds its 25 KiB table per workgroup; as many rows share it, up
     // to 8, as leave the workgroups that fit the GPU together.  A workgroup
