@@ -11,6 +11,7 @@ from __future__ import annotations
 import ctypes
 import os
 import threading
+import warnings
 
 import torch  # noqa: F401  (must precede the CDLL load, see module docstring)
 
@@ -193,21 +194,44 @@ def load() -> ctypes.CDLL:
         return lib
 
 
+class _GeneralRoute:
+    """Stands in for the native host calls: every call takes the general route."""
+
+    @staticmethod
+    def int8_linear(*args):
+        return None
+
+    sageattn = w8a8attn = int8_linear
+
+
 _host = None
 
 
 def host_calls():
     """The native host side of the hot calls (csrc/host_calls.cpp): functions
     that serve a call in its plain form and return None for every other, which
-    then takes the general route.  Not for code that is being compiled."""
+    then takes the general route.  Not for code that is being compiled.
+
+    The module is bound to the torch it was built against.  Where it is
+    missing, does not load or was built against another torch, a warning says
+    so once and every call takes the general route, which needs only
+    libtu_hip.so."""
     global _host
     if _host is None:
         load()
         try:
             from . import _host_calls
         except ImportError as exc:
-            raise RuntimeError(f"failed to load the native host calls: {exc}; {BUILD_HINT}") from exc
-        _host = _host_calls
+            reason = f"cannot be loaded: {exc}"
+        else:
+            built = getattr(_host_calls, "torch_version", None)
+            if built == torch.__version__:
+                _host = _host_calls
+                return _host
+            reason = f"was built against torch {built}, this is torch {torch.__version__}"
+        warnings.warn(f"the native host calls module {reason}; int8_linear, sageattn and w8a8attn take their slower "
+                      f"general route; {BUILD_HINT}", RuntimeWarning, stacklevel=3)
+        _host = _GeneralRoute
     return _host
 
 
@@ -236,8 +260,12 @@ def ptr(t: torch.Tensor | None) -> int | None:
     return None if t is None else t.data_ptr()
 
 
+def _stream_handle(index: int) -> int:
+    return torch.cuda.current_stream(index).cuda_stream
+
+
 # the current torch stream of a device index as a raw hipStream_t
-raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None)
+raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", _stream_handle)
 
 
 def stream_of(device: torch.device) -> int:

@@ -286,4 +286,13 @@ PyModuleDef module = {PyModuleDef_HEAD_INIT, "_host_calls", nullptr, -1, methods
 
 }  // namespace
 
-PyMODINIT_FUNC PyInit__host_calls() { return PyModule_Create(&module); }
+// torch_version: the torch whose headers and libraries this was built against;
+// the loader compares it with the running one.
+PyMODINIT_FUNC PyInit__host_calls() {
+    PyObject *m = PyModule_Create(&module);
+    if (m && PyModule_AddStringConstant(m, "torch_version", TU_TORCH_VERSION)) {
+        Py_DECREF(m);
+        return nullptr;
+    }
+    return m;
+}

@@ -181,3 +181,22 @@ def test_on_a_side_stream_and_under_capture(gpu_device):
         graph.replay()
         torch.cuda.synchronize()
         assert all(torch.equal(a, b) for a, b in zip(got, want))
+
+
+def test_without_the_module(gpu_device, monkeypatch):
+    """The three calls where the module does not load: the general route's results."""
+    import sys
+
+    import comfyui_turing_utils_kernel as package
+
+    x, w, ws, bias = _linear(gpu_device, rows=9)
+    q, k, v = (t.to(gpu_device) for t in inputs.attention(1, 4, 700, 128, 6))
+    calls = (lambda: integration.int8_linear(x, w, ws, bias, None, True, 128), lambda: core.sageattn(q, k, v),
+             lambda: core.w8a8attn(q, k, v))
+    want = [f() for f in calls]
+    monkeypatch.setattr(_lib, "_host", None)
+    monkeypatch.delattr(package, "_host_calls", raising=False)
+    monkeypatch.setitem(sys.modules, "comfyui_turing_utils_kernel._host_calls", None)
+    with pytest.warns(RuntimeWarning, match="cannot be loaded"):
+        got = [f() for f in calls]
+    assert all(torch.equal(a, b) for a, b in zip(got, want))
