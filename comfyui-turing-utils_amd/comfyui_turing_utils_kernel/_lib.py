@@ -33,6 +33,7 @@ SIGNATURES: dict[str, tuple[object, list[object]]] = {
     "tu_abi_version": (_i32, []),
     "tu_device_supported": (_i32, [_i32]),
     "tu_convrot_quant_i8": (_i32, [_c_void_p, _c_void_p, _c_void_p, _i64, _i64, _i32, _i32, _c_void_p]),
+    "tu_convrot_table_rows": (_i32, [_i64, _i64, _i32, _i32, _i32]),
     "tu_int8_gemm_bf16": (
         _i32,
         [_c_void_p, _c_void_p, _c_void_p, _c_void_p, _c_void_p, _c_void_p, _i64, _i64, _i64, _c_void_p],
@@ -163,7 +164,7 @@ SIGNATURES: dict[str, tuple[object, list[object]]] = {
     ),
 }
 
-ABI_VERSION = 16
+ABI_VERSION = 17
 
 _lock = threading.Lock()
 _lib: ctypes.CDLL | None = None

@@ -836,6 +836,69 @@ __global__ __launch_bounds__(kLnThreads) void ln_convrot_quant_kernel(
     });
 }
 
+// Few waves per row, each carrying up to kMaxPasses chunks: measured faster
+// than one chunk per wave (shorter barrier, more rows per CU).
+int row_passes(int k) { return std::min((k + kChunk - 1) / kChunk, kMaxPasses); }
+int row_waves(int k) { return ((k + kChunk - 1) / kChunk + row_passes(k) - 1) / row_passes(k); }
+
+// Time of `blocks` workgroups of `waves` on a CU that holds `resident` of them
+// at once, in waves at full rate: sets of `resident`, then the rest.  A set
+// takes its fullest SIMD's waves, but at least the `least` that hide its
+// latencies.
+int64_t cu_time(int64_t blocks, int resident, int waves, int64_t least) {
+    const auto set = [=](int64_t n) { return std::max<int64_t>(least, (n * waves + 3) / 4 * 4); };
+    const int64_t rest = blocks % resident;
+    return blocks / resident * set(resident) + (rest ? set(rest) : 0);
+}
+
+// Rows that share a workgroup's GELU table, 0 for none: the least of
+//   table:    cu_time x (rows x columns + kGeluTableCost)
+//   without:  cu_time x columns x 1.65, a row a workgroup
+// and 8 rows where nothing is predicted 7 % faster, or where the device holds
+// more than about two sets of such workgroups.  Rows of up to three passes of
+// one wave, 3072 columns, are fastest without (up to 3 % off the best of 171).
+// The waves a SIMD holds follow from the kernels' registers; a row of more
+// than four waves takes two on one SIMD, so of the group 256 table kernel's
+// three a SIMD a CU holds one such workgroup.  Over rows 1 .. 32760 x columns
+// 512 .. 32768 (461 shapes) the choice is 1.6 % off the best on average and at
+// most 3 % slower than 8 rows always.  Those left most CUs idle on few rows;
+// a rule that knew no residency and stopped at 24 rows a CU chose wrongly from
+// there on and for rows of five waves and more:
+//                        8 rows always   that rule   now
+//   16 x 512                25.9 us         4.8       4.8 (no table)
+//   512 x 4096              59.4           14.0      14.0 (no table)
+//   2050 x 13824            62.9           42.1      42.1 (3 rows)
+//   1560 x 20480 (256)      82.4           87.4      70.1 (no table)
+//   4096 x 16896            99.0          131.5      98.8 (8)
+//   6145 x 8192 (256)       83.9           84.8      74.1 (6)
+//   10000 x 5120            78.0           78.8      65.9 (5)
+int gelu_table_rows(int64_t rows, int k, int group, int cus) {
+    const int waves = row_waves(k);
+    if (waves * 64 > kTableThreads || k <= 3 * kChunk) return 0;
+    // waves a SIMD holds of the four-pass kernels
+    const int table_simd = group == 256 ? 3 : 4, plain_simd = group == 256 ? 5 : 6;
+    constexpr int kMany = 1 << 20;
+    int resident = 4 * table_simd / waves, plain = 4 * plain_simd / waves, least = 10;
+    if (waves > 4 && group == 256) resident = 1;
+    if (waves == 1) resident = plain = kMany, least = 12;
+    if (waves == 2) least = 9;
+    const auto per_cu = [&](int r) { return ((rows + r - 1) / r + cus - 1) / cus; };
+    const auto cost = [&](int64_t blocks, int r) {
+        return cu_time(blocks, resident, waves, least) * (static_cast<int64_t>(r) * k + kGeluTableCost);
+    };
+    // the eight rows' few workgroups past an even share hardly cost (6145 x
+    // 13824, 769 of them: 100 us, seven rows 108)
+    const int64_t eight = std::max<int64_t>(1, ((rows + 7) / 8 + cus - 1 - cus / 64) / cus);
+    if (eight > (waves == 1 ? 6 : std::max(3, 2 * resident))) return 8;
+    int best = 8;
+    int64_t lowest = cost(eight, 8) * 93 / 100;
+    const int64_t without = cu_time(per_cu(1), plain, waves, least) * k * 33 / 20;
+    if (without < lowest) best = 0, lowest = without;
+    for (int r = 1; r < 8; ++r)
+        if (const int64_t c = cost(per_cu(r), r); c < lowest) best = r, lowest = c;
+    return best;
+}
+
 // hidden = 256 per, per <= 20 (register-resident rows and rotated values).
 constexpr int kLnQuantMaxPer = 20;
 
@@ -882,43 +945,15 @@ extern "C" int32_t tu_convrot_quant_i8(const void *x_bf16, int8_t *q, float *sca
     if (rows == 0) return 0;
     const int k = static_cast<int>(cols);
     TU_REQUIRE(k <= kMaxCols, "ConvRot row of %d columns exceeds the %d-column limit", k, kMaxCols);
-    // Few waves per row, each carrying up to kMaxPasses chunks: measured
-    // faster than one chunk per wave (shorter barrier, more rows per CU).
-    const int nchunks = (k + kChunk - 1) / kChunk;
-    const int passes = nchunks < kMaxPasses ? nchunks : kMaxPasses;
-    const int waves = (nchunks + passes - 1) / passes;
+    const int passes = row_passes(k), waves = row_waves(k);
     const size_t lds = static_cast<size_t>(waves) * kScratchBytes;
     hipStream_t s = static_cast<hipStream_t>(stream);
     const auto *xp = static_cast<const uint16_t *>(x_bf16);
-    // The bf16 GELU of rows up to 8 waves builds a 7.5 KiB table per
-    // workgroup, which up to 8 rows share; wider rows compute every GELU.
-    // Eight rows each on few workgroups left most compute units idle and each
-    // workgroup its rows one after another, so up to 24 rows a CU (32 for rows
-    // of one wave) the rows per workgroup minimise (the most loaded CU's waves, at least the 12 that hide
-    // its latencies) x (rows x columns + a table's cost), against the same
-    // without a table, where an element costs 1.65 of a lookup's.  Both
-    // constants fit rows 1..16000 x columns 512..26880 to 0.7 % of the best
-    // choice on average, 6.5 % at most:
-    //   16 x 512      25.9 -> 4.8 us (no table)    2050 x 13824   62.9 -> 42.1 (3 rows)
-    //   512 x 4096    59.4 -> 14.0 (no table)      4096 x 8960    66.2 -> 50.7 (4)
-    //   512 x 13824   57.8 -> 15.3 (1 row)         8190 x 3072    56.2 -> 44.4 (no table)
-    // Past that 8 rows stay: 7800 x 8960 and 13824 gain under 1 %, and 8192 x
-    // 8192 of group 256 took 97.0 us in fours against 89.9.
-    bool table = act == TU_ACT_GELU_TANH && !f16 && waves * 64 <= kTableThreads;
-    int rpb = table ? 8 : 1;
-    if (table) {
-        int cus = 0;
-        if (device_cus(cus)) return -1;
-        if (rows <= (waves == 1 ? 32 : 24) * static_cast<int64_t>(cus)) {
-            const auto load = [&](int64_t blocks) { return std::max<int64_t>(12, (blocks + cus - 1) / cus * waves); };
-            int64_t best = load(rows) * k * 33 / 20;
-            table = false, rpb = 1;
-            for (int r = 1; r <= 8; ++r) {
-                const int64_t cost = load((rows + r - 1) / r) * (static_cast<int64_t>(r) * k + kGeluTableCost);
-                if (cost < best) best = cost, table = true, rpb = r;
-            }
-        }
-    }
+    int cus = 0;
+    if (act != TU_ACT_NONE && device_cus(cus)) return -1;
+    int rpb = act == TU_ACT_GELU_TANH && !f16 ? gelu_table_rows(rows, k, group, cus) : 0;
+    bool table = rpb > 0;
+    rpb = std::max(rpb, 1);
     // The bf16 SwiGLU of rows of three to eight waves (of three from two rows a
     // CU on) builds its 25 KiB table per workgroup; as many rows share it, up
     // to 8, as leave the workgroups that fit the GPU together.  A workgroup
@@ -929,8 +964,6 @@ extern "C" int32_t tu_convrot_quant_i8(const void *x_bf16, int8_t *q, float *sca
     // Narrower rows or fewer of them are faster without: 64 x 8448 11.5 us
     // against 12.9, 4000 x 5120 (two waves) 38.5 against 50.6.
     if (act == TU_ACT_SWIGLU && !f16 && waves >= 3 && waves * 64 <= kTableThreads) {
-        int cus = 0;
-        if (device_cus(cus)) return -1;
         if (waves > 3 || rows >= 2 * cus) {
             const int64_t resident = static_cast<int64_t>(cus) * (kSiluWaves * 4 / waves);
             table = true;
@@ -965,6 +998,12 @@ extern "C" int32_t tu_convrot_quant_i8(const void *x_bf16, int8_t *q, float *sca
 #undef TU_CONVROT_LAUNCH
 #undef TU_CONVROT_LAUNCH_T
     return check_launch("tu_convrot_quant_i8");
+}
+
+extern "C" int32_t tu_convrot_table_rows(int64_t rows, int64_t cols, int32_t group, int32_t act, int32_t cus) {
+    using namespace tu;
+    if (rows <= 0 || cols <= 0 || cols > kMaxCols || (group != 128 && group != 256) || cus <= 0) return 0;
+    return act == TU_ACT_GELU_TANH ? gelu_table_rows(rows, static_cast<int>(cols), group, cus) : 0;
 }
 
 namespace {

@@ -81,6 +81,12 @@ int32_t tu_device_supported(int32_t device);
 int32_t tu_convrot_quant_i8(const void *x_bf16, int8_t *q, float *scale, int64_t rows,
                             int64_t cols, int32_t group, int32_t act, void *stream);
 
+/* The rows that share one workgroup's activation table in tu_convrot_quant_i8
+ * of bf16 input on a device with `cus` compute units, 0 where the activation
+ * is computed (host only, no HIP call; every choice gives the same bits).
+ * No counterpart in the reference. */
+int32_t tu_convrot_table_rows(int64_t rows, int64_t cols, int32_t group, int32_t act, int32_t cus);
+
 /* INT8 GEMM ---------------------------------------------------------------- */
 
 /* out[m][n] = bf16_rn(((float(acc) * a_scale[m]) * w_scale[n]) + bias[n]),

@@ -1,0 +1,53 @@
+"""Host checks of the rules by which a launch picks its variant: the library's
+own host-only queries, at sizes where both sides were measured on 256 CUs."""
+from __future__ import annotations
+
+import pytest
+
+from comfyui_turing_utils_kernel import _lib
+
+CUS = 256
+
+
+@pytest.fixture(scope="module")
+def lib():
+    return _lib.load()
+
+
+# (rows, columns, group): the rows that share a table, 0 for none, and what was slower
+GELU_ROWS = [
+    (4096, 16896, 128, {8}),          # 99 us; 1 to 7 rows 117-154
+    (4096, 20480, 128, {8}),          # 116; 134-177
+    (1560, 20480, 256, {0, 7}),       # 70, 74; one row 87, eight 83
+    (4096, 20480, 256, {0}),          # 157; four rows 176, eight 172
+    (10000, 5120, 128, {5}),          # 66; eight 78
+    (6144, 8192, 256, {4, 6}),        # 63, 70; eight 84
+    (6145, 8192, 256, {4, 5, 6}),     # as 6144: no step between them
+    (6145, 13824, 128, {8}),          # 100; seven 108
+    (2050, 13824, 128, {2, 3}),       # 41; eight 59
+    (512, 13824, 128, {1}),           # 16; eight 58
+    (7800, 8960, 128, {4, 8}),        # 93; one row 119
+    (32760, 13824, 128, {8}),
+]
+
+
+@pytest.mark.parametrize("rows,k,group,good", GELU_ROWS)
+def test_gelu_rows(lib, rows, k, group, good):
+    assert lib.tu_convrot_table_rows(rows, k, group, 1, CUS) in good
+
+
+def test_gelu_rows_range(lib):
+    """Short rows, rows too wide for a table, other activations and bad
+    arguments have none; the choice never leaves 0 .. 8."""
+    for rows in (1, 300, 8190, 16000, 32760):
+        for k in (512, 1536, 3072):
+            assert lib.tu_convrot_table_rows(rows, k, 128, 1, CUS) == 0
+        assert lib.tu_convrot_table_rows(rows, 65536, 128, 1, CUS) == 0
+    for act in (0, 3):
+        assert lib.tu_convrot_table_rows(4096, 8960, 128, act, CUS) == 0
+    for rows, k, group, cus in ((0, 8960, 128, CUS), (5, 0, 128, CUS), (5, 8960, 64, CUS), (5, 8960, 128, 0), (5, 65537, 128, CUS)):
+        assert lib.tu_convrot_table_rows(rows, k, group, 1, cus) == 0
+    for cus in (1, 64, 256, 304):
+        for rows in (1, 2, 255, 257, 4097, 100003, 2 ** 31 - 1):
+            for k in (3200, 4096, 4224, 8192, 16896, 20480, 32768):
+                assert 0 <= lib.tu_convrot_table_rows(rows, k, 128, 1, cus) <= 8

@@ -20,11 +20,11 @@ def _quantize(x, group):
     return q.cpu().numpy(), s.cpu().numpy().reshape(-1)
 
 
-# on 256 CUs: no table, 1, 3 and 4 rows a workgroup, the last rows of the rule and the first past it (of one wave
-# and of two), 8 and 7 waves
+# on 256 CUs: no table, 1, 3, 4, 5, 6, 7 and 8 rows a workgroup, rows of one to eight waves
 @pytest.mark.parametrize("rows,k,group", [(1, 128, 128), (515, 4096, 256), (1, 8960, 128), (513, 13824, 128),
                                           (2050, 13824, 256), (4097, 8960, 128), (6144, 4352, 128), (6145, 4352, 128),
-                                          (8192, 1152, 128), (8193, 1152, 128), (3, 32768, 256), (257, 26880, 128)])
+                                          (8192, 1152, 128), (8193, 1152, 128), (3, 32768, 256), (257, 26880, 128),
+                                          (4001, 16640, 128), (5001, 5120, 128), (6145, 8192, 256), (1561, 20480, 256)])
 def test_rows_and_widths(gpu_device, rows, k, group):
     print(f"[gelu rows] rows={rows} k={k} group={group}", flush=True)
     x = torch.randn(rows, k, generator=torch.Generator().manual_seed(rows + k))
