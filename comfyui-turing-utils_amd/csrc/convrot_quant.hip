@@ -250,38 +250,76 @@ __device__ __forceinline__ uint32_t gelu_lut_entry(int idx) {
 }
 
 // SwiGLU's g / (1 + exp(-g)) by table: a function of the gate's 16 bits, as
-// fp32 values for |g| in [2^-18, 128) (25 exponents, 128 mantissas, both
-// signs, entry 2 (mag - kSiluLutLo) + sign), built in LDS by each workgroup
-// with the same operations.  A wave whose pass holds any other gate (about one
-// in 300 passes of unit-variance gates) computes all of it.  The upper end
-// covers outlier channels: with a table up to 16 and one channel in 1000 at
-// 20 times the others' scale, two passes in five were computed, and 2050 x
-// 14336 took 15 us longer than without a table.
-constexpr uint32_t kSiluLutLo = 109u << 7;  // magnitude bits of 2^-18
-constexpr int kSiluLutHalf = 25 * 128;
-constexpr int kSiluLut = 2 * kSiluLutHalf;
-constexpr int kSiluWaves = 3;  // waves per SIMD of the kernel with this table
+// fp32 values for |g| in [2^-24, 89) (both signs, entry 2 (mag - kSiluLutLo) +
+// sign), built in LDS by each workgroup
+// with the same operations, and behind them +inf and -0 for every other gate.
+// A wave whose pass holds one gives all of it the closed forms of
+// silu_outside, no exp: computing such passes made data with zero gates,
+// padded rows or large outlier channels slower than a kernel without a table
+// (2050 x 14336 group 256, all gates zero 53.5 -> 85.3 us, now 46.7).
+constexpr uint32_t kSiluLutLo = 103u << 7;  // magnitude bits of 2^-24
+constexpr int kSiluLutHalf = 30 * 128 + 50;
+constexpr int kSiluLut = 2 * kSiluLutHalf + 2;
+constexpr int kSiluWaves = 3;           // waves per SIMD of the kernel with this table
+constexpr int kSiluTableCost = 3000;    // building it, in lookups of row elements (fitted)
 
 __device__ __forceinline__ float silu_lut_entry(int idx) {
+    if ((idx >> 1) == kSiluLutHalf) return idx & 1 ? -0.0f : __builtin_inff();
     return silu(bf16_bits_to_f32((static_cast<uint32_t>(idx & 1) << 15) | (kSiluLutLo + static_cast<uint32_t>(idx >> 1))));
 }
 
 typedef uint16_t u16x2 __attribute__((ext_vector_type(2)));
 
-// Table values of the two gates packed in w (halves outside the table read its
-// last entries) and, or-ed into `unusual`, bit 15 of each half outside it.
+// Table values of the two gates packed in w (+inf or -0 for a half outside the
+// table) and, or-ed into `unusual`, bit 15 of each half outside it.
 __device__ __forceinline__ f32x2 silu_pair_lookup(uint32_t w, const float *lut, uint32_t &unusual) {
     const u16x2 rel = __builtin_bit_cast(u16x2, w & 0x7fff7fffu) - static_cast<uint16_t>(kSiluLutLo);
     // rel + (0x8000 - kSiluLutHalf), saturating: bit 15 set iff rel >= kSiluLutHalf
     unusual |= __builtin_bit_cast(uint32_t, __builtin_elementwise_add_sat(
                                                 rel, static_cast<u16x2>(static_cast<uint16_t>(0x8000 - kSiluLutHalf))));
-    const u16x2 in = __builtin_elementwise_min(rel, static_cast<u16x2>(static_cast<uint16_t>(kSiluLutHalf - 1)));
+    const u16x2 in = __builtin_elementwise_min(rel, static_cast<u16x2>(static_cast<uint16_t>(kSiluLutHalf)));
     const uint32_t t = __builtin_bit_cast(uint32_t, in << static_cast<uint16_t>(3));
     const uint32_t sg = __builtin_bit_cast(uint32_t, __builtin_bit_cast(u16x2, w) >> static_cast<uint16_t>(13));
     const uint32_t off = t | (sg & 0x00040004u);
     const unsigned char *base = reinterpret_cast<const unsigned char *>(lut);
     return f32x2{*reinterpret_cast<const float *>(base + (off & 0xffffu)),
                  *reinterpret_cast<const float *>(base + (off >> 16))};
+}
+
+// The 16 looked-up values v of a lane's gates x, right for gates inside the
+// table, made right for all, bit for bit silu() (checked over every gate):
+//   |g| >= 89: exp(-g) is 0 or inf, so g = min(+inf, g), or -0;
+//   below 2^-24, zeros among them: 1 + exp(-g) rounds to 2, so g / 2;
+//   -inf and NaN, where some lane of the wave has one: NaN.
+// v <= |g| for every gate inside the table, so the minimum leaves it alone.
+// Zeros alone in the wave, as a padded row has them, are told apart first (a
+// zero's sign is lost there; no code or scale depends on it).
+__device__ __forceinline__ void silu_outside(float (&v)[16], const u32x4 (&x)[2], bool active) {
+    uint32_t any = 0, special = 0;
+#pragma unroll
+    for (int j = 0; j < 8; ++j) {
+        const uint32_t mag = x[j / 4][j % 4] & 0x7fff7fffu;
+        any |= mag;
+        // bit 15 of a half: an infinity or NaN
+        special |= __builtin_bit_cast(uint32_t, __builtin_bit_cast(u16x2, mag) + static_cast<uint16_t>(0x80));
+    }
+    if (__builtin_amdgcn_ballot_w64(any != 0) == 0) {
+#pragma unroll
+        for (int i = 0; i < 16; ++i) v[i] = 0.0f;
+        return;
+    }
+    const auto gate = [&](int i) {
+        const uint32_t w = x[i / 8][i / 2 % 4];
+        return __uint_as_float(i & 1 ? w & 0xffff0000u : w << 16);
+    };
+#pragma unroll
+    for (int i = 0; i < 16; ++i) {
+        const float g = gate(i);
+        v[i] = fabsf(g) < 5.9604644775390625e-8f ? 0.5f * g : fminf(v[i], fabsf(g));
+    }
+    if (__builtin_amdgcn_ballot_w64(active && (special & 0x80008000u) != 0) == 0) return;
+#pragma unroll
+    for (int i = 0; i < 16; ++i) v[i] = gate(i) >= -3.38953139e38f ? v[i] : __builtin_nanf("");
 }
 
 // 0xffff in each 16-bit half of x whose bit 15 is set, else 0 (one
@@ -594,18 +632,17 @@ void convrot_quant_i8_kernel(
                 uint32_t unusual = 0;
 #pragma unroll
                 for (int j = 0; j < 8; ++j) {
-                    const uint32_t u = in[pass].up[j / 4][j % 4];
                     const f32x2 g = silu_pair_lookup(in[pass].x[j / 4][j % 4], silu_lut, unusual);
-                    v[2 * j] = g.x * __uint_as_float(u << 16);
-                    v[2 * j + 1] = g.y * __uint_as_float(u & 0xffff0000u);
+                    v[2 * j] = g.x;
+                    v[2 * j + 1] = g.y;
                 }
-                if (__builtin_expect(__builtin_amdgcn_ballot_w64(active && (unusual & 0x80008000u) != 0) != 0, 0)) {
+                if (__builtin_expect(__builtin_amdgcn_ballot_w64(active && (unusual & 0x80008000u) != 0) != 0, 0))
+                    silu_outside(v, in[pass].x, active);
 #pragma unroll
-                    for (int j = 0; j < 8; ++j) {
-                        const uint32_t w = in[pass].x[j / 4][j % 4], u = in[pass].up[j / 4][j % 4];
-                        v[2 * j] = swiglu(__uint_as_float(w << 16), __uint_as_float(u << 16));
-                        v[2 * j + 1] = swiglu(__uint_as_float(w & 0xffff0000u), __uint_as_float(u & 0xffff0000u));
-                    }
+                for (int j = 0; j < 8; ++j) {
+                    const uint32_t u = in[pass].up[j / 4][j % 4];
+                    v[2 * j] *= __uint_as_float(u << 16);
+                    v[2 * j + 1] *= __uint_as_float(u & 0xffff0000u);
                 }
             } else {
 #pragma unroll
@@ -899,6 +936,32 @@ int gelu_table_rows(int64_t rows, int k, int group, int cus) {
     return best;
 }
 
+// The same for SwiGLU's 30 KiB table, which only rows of four waves (12289 to
+// 16384 columns) take: three such workgroups share a CU in LDS and registers,
+// four without a table, where an element costs 1.4 of a lookup's (1.33: a gain
+// of 5 % or more, which gates outside the table take part of).  For rows of
+// three waves the table costs a fourth workgroup a CU (4096 x 8960 65 us
+// without, 75 with), for wider ones there is room for one or two (2050 x 20480
+// 106 us without, 117 with).  us without a table and with it, for unit-variance
+// gates, one channel in 1000 zero, and all gates zero:
+//   2050 x 14336 (group 256)   54.3 -> 46.4    54.6 -> 50.7    53.5 -> 46.7
+//   16380 x 13824               336 -> 285      339 -> 315      302 -> 286
+//   1 x 14336 (group 256)      14.4 -> 13.0    14.3 -> 13.9    14.3 -> 13.3
+//   4096 x 14336 (group 256)   91.8 -> 86.2    91.9 -> 92.4    88.0 -> 88.4
+// All gates nonzero and below 2^-24 cost up to 7 % more than without.
+int silu_table_rows(int64_t rows, int k, int cus) {
+    const int waves = row_waves(k);
+    if (waves != 4) return 0;
+    const auto per_cu = [&](int r) { return ((rows + r - 1) / r + cus - 1) / cus; };
+    int best = 0;
+    int64_t lowest = cu_time(per_cu(1), 4, waves, 10) * k * 133 / 100;
+    for (int r = 1; r <= 8; ++r) {
+        const int64_t c = cu_time(per_cu(r), kSiluWaves, waves, 10) * (static_cast<int64_t>(r) * k + kSiluTableCost);
+        if (c < lowest) best = r, lowest = c;
+    }
+    return best;
+}
+
 // hidden = 256 per, per <= 20 (register-resident rows and rotated values).
 constexpr int kLnQuantMaxPer = 20;
 
@@ -951,25 +1014,11 @@ extern "C" int32_t tu_convrot_quant_i8(const void *x_bf16, int8_t *q, float *sca
     const auto *xp = static_cast<const uint16_t *>(x_bf16);
     int cus = 0;
     if (act != TU_ACT_NONE && device_cus(cus)) return -1;
-    int rpb = act == TU_ACT_GELU_TANH && !f16 ? gelu_table_rows(rows, k, group, cus) : 0;
-    bool table = rpb > 0;
+    int rpb = 0;
+    if (act == TU_ACT_GELU_TANH && !f16) rpb = gelu_table_rows(rows, k, group, cus);
+    if (act == TU_ACT_SWIGLU && !f16) rpb = silu_table_rows(rows, k, cus);
+    const bool table = rpb > 0;
     rpb = std::max(rpb, 1);
-    // The bf16 SwiGLU of rows of three to eight waves (of three from two rows a
-    // CU on) builds its 25 KiB table per workgroup; as many rows share it, up
-    // to 8, as leave the workgroups that fit the GPU together.  A workgroup
-    // evaluates 6400 gates for it, against 8960 in the narrowest of these rows.
-    //   2050 x 14336 (group 256)   58.8 -> 46.8 us     32760 x 13824   672 -> 532
-    //   4096 x 8960                63.3 -> 50.4        4096 x 20480    194 -> 182
-    //   1 x 14336                  14.0 -> 11.2        300 x 14336     17.1 -> 14.9
-    // Narrower rows or fewer of them are faster without: 64 x 8448 11.5 us
-    // against 12.9, 4000 x 5120 (two waves) 38.5 against 50.6.
-    if (act == TU_ACT_SWIGLU && !f16 && waves >= 3 && waves * 64 <= kTableThreads) {
-        if (waves > 3 || rows >= 2 * cus) {
-            const int64_t resident = static_cast<int64_t>(cus) * (kSiluWaves * 4 / waves);
-            table = true;
-            rpb = static_cast<int>(std::min<int64_t>(8, (rows + resident - 1) / resident));
-        }
-    }
     const dim3 grid(static_cast<unsigned>((rows + rpb - 1) / rpb));
 #define TU_CONVROT_LAUNCH_T(G, A, F, T)                                                                          \
     do {                                                                                                         \
@@ -980,11 +1029,14 @@ extern "C" int32_t tu_convrot_quant_i8(const void *x_bf16, int8_t *q, float *sca
             default: convrot_quant_i8_kernel<G, A, 4, F, T><<<grid, waves * 64, lds, s>>>(xp, q, scale, k, staged_scale, rows, rpb); break; \
         }                                                                                                        \
     } while (0)
-#define TU_CONVROT_LAUNCH(G, A)                                         \
-    do {                                                                \
-        if (f16) TU_CONVROT_LAUNCH_T(G, A, true, false);                \
-        else if (table) TU_CONVROT_LAUNCH_T(G, A, false, (A != 0));     \
-        else TU_CONVROT_LAUNCH_T(G, A, false, false);                   \
+    // tables are for rows of four passes
+#define TU_CONVROT_LAUNCH(G, A)                                                                                  \
+    do {                                                                                                         \
+        if (f16) TU_CONVROT_LAUNCH_T(G, A, true, false);                                                         \
+        else if (table)                                                                                          \
+            convrot_quant_i8_kernel<G, A, 4, false, (A != 0)><<<grid, waves * 64, lds, s>>>(xp, q, scale, k,     \
+                                                                                            staged_scale, rows, rpb); \
+        else TU_CONVROT_LAUNCH_T(G, A, false, false);                                                            \
     } while (0)
     if (group == 256) {
         if (act == 0) TU_CONVROT_LAUNCH(256, 0);
@@ -1003,7 +1055,10 @@ extern "C" int32_t tu_convrot_quant_i8(const void *x_bf16, int8_t *q, float *sca
 extern "C" int32_t tu_convrot_table_rows(int64_t rows, int64_t cols, int32_t group, int32_t act, int32_t cus) {
     using namespace tu;
     if (rows <= 0 || cols <= 0 || cols > kMaxCols || (group != 128 && group != 256) || cus <= 0) return 0;
-    return act == TU_ACT_GELU_TANH ? gelu_table_rows(rows, static_cast<int>(cols), group, cus) : 0;
+    const int k = static_cast<int>(cols);
+    return act == TU_ACT_GELU_TANH ? gelu_table_rows(rows, k, group, cus)
+           : act == TU_ACT_SWIGLU  ? silu_table_rows(rows, k, cus)
+                                   : 0;
 }
 
 namespace {

@@ -43,7 +43,7 @@ def test_gelu_rows_range(lib):
         for k in (512, 1536, 3072):
             assert lib.tu_convrot_table_rows(rows, k, 128, 1, CUS) == 0
         assert lib.tu_convrot_table_rows(rows, 65536, 128, 1, CUS) == 0
-    for act in (0, 3):
+    for act in (0, 2, 3):
         assert lib.tu_convrot_table_rows(4096, 8960, 128, act, CUS) == 0
     for rows, k, group, cus in ((0, 8960, 128, CUS), (5, 0, 128, CUS), (5, 8960, 64, CUS), (5, 8960, 128, 0), (5, 65537, 128, CUS)):
         assert lib.tu_convrot_table_rows(rows, k, group, 1, cus) == 0
@@ -51,3 +51,16 @@ def test_gelu_rows_range(lib):
         for rows in (1, 2, 255, 257, 4097, 100003, 2 ** 31 - 1):
             for k in (3200, 4096, 4224, 8192, 16896, 20480, 32768):
                 assert 0 <= lib.tu_convrot_table_rows(rows, k, 128, 1, cus) <= 8
+
+
+@pytest.mark.parametrize("rows,k,good", [
+    (2050, 14336, {3}),           # 46 us; without a table 54
+    (16380, 13824, {4, 5, 8}),    # 285; 336
+    (1, 14336, {1}),              # 13.0; 14.4
+    (4096, 8960, {0}), (513, 8448, {0}), (2050, 20480, {0}), (1000, 32768, {0}), (4096, 5120, {0}),  # slower with one
+])
+def test_swiglu_rows(lib, rows, k, good):
+    """Only rows of four waves share a SwiGLU table."""
+    for group in (128, 256):
+        if k % group == 0:
+            assert lib.tu_convrot_table_rows(rows, k, group, 2, CUS) in good

@@ -45,8 +45,9 @@ def test_every_gate(gpu_device, group):
     np.testing.assert_array_equal(np.isnan(s[255:]), np.isnan(rs.reshape(-1)[255:]))
 
 
+# on 256 CUs: 1, 3 and 4 rows a workgroup, and rows without a table (of three, five and eight waves, and four)
 @pytest.mark.parametrize("rows,k,group", [(1, 12544, 256), (513, 8448, 256), (769, 14336, 256), (2050, 8320, 128), (515, 20480, 128),
-                                          (300, 32768, 256)])
+                                          (300, 32768, 256), (515, 12416, 128), (2051, 16384, 256), (3001, 12544, 128)])
 def test_rows_and_widths(gpu_device, rows, k, group):
     """Workgroups of one and several rows, the last one short; a few gates
     outside the table (0, 2^-19, 200, -130) in some passes."""
@@ -63,3 +64,43 @@ def test_rows_and_widths(gpu_device, rows, k, group):
     rq, rs = oracle.convrot_quant(inputs.bits(x[some].contiguous()), group, act=2)
     np.testing.assert_array_equal(s[some].view(np.uint32), rs.reshape(-1).view(np.uint32))
     np.testing.assert_array_equal(q[some], rq)
+
+
+@pytest.mark.parametrize("rows,k,group", [(3, 14336, 256), (2050, 12544, 128)])
+def test_gates_outside_the_table(gpu_device, rows, k, group):
+    """Rows of zero gates of both signs (with finite, infinite and NaN up
+    values), of gates around the table's ends, of single gates outside it, and
+    ordinary rows, in turn."""
+    import comfyui_turing_utils_kernel.ops  # noqa: F401
+
+    print(f"[silu table] outside rows={rows} k={k} group={group}", flush=True)
+    g = torch.Generator().manual_seed(rows + 1)
+    gate = torch.randn(rows, k, generator=g)
+    up = torch.randn(rows, k, generator=g)
+    ends = torch.tensor([0.0, -0.0, 2.0 ** -133, -2.0 ** -126, 2.0 ** -25, -2.0 ** -24, 2.0 ** -24, 2.0 ** -23, 88.5, -88.5,
+                         89.0, -89.0, 128.0, -130.0, 3e38, -3e38])
+    for r in range(rows):
+        kind = r % 6
+        if kind == 0:
+            gate[r] = torch.where(torch.arange(k) % 2 == 0, 0.0, -0.0)
+        elif kind == 1:
+            gate[r] = ends[torch.randint(0, 14, (k,), generator=g)]
+        elif kind == 2:
+            gate[r] = ends[torch.randint(0, 7, (k,), generator=g)]
+        elif kind == 3:
+            at = torch.arange(0, k, 1031)
+            gate[r, at] = ends[torch.arange(at.numel()) % 16]
+    x = torch.cat([gate, up], 1).to(torch.bfloat16)
+    q, s = _quantize(x.to(gpu_device), group)
+    some = [r for r in range(rows) if r < 12 or r >= rows - 8]
+    rq, rs = oracle.convrot_quant(inputs.bits(x[some].contiguous()), group, act=2)
+    np.testing.assert_array_equal(s[some].view(np.uint32), rs.reshape(-1).view(np.uint32))
+    np.testing.assert_array_equal(q[some], rq)
+    # a zero gate times an infinite or NaN up value is NaN, in this row alone
+    x[0, k + 5] = float("inf")
+    x[0, k + 2000] = float("nan")
+    q2, s2 = _quantize(x.to(gpu_device), group)
+    rq, rs = oracle.convrot_quant(inputs.bits(x[:1].contiguous()), group, act=2)
+    np.testing.assert_array_equal(s2[:1].view(np.uint32), rs.reshape(-1).view(np.uint32))
+    np.testing.assert_array_equal(q2[:1], rq)
+    np.testing.assert_array_equal(q2[1:], q[1:])
