@@ -50,6 +50,7 @@ SIGNATURES: dict[str, tuple[object, list[object]]] = {
         _i32,
         [_c_void_p, _c_void_p, _c_void_p, _c_void_p, _c_void_p, _c_void_p, _i32, _i64, _i64, _i64, _i32, _c_void_p],
     ),
+    "tu_int8_gemm_tile": (_i32, [_i64, _i64, _i64, _i32]),
     "tu_int8_gemm_tile_policy": (_i32, [_i64, _i64, _i32]),
     "tu_int8_gemm_bf16_residual": (
         _i32,
@@ -164,7 +165,7 @@ SIGNATURES: dict[str, tuple[object, list[object]]] = {
     ),
 }
 
-ABI_VERSION = 17
+ABI_VERSION = 18
 
 _lock = threading.Lock()
 _lib: ctypes.CDLL | None = None

@@ -663,10 +663,11 @@ constexpr double kHalfTileCost = TU_GEMM_HALF_TILE_COST;
 // K 5120 (0.75 of the MFMAs plus the fixed part).
 constexpr double kTile192Cost = 0.85;
 
-// The choice among the three tiles of tu_int8_gemm_ex from the grid alone: one
-// workgroup per CU, so tiles run in rounds of `cus`; 128 x 256 or 256 x 192
-// tiles are chosen when their rounds cost less than the 256 x 256 tiles' (a
-// grid of a few, partly empty rounds).  A launch that is left to choose
+// What tu_int8_gemm_tile_policy answers: the best of tu_int8_gemm_ex's three
+// tiles from the grid alone, for a caller that names one.  One workgroup per
+// CU, so tiles run in rounds of `cus`; 128 x 256 or 256 x 192 tiles are chosen
+// when their rounds cost less than the 256 x 256 tiles' (a grid of a few,
+// partly empty rounds).  No launch takes it: one that is left to choose
 // (pick_tile below) knows K and the smaller tiles too.
 int pick_tile_policy(int64_t m, int64_t n, int cus) {
     const int64_t t256 = (m + 255) / 256 * ((n + 255) / 256);
@@ -685,44 +686,57 @@ constexpr int kTile128x192 = 16, kTile128x128 = 17, kTile128x64 = 18, kTile64x64
 
 // Automatic tile: the least of first + rounds * (fixed + per_step * steps),
 // rounds = tiles / CUs rounded up and steps of 128 bytes of K, in us.  The
-// constants are fitted to times at K 1536 and 5120 with one and several
-// rounds (graph of 12 launches, bf16 out with bias, three operand sets).  A
-// step of a small grid costs the bytes that a CU pulls past its L2, about 70
+// constants are fitted to the times of every tile at 228 shapes of M 1 to
+// 28567, N 256 to 19872 and K 512 to 14336 (graph of 3 to 24 launches, bf16 out
+// with bias, three operand sets): the tile taken is at most 2.9 % slower than
+// the best one there, at 90 other shapes 1.6 %, 0.05 % on average at both.
+// A step of a small grid costs the bytes that a CU pulls past its L2, about 70
 // GB/s, so its time goes with BM + BN whatever the MFMAs do; the fewer
 // columns and rows a CU has to pull while all CUs have a tile, the better,
 // and the smallest two tiles leave room for a second workgroup on the CU.
-//   M x N x K             before (128 x 256 x 2 stages)   now
-//   1 x 9216 x 1536       14.3 us                          6.8 us (64 x 64)
-//   128 x 5120 x 5120     39.3                             12.6 (64 x 64)
-//   1024 x 1536 x 1536    16.2                             8.5 (128 x 64)
-//   512 x 5120 x 5120     38.8                             22.5 (128 x 128)
-//   512 x 10240 x 5120    39.4                             30.0 (128 x 192)
-// 256 x 192 stays best from 1024 x 8960 x 1536 (20.2 us against 25.5 with
-// 128 x 192) and 256 x 256 from about ten rounds on.
+// Over ten rounds it is the MFMAs and the power they take that count, and the
+// larger tile reads its operands less often.
+//                       256x256  256x192  128x256  128x192  128x128   128x64    64x64  (us; * taken)
+//   1 x 8960 x 1536          19.4     16.2     13.1     10.7      9.0      7.3      6.1*
+//   512 x 5120 x 5120        51.0     44.9     32.6     27.6     22.6*    27.9     29.9
+//   512 x 10240 x 5120       51.8     45.4     34.4     29.9*    44.4     42.3     48.7
+//   1024 x 1536 x 1536       21.1     18.2     14.4     11.6     10.0      8.2*     9.4
+//   1024 x 8960 x 1536       23.2     20.8*    30.4     26.0     29.1     28.4     35.9
+//   2050 x 8960 x 1536       47.6     40.9*    47.2     50.4     49.2     54.6     72.8
+//   16380 x 1536 x 1536      49.8     44.6*    49.9     52.3     59.8     66.1     87.1
+//   4096 x 10240 x 5120     183.0*   203.2    201.5    216.5    241.0    285.9    374.4
+//   7800 x 5120 x 5120      184.0*   198.8    198.3    212.0    231.2    273.4    353.2
+//   1560 x 5120 x 13824     153.4    144.9    166.7    136.2*   153.9    168.4    188.3
+//   4096 x 5120 x 13824     323.7    293.3    298.9*   323.9    322.7    407.5    489.6
 struct TileCost {
     int policy, bm, bn;
     double first, fixed, per_step;
 };
 constexpr TileCost kTileCosts[] = {
-    {TU_GEMM_TILE_256, 256, 256, 1.5, 10.0, 1.125}, {TU_GEMM_TILE_192, 256, 192, 1.5, 8.7, 0.957},
-    {TU_GEMM_TILE_128, 128, 256, 1.5, 5.3, 0.668},  {kTile128x192, 128, 192, 1.5, 3.9, 0.56},
-    {kTile128x128, 128, 128, 1.5, 3.2, 0.44},       {kTile128x64, 128, 64, 3.0, 1.6, 0.27},
-    {kTile64x64, 64, 64, 2.3, 1.65, 0.178},
+    {TU_GEMM_TILE_256, 256, 256, 0.085, 8.17, 1.23}, {TU_GEMM_TILE_192, 256, 192, 0.225, 5.69, 1.2},
+    {TU_GEMM_TILE_128, 128, 256, 0.0, 8.67, 0.718},  {kTile128x192, 128, 192, 0.0, 7.98, 0.548},
+    {kTile128x128, 128, 128, 0.477, 4.61, 0.465},    {kTile128x64, 128, 64, 2.03, 1.95, 0.299},
+    {kTile64x64, 64, 64, 1.17, 1.34, 0.249},
 };
 
-int pick_tile(int64_t m, int64_t n, int64_t k, int cus) {
+// A launch takes fewer than 2^32 threads: a tile of fewer rows than the grid
+// limit allows is passed over (64 x 64 from 536 million rows on).
+constexpr int64_t kMaxTiles = 0xffffffffll / kThreads;
+
+const TileCost &pick_tile(int64_t m, int64_t n, int64_t k, int cus) {
     const double steps = static_cast<double>((k + kBK - 1) / kBK);
-    int best = TU_GEMM_TILE_256;
+    const TileCost *best = kTileCosts;
     double best_cost = 0.0;
     for (const TileCost &t : kTileCosts) {
         const int64_t tiles = (m + t.bm - 1) / t.bm * ((n + t.bn - 1) / t.bn);
+        if (&t != kTileCosts && tiles > kMaxTiles) continue;
         const double cost = t.first + static_cast<double>((tiles + cus - 1) / cus) * (t.fixed + t.per_step * steps);
         if (&t == kTileCosts || cost < best_cost) {
-            best = t.policy;
+            best = &t;
             best_cost = cost;
         }
     }
-    return best;
+    return *best;
 }
 
 template <int kOut, bool kResidual = false>
@@ -733,7 +747,7 @@ int32_t launch_gemm(const int8_t *a, const int8_t *w, const float *as, const flo
     if (policy == TU_GEMM_TILE_AUTO) {
         int cus = 0;
         if (device_cus(cus)) return -1;
-        policy = pick_tile(m, n, k, cus);
+        policy = pick_tile(m, n, k, cus).policy;
     }
     hipStream_t st = static_cast<hipStream_t>(stream);
 #define TU_TILE(BM, BN, NST, WPE)                                                                                 \
@@ -875,4 +889,10 @@ extern "C" int32_t tu_int8_gemm_ex(const int8_t *a, const int8_t *w, const float
 extern "C" int32_t tu_int8_gemm_tile_policy(int64_t m, int64_t n, int32_t cus) {
     if (m <= 0 || n <= 0 || cus <= 0) return TU_GEMM_TILE_256;
     return tu::pick_tile_policy(m, n, cus);
+}
+
+extern "C" int32_t tu_int8_gemm_tile(int64_t m, int64_t n, int64_t k, int32_t cus) {
+    if (m <= 0 || n <= 0 || k <= 0 || cus <= 0) return 0;
+    const tu::TileCost &t = tu::pick_tile(m, n, k, cus);
+    return t.bm << 16 | t.bn;
 }

@@ -145,6 +145,11 @@ int32_t tu_int8_gemm_ex(const int8_t *a, const int8_t *w, const float *a_scale, 
  * w4a8.cu:837-851. */
 int32_t tu_int8_gemm_tile_policy(int64_t m, int64_t n, int32_t cus);
 
+/* The tile of a launch that is left to choose (TU_GEMM_TILE_AUTO and the
+ * entry points without a policy), rows << 16 | columns; 0 for bad arguments
+ * (host only, no HIP call).  No counterpart in the reference. */
+int32_t tu_int8_gemm_tile(int64_t m, int64_t n, int64_t k, int32_t cus);
+
 /* The same GEMM with a gated residual add fused into the epilogue, for a DiT
  * block's x + y * gate: out[m][n] = bf16_rn(fma(y, g, residual[m][n])) with
  * y the tu_int8_gemm_bf16 value above, g = gate[m / gate_rows][n] (bf16 [G, n],

@@ -64,3 +64,39 @@ def test_swiglu_rows(lib, rows, k, good):
     for group in (128, 256):
         if k % group == 0:
             assert lib.tu_convrot_table_rows(rows, k, group, 2, CUS) in good
+
+
+# (m, n, k): the tiles within 3 % of the best one, and what was slower
+GEMM_TILES = [
+    (2050, 8960, 1536, {(256, 192)}),                # 40.9 us; 128 x 256 47.2
+    (16380, 1536, 1536, {(256, 192)}),               # 44.6; 256 x 256 and 128 x 256 50
+    (4096, 10240, 5120, {(256, 256)}),               # 183; 128 x 256 202
+    (7800, 5120, 5120, {(256, 256)}),                # 184; 128 x 256 198
+    (7800, 5120, 13824, {(256, 256)}),               # 469; 128 x 256 503
+    (16380, 5376, 14336, {(256, 256)}),              # 1032; 256 x 192 1078
+    (1560, 5120, 13824, {(128, 192)}),               # 136; 256 x 192 145
+    (32760, 13824, 5120, {(256, 256)}),              # 1845; 256 x 192 2058
+    (1024, 8960, 1536, {(256, 192)}),                # 20.8; 256 x 256 23.2, 128 x 192 26.0
+    (512, 10240, 5120, {(128, 192)}),                # 29.9; 128 x 256 34.4
+    (512, 5120, 5120, {(128, 128)}),                 # 22.6; 128 x 192 27.6
+    (1024, 1536, 1536, {(128, 64)}),                 # 8.2; 64 x 64 9.4
+    (1, 8960, 1536, {(64, 64)}),                     # 6.1; 128 x 64 7.3
+]
+
+
+@pytest.mark.parametrize("m,n,k,good", GEMM_TILES)
+def test_gemm_tile(lib, m, n, k, good):
+    t = lib.tu_int8_gemm_tile(m, n, k, CUS)
+    assert (t >> 16, t & 0xFFFF) in good
+
+
+def test_gemm_tile_range(lib):
+    """A grid of the tile taken holds fewer than 2^32 threads wherever one of
+    256 x 256 tiles does, and bad arguments are answered with 0."""
+    for m in (1, 2 ** 20, 2 ** 29 - 64, 2 ** 29, 2 ** 30, 2 ** 30 + 1, 2 ** 31 - 256):
+        for n, k in ((8, 16), (64, 16), (64, 4096), (128, 256), (256, 512)):
+            t = lib.tu_int8_gemm_tile(m, n, k, CUS)
+            bm, bn = t >> 16, t & 0xFFFF
+            assert -(-m // bm) * -(-n // bn) * 512 < 2 ** 32, (m, n, k)
+    for bad in ((0, 8, 16, 256), (8, 0, 16, 256), (8, 8, 0, 256), (8, 8, 16, 0)):
+        assert lib.tu_int8_gemm_tile(*bad) == 0
