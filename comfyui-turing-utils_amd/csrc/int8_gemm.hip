@@ -686,8 +686,8 @@ constexpr int kTile128x192 = 16, kTile128x128 = 17, kTile128x64 = 18, kTile64x64
 
 // Automatic tile: the least of first + rounds * (fixed + per_step * steps),
 // rounds = tiles / CUs rounded up and steps of 128 bytes of K, in us.  The
-// constants are fitted to the times of every tile at 228 shapes of M 1 to
-// 28567, N 256 to 19872 and K 512 to 14336 (graph of 3 to 24 launches, bf16 out
+// constants are fitted to the times of every tile at 340 shapes of M 1 to
+// 32760, N 256 to 19872 and K 64 to 14336 (graph of 3 to 24 launches, bf16 out
 // with bias, three operand sets): the tile taken is at most 2.9 % slower than
 // the best one there, at 90 other shapes 1.6 %, 0.05 % on average at both.
 // A step of a small grid costs the bytes that a CU pulls past its L2, about 70
@@ -713,10 +713,10 @@ struct TileCost {
     double first, fixed, per_step;
 };
 constexpr TileCost kTileCosts[] = {
-    {TU_GEMM_TILE_256, 256, 256, 0.085, 8.17, 1.23}, {TU_GEMM_TILE_192, 256, 192, 0.225, 5.69, 1.2},
-    {TU_GEMM_TILE_128, 128, 256, 0.0, 8.67, 0.718},  {kTile128x192, 128, 192, 0.0, 7.98, 0.548},
-    {kTile128x128, 128, 128, 0.477, 4.61, 0.465},    {kTile128x64, 128, 64, 2.03, 1.95, 0.299},
-    {kTile64x64, 64, 64, 1.17, 1.34, 0.249},
+    {TU_GEMM_TILE_256, 256, 256, 0.0, 8.09, 1.25},  {TU_GEMM_TILE_192, 256, 192, 0.097, 6.81, 1.19},
+    {TU_GEMM_TILE_128, 128, 256, 0.0, 6.94, 0.757}, {kTile128x192, 128, 192, 0.0, 6.18, 0.569},
+    {kTile128x128, 128, 128, 0.3, 4.8, 0.478},      {kTile128x64, 128, 64, 2.63, 1.45, 0.323},
+    {kTile64x64, 64, 64, 2.31, 1.12, 0.25},
 };
 
 // A launch takes fewer than 2^32 threads: a tile of fewer rows than the grid

@@ -70,6 +70,7 @@ def test_swiglu_rows(lib, rows, k, good):
 GEMM_TILES = [
     (2050, 8960, 1536, {(256, 192)}),                # 40.9 us; 128 x 256 47.2
     (16380, 1536, 1536, {(256, 192)}),               # 44.6; 256 x 256 and 128 x 256 50
+    (1024, 5120, 256, {(128, 192)}),                 # 7.5; 256 x 192 9.2
     (4096, 10240, 5120, {(256, 256)}),               # 183; 128 x 256 202
     (7800, 5120, 5120, {(256, 256)}),                # 184; 128 x 256 198
     (7800, 5120, 13824, {(256, 256)}),               # 469; 128 x 256 503
