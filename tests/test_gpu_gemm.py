@@ -155,16 +155,19 @@ def test_int8_linear_residual_exact(gpu_device, m, n, k, with_bias, gate_rows):
     np.testing.assert_array_equal(inputs.bits(res_dev), inputs.bits(residual))
 
 
-def test_residual_and_bf16_on_192_wide_tiles(gpu_device):
-    """A grid that the tile policy runs on 256 x 192 tiles (2048 x 8968: two
-    rounds of them on 256 CUs, a ragged last 192-wide tile): the bf16 output
-    and the gated residual epilogue, 96 sampled rows bit-exact against the
-    oracle."""
+@pytest.mark.parametrize("m,n,k,tile", [(2048, 8968, 256, (256, 192)), (3008, 4104, 272, (256, 256)), (3008, 2568, 1040, (256, 192)),
+                                        (1504, 4104, 1040, (128, 256)), (1008, 4104, 528, (128, 192))])
+def test_residual_and_bf16_on_large_tiles(gpu_device, m, n, k, tile):
+    """Grids that a launch runs on each of the larger tiles (several rounds,
+    ragged last rows and columns): the bf16 output and the gated residual
+    epilogue, 96 sampled rows bit-exact against the oracle."""
     from comfyui_turing_utils_kernel import _lib
 
-    m, n, k, gate_rows = 2048, 8968, 256, 16
-    print(f"[gemm 256x192] m={m} n={n} k={k} policy={_lib.load().tu_int8_gemm_tile_policy(m, n, 256)}", flush=True)
-    assert _lib.load().tu_int8_gemm_tile_policy(m, n, 256) == 3
+    gate_rows = 16
+    cus = torch.cuda.get_device_properties(gpu_device).multi_processor_count
+    got = _lib.load().tu_int8_gemm_tile(m, n, k, cus)
+    print(f"[gemm tiles] m={m} n={n} k={k} tile={got >> 16} x {got & 0xFFFF}", flush=True)
+    assert cus != 256 or (got >> 16, got & 0xFFFF) == tile
     a = _rand_i8((m, k), 5)
     w, ws, bias = inputs.weights(n, k, 6, True)
     g = torch.Generator().manual_seed(9)

@@ -17,12 +17,21 @@ def _rand_i8(shape, seed):
     return torch.randint(-128, 128, shape, generator=torch.Generator().manual_seed(seed), dtype=torch.int8)
 
 
+def _tile(device, m, n, k):
+    """The tile of the launch, None on another number of CUs than the shapes were chosen for."""
+    cus = torch.cuda.get_device_properties(device).multi_processor_count
+    t = _lib.load().tu_int8_gemm_tile(m, n, k, cus)
+    return (t >> 16, t & 0xFFFF) if cus == 256 else None
+
+
 # K of 0 to 6 full 128-byte steps with and without a partial one, and long
 @pytest.mark.parametrize("k", [16, 112, 128, 256, 272, 384, 512, 528, 640, 768, 5120])
-# one tile and less; 64 x 64; 128 x 64; 128 x 128; 128 x 192 (by K, on 256 CUs)
-@pytest.mark.parametrize("m,n", [(1, 8), (65, 72), (63, 1032), (130, 5128), (515, 2568), (1000, 5000)])
+# one tile of 64 x 64 and several (the first four), 128 x 64, 128 x 128, 128 x 192
+@pytest.mark.parametrize("m,n", [(1, 8), (65, 72), (63, 1032), (130, 5128), (515, 2568), (515, 4104), (1000, 5000)])
 def test_small_tiles_exact(gpu_device, m, n, k):
-    print(f"[gemm tiles] m={m} n={n} k={k}", flush=True)
+    tile = _tile(gpu_device, m, n, k)
+    print(f"[gemm tiles] m={m} n={n} k={k} tile={tile}", flush=True)
+    assert tile in (None, {2568: (128, 64), 4104: (128, 128), 5000: (128, 192)}.get(n, (64, 64)))
     a, w = _rand_i8((m, k), m + k), _rand_i8((n, k), n + k)
     ad, wd = a.to(gpu_device), w.to(gpu_device)
     got = torch.ops.turing_utils.int8_gemm_i32(ad, wd)
@@ -35,10 +44,13 @@ def test_small_tiles_exact(gpu_device, m, n, k):
     assert torch.equal(got, whole)
 
 
-@pytest.mark.parametrize("m,n,k", [(1, 1032, 528), (130, 5128, 640), (515, 2568, 5120), (1000, 5000, 5120)])
-def test_small_tile_epilogues(gpu_device, m, n, k):
+@pytest.mark.parametrize("m,n,k,want", [(1, 1032, 528, (64, 64)), (130, 5128, 640, (64, 64)), (515, 2568, 5120, (128, 64)),
+                                        (515, 4104, 640, (128, 128)), (1000, 5000, 5120, (128, 192))])
+def test_small_tile_epilogues(gpu_device, m, n, k, want):
     """Each output type and the gated residual against the 256 x 256 tile."""
-    print(f"[gemm tiles] epilogues m={m} n={n} k={k}", flush=True)
+    tile = _tile(gpu_device, m, n, k)
+    print(f"[gemm tiles] epilogues m={m} n={n} k={k} tile={tile}", flush=True)
+    assert tile in (None, want)
     dev = gpu_device
     a = _rand_i8((m, k), m).to(dev)
     w, ws, bias = (t.to(dev) for t in inputs.weights(n, k, 3))
