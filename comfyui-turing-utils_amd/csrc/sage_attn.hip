@@ -576,6 +576,11 @@ __global__ __launch_bounds__(kThreads, 1) void sage_attn_kernel(
     }
     wg_barrier();
     if (grp == 1) softmax(0, std::true_type{});
+    // No scalar load may be left in flight here: they return out of order with
+    // the LDS reads, so with one pending every step's first K fragment could
+    // only wait for all of them (the split kernel loaded plan fields here that
+    // it needs after the loop: B1 H12 L8190 D128 279 us, 268 without).
+    __builtin_amdgcn_s_waitcnt(lgkmcnt_imm(0));
     // Intervals 1 .. main_steps, one barrier each.  Both groups run the same
     // sequence M_it = {QK(it + 1), PV(it)}, softmax(it + 1); group 0's
     // barrier follows the softmax, group 1's precedes it, so interval it + 1
