@@ -46,3 +46,16 @@ def test_main_cluster_waits_for_single_fragments(kernels, d, causal, split):
     waits = [int(n) for x in block[:first] for n in re.findall(r"lgkmcnt\((\d+)\)", x)]
     reads = sum(x.startswith("ds_read") for x in block[:first])
     assert reads >= 4 and waits and min(waits) > 0, (reads, waits)
+
+
+@pytest.mark.parametrize("causal,split", [(0, 0), (0, 1), (1, 0), (1, 1)])
+def test_exponentials_of_head_dim_64_are_apart(kernels, causal, split):
+    """At head_dim 64 a tile's exponentials alternate with other instructions
+    (a run of eight holds the wave up)."""
+    clusters = 0
+    for block in kernels[64, causal, split]:
+        runs = [len(r) for r in re.findall("E+", "".join("E" if x.startswith("v_exp") else "." for x in block))]
+        if sum(runs) >= 16:
+            clusters += 1
+            assert sum(runs) <= 1.5 * len(runs) and max(runs) <= 3, runs
+    assert clusters >= 2
