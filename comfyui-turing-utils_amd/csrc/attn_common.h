@@ -54,12 +54,4 @@ __device__ __forceinline__ void wg_barrier() {
     __builtin_amdgcn_sched_barrier(0);
 }
 
-// Workgroup i of n (XCD i mod 8) -> its place in the plan: XCD x owns the
-// contiguous x-th eighth of the n, so the query blocks of a head run on one
-// XCD and its L2 reads that head's K and V^T once for all of them.
-__device__ __forceinline__ uint32_t xcd_chunk(uint32_t i, uint32_t n) {
-    const uint32_t x = i & 7, q = n >> 3, r = n & 7;
-    return x * q + min(x, r) + (i >> 3);
-}
-
 }  // namespace tu

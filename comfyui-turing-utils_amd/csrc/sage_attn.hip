@@ -41,6 +41,7 @@
 #include <type_traits>
 
 #include "attn_common.h"
+#include "attn_plan.h"
 #include "sage_prep.h"
 
 namespace tu {
@@ -422,25 +423,6 @@ __device__ __forceinline__ void mfma_cluster(const int8_t *kst, const int8_t *vs
 constexpr int kStages = 4;
 constexpr int kAhead = kStages - 1;
 
-// Work plan of a launch.  Query blocks are numbered head-major (block =
-// (batch * hq + head) * nqb + query block).  Non-causal: blocks below
-// split_from run whole, one workgroup each; every later block runs as
-// `parts` workgroups of seg_tiles key tiles (the last range may be shorter),
-// all blocks' first ranges before any second range.  Causal: every block
-// runs as ceil(its key tiles / seg_tiles) workgroups; workgroups are numbered
-// by query block from the last, longest one to the first (heads fastest,
-// then ranges), so the long ones start first and the short ones fill the
-// end: at B2 H16 L4001 D128 that took the kernel from 177 to 115 us.
-struct AttnPlan {
-    uint32_t nqb;         // query blocks of a head
-    uint32_t bh;          // batch * hq
-    uint32_t split_from;  // first split block (non-causal)
-    uint32_t parts;       // key ranges of a split block (causal: of the last query block)
-    int seg_tiles;        // key tiles of a range
-    int64_t part_row0;    // query row (batch * hq * lq numbering) of the first split block
-    int64_t part_rows;    // query rows of the split blocks
-};
-
 // kSplit: workgroups that cover only a range of their block's key tiles write
 // the unnormalized O with each row's exponent base and row sum to `part` for
 // sage_combine_kernel.
@@ -466,32 +448,8 @@ __global__ __launch_bounds__(kThreads, 1) void sage_attn_kernel(
     // (batch * head, query block, key range) of this workgroup, in 32-bit
     // arithmetic: 64-bit divisions are long instruction sequences, and a
     // short key sequence pays for them in every workgroup
-    uint32_t bh, qb, z = 0;
-    bool whole = true;
-    if constexpr (kCausal) {
-        uint32_t id = blockIdx.x;
-        bh = id % plan.bh;
-        id /= plan.bh;
-        if constexpr (kSplit) {
-            z = id % plan.parts;
-            id /= plan.parts;
-        }
-        qb = plan.nqb - 1 - id;
-    } else {
-        const uint32_t blocks = plan.nqb * plan.bh;
-        uint32_t blk = blockIdx.x;
-        if (kSplit && blk >= plan.split_from) {
-            const uint32_t n = blocks - plan.split_from;
-            const uint32_t i = xcd_chunk(blk - plan.split_from, n * plan.parts);
-            z = i / n;
-            blk = plan.split_from + i - z * n;
-            whole = false;
-        } else {
-            blk = xcd_chunk(blk, kSplit ? plan.split_from : blocks);
-        }
-        bh = blk / plan.nqb;
-        qb = blk % plan.nqb;
-    }
+    const auto [bh, qb, z, in_one] = sage_place<kCausal, kSplit>(plan, blockIdx.x);
+    bool whole = in_one;
     const uint32_t b = bh / hq, h = bh % hq, hk = h / groups;
     const uint32_t hkv = hq / groups;
     const int64_t qblock0 = static_cast<int64_t>(qb) * kBQ;
@@ -816,11 +774,8 @@ int32_t launch_planned(const AttnPlan &plan, const int8_t *q8, const float *q_sc
     while ((kBKey << kscale_shift) < blkk) ++kscale_shift;
     const uint32_t nbq = static_cast<uint32_t>((lq + blkq - 1) / blkq);
     const uint32_t nbk = static_cast<uint32_t>((lk + blkk - 1) / blkk);
-    const int64_t blocks = static_cast<int64_t>(plan.nqb) * plan.bh;
     const bool split = plan.parts > 1;
-    const int64_t grid = !split    ? blocks
-                         : kCausal ? blocks * plan.parts
-                                   : plan.split_from + (blocks - plan.split_from) * plan.parts;
+    const int64_t grid = sage_grid<kCausal>(plan);
     TU_REQUIRE(grid <= 0x7fffffff, "Sage attention grid too large");
 #define TU_ATTN_ARGS                                                                                             \
     q8, q_scale, static_cast<uint32_t>(blkq), nbq, k8, k_scale, kscale_shift, nbk,                                \

@@ -40,6 +40,7 @@
 #include <type_traits>
 
 #include "attn_common.h"
+#include "attn_plan.h"
 
 namespace tu {
 namespace {
@@ -514,48 +515,12 @@ __device__ __forceinline__ void w8a8_block(TU_W8_TENSORS, const W8Dims &a, int8_
 
 #define TU_W8_POINTERS q8, q_scale, k8, k_scale, vt, v_scale, o
 
-// Work plan of a launch.  Query blocks of 256 rows are numbered head-major.
-// Blocks below split_from run whole, one workgroup of 32 rows a wave; every
-// later one as two workgroups of 128 rows, 16 a wave (an end block of at most
-// 128 rows leaves its second one empty).  Neither changes a row's arithmetic.
-// Causal workgroups are numbered by query block from the last, longest one
-// to the first, heads fastest.
-struct W8Plan {
-    uint32_t nqb;         // query blocks of a head
-    uint32_t bh;          // batch * hq
-    uint32_t split_from;  // first block that runs as two workgroups (causal: all or none)
-};
-
 // kMode: 0 every block whole, 1 every block in two, 2 both.
 template <bool kCausal, bool kFp16Out, int kMode>
 __global__ __launch_bounds__(kThreads, 1) void w8a8_attn_kernel(TU_W8_TENSORS, W8Dims a,
                                                                 W8Plan plan) {
     __shared__ __align__(1024) int8_t lds[kStages][kStageBytes];
-    uint32_t id = blockIdx.x, half = 0;
-    bool whole = kMode == 0;
-    uint32_t bh, qb;
-    if constexpr (kCausal) {
-        bh = id % plan.bh;
-        id /= plan.bh;
-        if constexpr (kMode == 1) {
-            half = 1 - (id & 1);  // the later rows are the longer ones
-            id >>= 1;
-        }
-        qb = plan.nqb - 1 - id;
-    } else {
-        const uint32_t blocks = plan.nqb * plan.bh;
-        if constexpr (kMode == 2) whole = id < plan.split_from;
-        if (whole) {
-            id = xcd_chunk(id, kMode == 0 ? blocks : plan.split_from);
-        } else {
-            const uint32_t from = kMode == 1 ? 0 : plan.split_from;
-            id = xcd_chunk(id - from, 2 * (blocks - from));
-            half = id & 1;
-            id = from + (id >> 1);
-        }
-        bh = id / plan.nqb;
-        qb = id % plan.nqb;
-    }
+    const auto [bh, qb, half, whole] = w8_place<kCausal, kMode>(plan, blockIdx.x);
     const int64_t q0 = static_cast<int64_t>(qb) * kBQ + 128 * half;
     if (q0 >= a.lq) return;  // the whole workgroup
     if constexpr (kMode == 2) {
@@ -601,7 +566,7 @@ template <bool kCausal, bool kFp16Out>
 int32_t launch_w8(const W8Plan &plan, TU_W8_TENSORS, const W8Dims &a, hipStream_t s) {
     const int64_t blocks = static_cast<int64_t>(plan.nqb) * plan.bh;
     const int64_t whole = std::min<int64_t>(plan.split_from, blocks);
-    const int64_t grid = whole + 2 * (blocks - whole);
+    const int64_t grid = w8_grid(plan);
     TU_REQUIRE(grid <= 0x7fffffff, "W8A8 attention grid too large");
     const dim3 g(static_cast<unsigned>(grid));
     if (whole == blocks) {

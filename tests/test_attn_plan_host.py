@@ -7,6 +7,7 @@ import os
 import pytest
 
 from comfyui_turing_utils_kernel import _lib
+from tests.test_attn_numbering import places  # noqa: F401
 from tests.test_attn_schedule import KBKEY, KBQ, check_schedule, kernel_program
 
 
@@ -33,17 +34,12 @@ def test_causal_ranges(lq, lk, seg, kernel):
 
 
 @pytest.mark.parametrize("nqb,bh,full,parts", [(4, 3, 0, 2), (5, 7, 11, 3), (32, 12, 256, 2)])
-def test_noncausal_numbering(nqb, bh, full, parts):
-    """Workgroup number -> (block, range), as the kernel computes it: every
+def test_noncausal_numbering(places, nqb, bh, full, parts):  # noqa: F811
+    """Workgroup number -> (block, range), by the kernel's own function: every
     whole block once, every range of every later block once."""
-    n = nqb * bh - full
-    seen = []
-    for wg in range(full + n * parts):
-        z, blk = (0, wg) if wg < full else ((wg - full) // n, wg - (wg - full) // n * n)
-        seen.append((blk // nqb, blk % nqb, z if wg >= full else None))
-    want = [(b // nqb, b % nqb, None) for b in range(full)]
-    want += [(b // nqb, b % nqb, z) for z in range(parts) for b in range(full, nqb * bh)]
-    assert sorted(seen, key=str) == sorted(want, key=str)
+    want = [(b // nqb, b % nqb, 0, 1) for b in range(full)]
+    want += [(b // nqb, b % nqb, z, 0) for z in range(parts) for b in range(full, nqb * bh)]
+    assert sorted(places("sage", 0, nqb, bh, full, parts)) == sorted(want)
 
 
 def test_workspace_plan():
