@@ -59,8 +59,13 @@ TU_HOST_DEVICE SagePlace sage_place(const AttnPlan &plan, uint32_t id) {
     } else {
         const uint32_t blocks = plan.nqb * plan.bh;
         if (kSplit && id >= plan.split_from) {
+            // Split blocks keep their order: the ranges of a launch that is
+            // split are short, and 16 or more blocks of a head on one XCD
+            // would all read the same key tile at once (B1 H4 L4001 D128,
+            // four ranges: 39.1 us spread over the XCDs, 41.0 with a head's
+            // on one; B1 H6 L3000 D64 27.5 and 31.4).
             const uint32_t n = blocks - plan.split_from;
-            const uint32_t i = xcd_chunk(id - plan.split_from, n * plan.parts);
+            const uint32_t i = id - plan.split_from;
             p.z = i / n;
             id = plan.split_from + i - p.z * n;
             p.whole = false;

@@ -72,7 +72,8 @@ def test_sage_noncausal(places, nqb, bh):
         for parts in (2, 3, 7, 16):
             got = places("sage", 0, nqb, bh, full, parts)
             assert sorted(got[:full]) == [(b, q, 0, 1) for b, q in blocks[:full]]
-            assert sorted(got[full:]) == sorted((b, q, z, 0) for b, q in blocks[full:] for z in range(parts))
+            # all first ranges before any second, blocks in turn over the XCDs
+            assert got[full:] == [(b, q, z, 0) for z in range(parts) for b, q in blocks[full:]]
 
 
 @pytest.mark.parametrize("nqb,bh", GRIDS)
