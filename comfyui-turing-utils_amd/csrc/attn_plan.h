@@ -86,16 +86,17 @@ inline int64_t sage_grid(const AttnPlan &plan) {
     return kCausal ? blocks * plan.parts : plan.split_from + (blocks - plan.split_from) * plan.parts;
 }
 
-// Work plan of a W8A8 launch.  Query blocks of 256 rows are numbered head-major.
-// Blocks below split_from run whole, one workgroup of 32 rows a wave; every
-// later one as two workgroups of 128 rows, 16 a wave (an end block of at most
-// 128 rows leaves its second one empty).  Neither changes a row's arithmetic.
-// Causal workgroups are numbered by query block from the last, longest one
-// to the first, heads fastest.
+// Work plan of a W8A8 launch.  Query blocks of 256 rows are numbered
+// head-major.  Blocks below split_from run whole, one workgroup of 32 rows a
+// wave; every later one as two workgroups of 128 rows, 16 a wave (an end block
+// of at most 128 rows leaves its second one empty).  Neither changes a row's
+// arithmetic.  Causal workgroups are numbered by query block from the last,
+// longest one to the first, heads fastest.
 struct W8Plan {
     uint32_t nqb;         // query blocks of a head
     uint32_t bh;          // batch * hq
     uint32_t split_from;  // first block that runs as two workgroups (causal: all or none)
+    uint32_t in_order;    // workgroups in the order of the blocks, whatever their XCD
 };
 
 struct W8Place {
@@ -107,7 +108,7 @@ struct W8Place {
 template <bool kCausal, int kMode>
 TU_HOST_DEVICE W8Place w8_place(const W8Plan &plan, uint32_t id) {
     W8Place p{0, 0, 0, kMode == 0};
-    if constexpr (kCausal) {
+    if (kCausal && !plan.in_order) {
         p.bh = id % plan.bh;
         id /= plan.bh;
         if constexpr (kMode == 1) {
@@ -115,20 +116,81 @@ TU_HOST_DEVICE W8Place w8_place(const W8Plan &plan, uint32_t id) {
             id >>= 1;
         }
         p.qb = plan.nqb - 1 - id;
-    } else {
-        const uint32_t blocks = plan.nqb * plan.bh;
-        if constexpr (kMode == 2) p.whole = id < plan.split_from;
-        if (p.whole) {
-            id = xcd_chunk(id, kMode == 0 ? blocks : plan.split_from);
-        } else {
-            const uint32_t from = kMode == 1 ? 0 : plan.split_from;
-            id = xcd_chunk(id - from, 2 * (blocks - from));
-            p.half = id & 1;
-            id = from + (id >> 1);
-        }
-        p.bh = id / plan.nqb;
-        p.qb = id % plan.nqb;
+        return p;
     }
+    const uint32_t blocks = plan.nqb * plan.bh;
+    if constexpr (kMode == 2) p.whole = id < plan.split_from;
+    if (p.whole) {
+        if (!plan.in_order) id = xcd_chunk(id, kMode == 0 ? blocks : plan.split_from);
+    } else {
+        const uint32_t from = kMode == 1 ? 0 : plan.split_from;
+        id -= from;
+        if (!plan.in_order) id = xcd_chunk(id, 2 * (blocks - from));
+        p.half = id & 1;
+        id = from + (id >> 1);
+    }
+    p.bh = id / plan.nqb;
+    p.qb = id % plan.nqb;
+    return p;
+}
+
+constexpr int64_t kW8BlockRows = 256, kW8TileKeys = 64;
+
+// Time of causal workgroups of `rows` rows over all query blocks on `cus`
+// compute units, in key tiles of one: the longest start first, so the time is
+// their even share, or that of the rounds that hold all blocks of some length
+// and longer.  `fixed` is a workgroup's time beside its tiles.
+inline double w8_causal_time(const W8Plan &p, int64_t lq, int64_t lk, int64_t rows, double fixed, int64_t cus) {
+    double even = 0.0, rounds = 0.0;
+    int64_t count = 0;
+    for (int64_t i = (lq + rows - 1) / rows; i > 0; --i) {
+        const int64_t keys = std::min(lk, i * rows);
+        const double t = static_cast<double>((keys + kW8TileKeys - 1) / kW8TileKeys) + fixed;
+        count += p.bh;
+        even += t * p.bh;
+        rounds = std::max(rounds, static_cast<double>((count + cus - 1) / cus) * t);
+    }
+    return std::max(even / static_cast<double>(cus), rounds);
+}
+
+// Workgroups of 128 rows read K and V^T once for half the rows: a tile takes
+// 1.22 us against 2.0 of a whole block's, and 6.3 us are spent beside the
+// tiles against 9.  They pay where whole blocks leave compute units idle:
+//   non-causal, the blocks past the last full round when they are at most
+//     half a round: B1 H12 L1560 (84 blocks) 61.5 -> 37 us, H56 L4096 (896)
+//     509 -> 461, B1 H12 L8190 (384) 461 -> 368; with more left over, two
+//     half rounds are slower than one whole one (H60 L4096, 192 left: 512 and
+//     531 us).  After full rounds the kernel for both forms takes more
+//     than halves of a single key tile save;
+//   causal, every block when the time by w8_causal_time is less: H4 L4001 117
+//     -> 72 us, H40 L1000 41 -> 26, H12 L1560 x 512 25 -> 16; B2 H16 L4001
+//     stays whole (149 against 166), and so does H10 L5000 x 128 (14.8 against
+//     16.3: all blocks have two tiles, one round of whole ones against two).
+// In a single round of blocks a head's workgroups run on all XCDs where they
+// have at most four key tiles, or are at least 16: on one XCD they read the
+// same key tile at once, and there is little to share from its L2 (B1 H3
+// L20000 x 256 18.4 us on all XCDs, 19.0 on one, x 1024 42.9 and 43.2).  Over
+// several rounds those of more than one tile stay on one (B1 H40 L7800 x 256
+// 81.9 us, 83.7 on all; B1 H9 L8190 x 16 22.3, 22.0).
+// Causal blocks of at most four tiles are equally long and go in order, as do
+// whole ones of a single round, which all start at once (B2 H8 L4096 x 320
+// 21.7 us from the longest on, 21.0 in order).
+inline W8Plan w8_plan(int64_t batch, int64_t hq, int64_t lq, int64_t lk, bool causal, int64_t cus) {
+    W8Plan p{static_cast<uint32_t>((lq + kW8BlockRows - 1) / kW8BlockRows), static_cast<uint32_t>(batch * hq), 0xffffffffu, 0};
+    const int64_t blocks = static_cast<int64_t>(p.nqb) * p.bh;
+    const bool few_keys = lk <= 4 * kW8TileKeys;
+    p.in_order = causal ? few_keys : blocks <= cus ? few_keys || p.nqb >= 16 : lk <= kW8TileKeys;
+    if (!causal) {
+        const int64_t full = blocks / cus * cus;
+        if (full < 0x7fffffff && 2 * (blocks - full) <= cus && (full == 0 || lk > kW8TileKeys))
+            p.split_from = static_cast<uint32_t>(full);
+        return p;
+    }
+    if (blocks >= 8 * cus) return p;  // an even share longer than any block
+    if (0.58 * w8_causal_time(p, lq, lk, kW8BlockRows / 2, 5.2, cus) < w8_causal_time(p, lq, lk, kW8BlockRows, 4.5, cus))
+        p.split_from = 0;
+    else if (blocks <= cus)
+        p.in_order = 1;
     return p;
 }
 

@@ -520,6 +520,7 @@ template <bool kCausal, bool kFp16Out, int kMode>
 __global__ __launch_bounds__(kThreads, 1) void w8a8_attn_kernel(TU_W8_TENSORS, W8Dims a,
                                                                 W8Plan plan) {
     __shared__ __align__(1024) int8_t lds[kStages][kStageBytes];
+    static_assert(kBQ == kW8BlockRows && kBKey == kW8TileKeys, "the plan's block and tile");
     const auto [bh, qb, half, whole] = w8_place<kCausal, kMode>(plan, blockIdx.x);
     const int64_t q0 = static_cast<int64_t>(qb) * kBQ + 128 * half;
     if (q0 >= a.lq) return;  // the whole workgroup
@@ -529,37 +530,6 @@ __global__ __launch_bounds__(kThreads, 1) void w8a8_attn_kernel(TU_W8_TENSORS, W
     } else {
         w8a8_block<kCausal, kFp16Out, kMode == 0 ? 2 : 1>(TU_W8_POINTERS, a, lds, bh, q0);
     }
-}
-
-// Workgroups of 128 rows read K and V^T once for half the rows: they take
-// 0.55-0.6 of a whole block's time (28.7 and 51.4 us for 8 and 25 key tiles
-// of 84 blocks against 26.1 and 61.5 for whole ones).  They pay where whole
-// blocks leave compute units idle:
-//   non-causal, the blocks past the last full round when they are at most
-//     half a round: B1 H12 L1560 (84 blocks) 61.5 -> 37 us, H56 L4096 (896)
-//     509 -> 461, B1 H12 L8190 (384) 461 -> 368; with more left over, two
-//     half rounds are slower than one whole one (H60 L4096, 192 left: 512 and
-//     531 us);
-//   causal, every block when the longest block outweighs the even share of
-//     all of them by more than the halves' extra work: H4 L4001 117 -> 72 us,
-//     H40 L1000 41 -> 26; B2 H16 L4001 stays whole (149 against 166).
-W8Plan w8_plan(int64_t batch, int64_t hq, int64_t lq, int64_t lk, bool causal, int64_t cus) {
-    W8Plan p{static_cast<uint32_t>((lq + kBQ - 1) / kBQ), static_cast<uint32_t>(batch * hq), 0xffffffffu};
-    const int64_t blocks = static_cast<int64_t>(p.nqb) * p.bh;
-    if (!causal) {
-        const int64_t full = blocks / cus * cus;
-        if (full < 0x7fffffff && 2 * (blocks - full) <= cus) p.split_from = static_cast<uint32_t>(full);
-        return p;
-    }
-    if (blocks >= 8 * cus) return p;  // an even share longer than any block
-    int64_t work = 0, longest = 0;
-    for (uint32_t qb = 0; qb < p.nqb; ++qb) {
-        const int64_t t = (std::min<int64_t>(lk, (qb + int64_t{1}) * kBQ) + kBKey - 1) / kBKey;
-        work += t;
-        longest = std::max(longest, t);
-    }
-    if (8 * work * p.bh < 7 * longest * cus) p.split_from = 0;
-    return p;
 }
 
 template <bool kCausal, bool kFp16Out>

@@ -19,6 +19,11 @@ pytestmark = pytest.mark.gpu
     (200, 250, 130, torch.bfloat16, False),   # more than half a round left over: whole
     (256, 300, 300, torch.bfloat16, True),    # causal, whole blocks
     (16, 700, 300, torch.float16, True),      # causal, half blocks, more queries than keys
+    (300, 257, 64, torch.bfloat16, False),    # one key tile over several rounds: whole, in order
+    (12, 5000, 200, torch.float16, False),    # one round of many blocks of a head, in order
+    (40, 700, 200, torch.bfloat16, True),     # causal, few keys: half blocks in order
+    (240, 250, 200, torch.bfloat16, True),    # whole ones in order
+    (16, 4096, 320, torch.float16, True),     # causal, one round of whole blocks, in order
 ])
 def test_rows_do_not_depend_on_the_grid(gpu_device, h, lq, lk, dtype, causal):
     from comfyui_turing_utils_kernel.turing_sage import w8a8attn
