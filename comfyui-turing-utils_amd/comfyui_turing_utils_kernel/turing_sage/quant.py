@@ -115,11 +115,11 @@ def sage_prologue(
     q_scale = torch.empty((batch, hq, (lq + BLKQ - 1) // BLKQ), dtype=torch.float32, device=device)
     k_scale = torch.empty((batch, hkv, (lk + BLKK - 1) // BLKK), dtype=torch.float32, device=device)
     value_t = torch.empty((batch, hkv, dim, lpad), dtype=torch.bfloat16, device=device)
-    nbytes = int(_lib.load().tu_sage_prep_workspace(batch, hkv, lk, dim, int(smooth_k)))
+    nbytes = int(_lib.load().tu_sage_prep_workspace(batch, hkv, lk, dim, int(bool(smooth_k))))
     workspace = torch.empty(nbytes, dtype=torch.uint8, device=device) if nbytes else None
     with torch.cuda.device(device):
         _lib.call("tu_sage_prep", q.data_ptr(), k.data_ptr(), v.data_ptr(), batch, hq, hkv, lq, lk, dim, *q_strides,
-                  *k_strides, *v_strides, int(smooth_k), BLKQ, BLKK, q_int8.data_ptr(),
+                  *k_strides, *v_strides, int(bool(smooth_k)), BLKQ, BLKK, q_int8.data_ptr(),
                   *_layout_dims(q_int8, tensor_layout)[2:], k_int8.data_ptr(), *_layout_dims(k_int8, tensor_layout)[2:],
                   q_scale.data_ptr(), k_scale.data_ptr(), value_t.data_ptr(), lpad, _lib.ptr(workspace), nbytes,
                   _lib.stream_of(device))

@@ -184,6 +184,21 @@ def test_key_split_workspace_checked_and_sized():
             core.attention_from_vt(q8, qs, k8, ks, vt, kv_splits=2, workspace=bad)
 
 
+@pytest.mark.parametrize("smooth_k,flag", [(None, 0), (False, 0), (0, 0), ("", 0), (True, 1), (2, 1), ("yes", 1)])
+def test_smooth_k_by_its_truth(monkeypatch, smooth_k, flag):
+    """The shared prologue takes smooth_k by its truth value, as the parts do."""
+    import contextlib
+
+    calls = []
+    monkeypatch.setattr(quant._lib, "call", lambda name, *args: calls.append((name, args)))
+    monkeypatch.setattr(quant._lib, "stream_of", lambda device: 0)
+    monkeypatch.setattr(torch.cuda, "device", lambda device: contextlib.nullcontext())
+    q = torch.zeros(1, 2, 64, 64, dtype=torch.bfloat16)
+    quant.sage_prologue(q, q, q, smooth_k=smooth_k)
+    (name, args), = calls
+    assert name == "tu_sage_prep" and args[18] == flag and type(args[18]) is int
+
+
 def test_preflight_refuses_cpu():
     with pytest.raises(RuntimeError, match="GPU"):
         turing_sage.preflight(torch.device("cpu"))
