@@ -91,6 +91,9 @@ struct ReleaseGil {
     ~ReleaseGil() { PyEval_RestoreThread(state); }
 };
 
+// The quantizer's widest row; the general route refuses a wider one with a ValueError.
+constexpr int64_t kMaxColumns = 65536;
+
 // int8_linear(x, weight, weight_scale, bias, out_kind, group, act, stream):
 // ConvRot quantizer and INT8 GEMM.  out_kind 0 bf16, 1 fp16, 2 fp32.
 PyObject *int8_linear(PyObject *, PyObject *const *args, Py_ssize_t nargs) {
@@ -110,7 +113,7 @@ PyObject *int8_linear(PyObject *, PyObject *const *args, Py_ssize_t nargs) {
         !ws->is_contiguous() || (group != 128 && group != 256) || act < 0 || act > 2 || kind < 0 || kind > 2)
         Py_RETURN_NONE;
     const int64_t n = w->size(0), k = w->size(1), width = act == TU_ACT_SWIGLU ? 2 * k : k;
-    if (n <= 0 || n % 8 || k <= 0 || k % group || x->size(-1) != width || x->numel() == 0 || ws->numel() != n ||
+    if (n <= 0 || n % 8 || k <= 0 || k > kMaxColumns || k % group || x->size(-1) != width || x->numel() == 0 || ws->numel() != n ||
         (bias && (bias->scalar_type() != at::kFloat || !bias->is_contiguous() || bias->numel() != n)))
         Py_RETURN_NONE;
     const int64_t m = x->numel() / width;

@@ -63,6 +63,14 @@ def test_linear(gpu_device, both, act, out_dtype, group, with_bias):
     assert torch.equal(native, general)
 
 
+@pytest.mark.parametrize("act", [None, "swiglu"])
+def test_rows_too_wide_for_the_quantizer(gpu_device, act):
+    """The general route's error, with the module and without."""
+    x, w, ws, bias = _linear(gpu_device, rows=1, k=65536 + 256, n=8, act=act)
+    with pytest.raises(ValueError, match="65536-column limit"):
+        integration.int8_linear(x, w, ws, bias, None, True, 256, act)
+
+
 def test_linear_forms_that_are_not_plain(gpu_device, both):
     x, w, ws, bias = _linear(gpu_device, rows=8)
     off = torch.empty(8 * 512 + 1, dtype=torch.bfloat16, device=gpu_device)[1:].reshape(8, 512).copy_(x)
