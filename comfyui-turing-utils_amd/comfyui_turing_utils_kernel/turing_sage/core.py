@@ -267,7 +267,9 @@ def attention_from_vt(
         elif kv_splits is not None:
             _lib.call("tu_sage_attn_fwd", *shape, int(bool(is_causal)), _lib.stream_of(device))
         else:
-            partial = workspace if usable and workspace.data_ptr() % 16 == 0 else None
+            # one that was not asked for and is not aligned is left alone; one
+            # that is needed goes to the kernel's own check
+            partial = workspace if usable and (required > 1 or workspace.data_ptr() % 16 == 0) else None
             if partial is None:
                 nbytes = int(lib.tu_sage_attn_workspace(batch, hq, lq, lk, width, int(bool(is_causal)), cus))
                 partial = torch.empty(nbytes // 4, dtype=torch.float32, device=device) if nbytes else None

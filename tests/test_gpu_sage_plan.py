@@ -77,3 +77,22 @@ def test_output_rows_on_8_byte_boundaries(gpu_device, d):
     wide = torch.full((1, 2, 300, d + 4), 7.0, dtype=torch.bfloat16, device=gpu_device)
     core.attention_from_vt(*args, output=wide[..., :d])
     assert torch.equal(wide[..., :d], want) and bool((wide[..., d:] == 7.0).all())
+
+
+def test_misaligned_workspace(gpu_device):
+    """A workspace that a split call needs is refused off 16 bytes; where none
+    is needed it is not used."""
+    for lk, needed in ((4096, True), (300, False)):
+        q, k, v = inputs.attention(1, 2, lk, 128, 7)
+        state = core.prequantize_sageattn(q[:, :, :200].contiguous().to(gpu_device), k.to(gpu_device), v.to(gpu_device))
+        args = (state.query_int8, state.query_scale, state.key_int8, state.key_scale, state.value_t)
+        cus = core._compute_units(gpu_device)
+        splits = _lib.load().tu_sage_attn_kv_splits(1, 2, 200, lk, 0, cus)
+        assert (splits > 1) == needed
+        ws = torch.zeros(core.split_workspace_bytes(1, 2, 200, lk, 128, splits) // 4 + 1, dtype=torch.float32, device=gpu_device)[1:]
+        if needed:
+            with pytest.raises(RuntimeError, match="aligned"):
+                core.attention_from_vt(*args, workspace=ws)
+        else:
+            assert torch.equal(core.attention_from_vt(*args, workspace=ws), core.attention_from_vt(*args))
+            assert not ws.any()
