@@ -686,10 +686,14 @@ constexpr int kTile128x192 = 16, kTile128x128 = 17, kTile128x64 = 18, kTile64x64
 
 // Automatic tile: the least of first + rounds * (fixed + per_step * steps),
 // rounds = tiles / CUs rounded up and steps of 128 bytes of K, in us.  The
-// constants are fitted to the times of every tile at 340 shapes of M 1 to
-// 32760, N 256 to 19872 and K 64 to 14336 (graph of 3 to 24 launches, bf16 out
-// with bias, three operand sets): the tile taken is at most 2.9 % slower than
-// the best one there, at 90 other shapes 1.6 %, 0.05 % on average at both.
+// constants are fitted to the times of every tile at 576 shapes of M 1 to
+// 33000, N 256 to 21504 and K 64 to 14336 (bf16 out with bias, codes of normal
+// data, three operand sets): the tile taken is at most 6.7 % slower than the
+// best one, at five over 3 %, and 0.1 % on average.  372 of them have the
+// quantizer before each product and its own time taken off, as a linear runs:
+// products in a row hold the chip at its power limit, where the tiles that
+// keep the MFMAs busiest gain nothing (2050 x 5376 x 14336 139 us with 256 x
+// 192 and 161 with 128 x 192 after the quantizer, 157 and 158 in a row).
 // A step of a small grid costs the bytes that a CU pulls past its L2, about 70
 // GB/s, so its time goes with BM + BN whatever the MFMAs do; the fewer
 // columns and rows a CU has to pull while all CUs have a tile, the better,
@@ -697,26 +701,27 @@ constexpr int kTile128x192 = 16, kTile128x128 = 17, kTile128x64 = 18, kTile64x64
 // Over ten rounds it is the MFMAs and the power they take that count, and the
 // larger tile reads its operands less often.
 //                       256x256  256x192  128x256  128x192  128x128   128x64    64x64  (us; * taken)
-//   1 x 8960 x 1536          19.4     16.2     13.1     10.7      9.0      7.3      6.1*
-//   512 x 5120 x 5120        51.0     44.9     32.6     27.6     22.6*    27.9     29.9
-//   512 x 10240 x 5120       51.8     45.4     34.4     29.9*    44.4     42.3     48.7
-//   1024 x 1536 x 1536       21.1     18.2     14.4     11.6     10.0      8.2*     9.4
-//   1024 x 8960 x 1536       23.2     20.8*    30.4     26.0     29.1     28.4     35.9
-//   2050 x 8960 x 1536       47.6     40.9*    47.2     50.4     49.2     54.6     72.8
-//   16380 x 1536 x 1536      49.8     44.6*    49.9     52.3     59.8     66.1     87.1
-//   4096 x 10240 x 5120     183.0*   203.2    201.5    216.5    241.0    285.9    374.4
-//   7800 x 5120 x 5120      184.0*   198.8    198.3    212.0    231.2    273.4    353.2
-//   1560 x 5120 x 13824     153.4    144.9    166.7    136.2*   153.9    168.4    188.3
-//   4096 x 5120 x 13824     323.7    293.3    298.9*   323.9    322.7    407.5    489.6
+//   1 x 8960 x 1536          19.3     16.2     13.2     10.7      9.0      7.3      6.1*
+//   512 x 5120 x 5120        50.7     45.0     32.5     27.8     22.7*    27.8     29.5
+//   512 x 10240 x 5120       51.2     45.0     33.0     29.2*    43.5     40.9     46.3
+//   1024 x 1536 x 1536       20.8     18.1     14.2     11.9     10.2      8.6*     9.4
+//   1024 x 8960 x 1536       21.9     19.0*    28.9     23.3     26.9     26.1     31.9
+//   2050 x 8960 x 1536       45.2     36.7*    42.6     44.3     42.8     49.0     64.8
+//   16380 x 1536 x 1536      45.6     38.9*    42.7     45.0     51.6     56.9     79.0
+//   4096 x 10240 x 5120     221.1*   232.2    225.4    258.9    290.4    338.7    388.9
+//   7800 x 5120 x 5120      188.6*   215.0    192.1    208.9    235.9    276.0    349.9
+//   1560 x 5120 x 13824     145.0    126.9*   161.5    137.8    159.2    173.9    189.0
+//   2050 x 5376 x 14336     154.1    139.0*   177.0    161.3    188.3    233.0    286.2
+//   4096 x 5120 x 13824     318.7    280.0    287.3*   315.1    318.0    394.7    471.7
 struct TileCost {
     int policy, bm, bn;
     double first, fixed, per_step;
 };
 constexpr TileCost kTileCosts[] = {
-    {TU_GEMM_TILE_256, 256, 256, 0.0, 8.09, 1.25},  {TU_GEMM_TILE_192, 256, 192, 0.097, 6.81, 1.19},
-    {TU_GEMM_TILE_128, 128, 256, 0.0, 6.94, 0.757}, {kTile128x192, 128, 192, 0.0, 6.18, 0.569},
-    {kTile128x128, 128, 128, 0.3, 4.8, 0.478},      {kTile128x64, 128, 64, 2.63, 1.45, 0.323},
-    {kTile64x64, 64, 64, 2.31, 1.12, 0.25},
+    {TU_GEMM_TILE_256, 256, 256, 0.0, 8.87, 1.16},  {TU_GEMM_TILE_192, 256, 192, 0.0, 7.27, 1.09},
+    {TU_GEMM_TILE_128, 128, 256, 0.0, 6.55, 0.701}, {kTile128x192, 128, 192, 0.0, 5.34, 0.574},
+    {kTile128x128, 128, 128, 0.786, 4.16, 0.466},   {kTile128x64, 128, 64, 2.26, 1.57, 0.3},
+    {kTile64x64, 64, 64, 1.97, 0.989, 0.243},
 };
 
 // A launch takes fewer than 2^32 threads: a tile of fewer rows than the grid

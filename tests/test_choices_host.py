@@ -75,7 +75,8 @@ GEMM_TILES = [
     (7800, 5120, 5120, {(256, 256)}),                # 184; 128 x 256 198
     (7800, 5120, 13824, {(256, 256)}),               # 469; 128 x 256 503
     (16380, 5376, 14336, {(256, 256)}),              # 1032; 256 x 192 1078
-    (1560, 5120, 13824, {(128, 192)}),               # 136; 256 x 192 145
+    (1560, 5120, 13824, {(256, 192)}),               # 127; 128 x 192 138
+    (2050, 5376, 14336, {(256, 192)}),               # 139; 128 x 192 161
     (32760, 13824, 5120, {(256, 256)}),              # 1845; 256 x 192 2058
     (1024, 8960, 1536, {(256, 192)}),                # 20.8; 256 x 256 23.2, 128 x 192 26.0
     (512, 10240, 5120, {(128, 192)}),                # 29.9; 128 x 256 34.4
