@@ -458,10 +458,10 @@ CSRC_DIR = os.path.join(ROOT, "comfyui-turing-utils_amd", "csrc")
 KERNEL_SOURCES = (
     ("convrot_quant", ("convrot_quant.hip", "ln_common.h")),
     ("int8_gemm", ("int8_gemm.hip",)),
-    ("sage_kmean", ("sage_quant.hip",)),
-    ("sage_quant", ("sage_quant.hip",)),
-    ("sage_v_prep", ("sage_attn.hip", "attn_common.h")),
-    ("sage_attn", ("sage_attn.hip", "attn_common.h")),
+    ("sage_kmean", ("sage_quant.hip", "sage_prep.h")),
+    ("sage_quant", ("sage_quant.hip", "sage_prep.h")),
+    ("sage_v_prep", ("sage_attn.hip", "attn_common.h", "attn_plan.h", "sage_prep.h")),
+    ("sage_attn", ("sage_attn.hip", "attn_common.h", "attn_plan.h", "sage_prep.h")),
 )
 
 
